@@ -191,9 +191,16 @@ __device__ __forceinline__ uint32_t to_qbyte(float t, int out_dtype) {
 // SPEC 2: SPEC 1 + jax.random.uniform noise in the original threefry counter layout (the
 //         gradient-side operands).  With PAIR the two elements that share one threefry block
 //         (indices i and i + total/2) are produced by the same thread from a single block.
+// SPEC 6, 7: SPEC 1 and SPEC 2 with float32 values and scales (no intermediate is rounded).  On SPEC 0 a float32
+//         layer was bound by the run-time flags and the 64-bit noise counters: 8.4 million gradients with noise took
+//         131 us (tiles; 18 on SPEC 7) and 32 us (rows; 19), 8.4 million activations without it 23 us (11 on SPEC 6),
+//         and the step of a 4096 x 512 -> 2048 -> 512 block 852 us (374).
+constexpr bool spec_is_f32(int spec) { return spec == 6 || spec == 7; }
+constexpr bool spec_has_uniform_noise(int spec) { return spec == 2 || spec == 7; }
 template <int SPEC>
 __device__ __forceinline__ float spec_scale(float v, float inv, const QArgs& a) {
   if constexpr (SPEC == 0) return rnd(v * inv, a.cbf & a.sbf);
+  if constexpr (spec_is_f32(SPEC)) return v * inv;
   return round_bf16(v * inv);
 }
 __device__ __forceinline__ float uniform_noise(uint32_t bits) {
@@ -241,6 +248,7 @@ __device__ __forceinline__ uint32_t spec_quant(float v, float inv, uint64_t ctr,
   } else {
     float t = spec_scale<SPEC>(v, inv, a);
     if constexpr (SPEC == 2) t = round_bf16(t + uniform_noise(a.gen.word_original((uint32_t)ctr)));
+    if constexpr (SPEC == 7) t = t + uniform_noise(a.gen.word_original((uint32_t)ctr));
     if constexpr (SPEC == 5) {
       const uint32_t w = a.gen.word_original((uint32_t)(ctr >> 1));
       t = bf16_mantissa_sr(t, (ctr & 1) ? (w >> 16) : w, a.out_dtype == AQTX_E4M3 ? 0xFu : 0x1Fu);
@@ -248,35 +256,38 @@ __device__ __forceinline__ uint32_t spec_quant(float v, float inv, uint64_t ctr,
     return spec_finish<SPEC>(t, a);
   }
 }
-// The same for the noiseless integer pipelines (SPEC 0 with integer out, SPEC 1), which also hands out the clipped
+// The same for the noiseless integer pipelines (SPEC 0 with integer out, SPEC 1, SPEC 6), which also hands out the clipped
 // value before rounding: |q| = rint(|t|) and rint is monotonic, so a maximum of |q| can be kept as a maximum of
 // |t| (one instruction per element) and rounded once at the end.
 template <int SPEC>
 __device__ __forceinline__ uint32_t spec_quant_mag(float v, float inv, uint64_t ctr, const QArgs& a, float& t_clipped) {
-  static_assert(SPEC == 0 || SPEC == 1, "noiseless integer pipelines");
+  static_assert(SPEC == 0 || SPEC == 1 || SPEC == 6, "noiseless integer pipelines");
   if constexpr (SPEC == 0) {
     t_clipped = scaled_noisy_clipped(v, inv, ctr, a);
     return to_qbyte(t_clipped, a.out_dtype);
   } else {
-    t_clipped = __builtin_amdgcn_fmed3f(spec_scale<1>(v, inv, a), -a.clip_bound, a.clip_bound);
+    t_clipped = __builtin_amdgcn_fmed3f(spec_scale<SPEC>(v, inv, a), -a.clip_bound, a.clip_bound);
     return __float_as_uint(t_clipped + 12582912.0f) & 0xFFu;
   }
 }
-// the pair (i, i + half) from one threefry block (SPEC 2, original layout, i < half)
+// the pair (i, i + half) from one threefry block (SPEC 2 and 7, original layout, i < half)
+template <int SPEC>
 __device__ __forceinline__ void pair_quant(float v0, float inv0, float v1, float inv1, uint32_t i,
                                            const QArgs& a, uint32_t& q0, uint32_t& q1) {
   const U2 bits = threefry2x32(a.gen.k0, a.gen.k1, i, i + a.gen.half);
+  static_assert(spec_has_uniform_noise(SPEC), "pipelines with one 32-bit draw per element");
   float t0 = v0 * inv0, t1 = v1 * inv1;
-  round_bf16_pair(t0, t1);
+  if constexpr (SPEC == 2) round_bf16_pair(t0, t1);
   t0 += uniform_noise(bits.x);
   t1 += uniform_noise(bits.y);
-  round_bf16_pair(t0, t1);
-  q0 = spec_finish<2>(t0, a);
-  q1 = spec_finish<2>(t1, a);
+  if constexpr (SPEC == 2) round_bf16_pair(t0, t1);
+  q0 = spec_finish<SPEC>(t0, a);
+  q1 = spec_finish<SPEC>(t1, a);
 }
 template <int SPEC>
 __device__ __forceinline__ float spec_prescale(float v, float ps, const QArgs& a) {
   if constexpr (SPEC == 0) return apply_prescale(v, ps, a);
+  if constexpr (spec_is_f32(SPEC)) return v * ps;
   return round_bf16(v * round_bf16(ps));
 }
 template <int SPEC>
@@ -284,9 +295,10 @@ __device__ __forceinline__ void spec_scale_from_absmax(float amax, const QArgs& 
   if constexpr (SPEC == 0) {
     scale_from_absmax(amax, a, scale, inv);
   } else {
+    constexpr bool bf = !spec_is_f32(SPEC);
     if (amax == 0.0f) amax = 1.0f;
-    scale = round_bf16(amax / a.quant_bound);
-    inv = round_bf16(1.0f / scale);
+    scale = round_to<bf>(amax / a.quant_bound);
+    inv = round_to<bf>(1.0f / scale);
     if (isinf(inv)) inv = 1.0f;
   }
 }
@@ -357,7 +369,7 @@ __device__ __forceinline__ uint2 pack8(const uint32_t (&q)[8], int even_odd8) {
 }
 
 // ---- rows kernel: reduced axis contiguous -------------------------------------
-// PAIR (SPEC 2 only): the block owns segment s and segment s + nseg/2, whose elements share
+// PAIR (SPEC 2 and 7): the block owns segment s and segment s + nseg/2, whose elements share
 // threefry blocks; requires whole rows as segments and the natural noise layout.
 // A block is 256 threads, or 512 (LANES = 512: one long segment per block, half the row values per
 // thread, so that six waves fit a SIMD: the stochastic pipeline is bound by vector instruction
@@ -368,7 +380,7 @@ __device__ __forceinline__ uint2 pack8(const uint32_t (&q)[8], int even_odd8) {
 // quantized values over the rows needs instead of reading them again.
 template <typename TIn, int LANES, int ITERS, int SPEC, bool PAIR, bool COLMAX = false>
 __global__ __launch_bounds__(LANES == 512 ? 512 : 256,
-                             (COLMAX && ITERS <= 2 && SPEC != 0) ? 7 : LANES == 512 ? 3 : (sizeof(TIn) == 2 && SPEC != 0) ? 4 : 1)
+                             (COLMAX && ITERS <= 2 && SPEC == 1) ? 7 : LANES == 512 ? 3 : SPEC != 0 && !COLMAX ? 4 : 1)
 void quant_rows_kernel(const QArgs a_in) {
   const QArgs a = with_device_key(a_in);
   constexpr int VEC = 8;
@@ -396,6 +408,7 @@ void quant_rows_kernel(const QArgs a_in) {
   const int64_t segs_per_row = a.cols / a.L;
 
   constexpr bool PACKED = (sizeof(TIn) == 2) && (SPEC != 0);
+  static_assert(!(sizeof(TIn) == 2 && spec_is_f32(SPEC)), "bf16 input is held in bf16");
   RowVals<PACKED> v[NSET][ITERS];
   float scale[NSET], inv[NSET];
   int64_t grow[NSET], col0[NSET];
@@ -477,7 +490,7 @@ void quant_rows_kernel(const QArgs a_in) {
         v[1][it].get(t1);
 #pragma unroll
         for (int e = 0; e < VEC; ++e)
-          pair_quant(t0[e], inv[0], t1[e], inv[1], ctr_row + (uint32_t)(j0 + e), a, q0[e], q1[e]);
+          pair_quant<SPEC>(t0[e], inv[0], t1[e], inv[1], ctr_row + (uint32_t)(j0 + e), a, q0[e], q1[e]);
         *reinterpret_cast<uint2*>(qp0 + j0) = pack8(q0, a.even_odd8);
         *reinterpret_cast<uint2*>(qp1 + j0) = pack8(q1, a.even_odd8);
       }
@@ -733,7 +746,7 @@ __global__ __launch_bounds__(256) void finalize_partials_kernel(const QArgs a, i
 constexpr int kTileR = 128, kTileC = 64, kTilePad = 132;
 
 // 128x64 tile: thread (rg = tid/8, cc = tid%8) owns rows 4*rg..+3, cols 8*cc..+7.
-// PAIR (SPEC 2, and SPEC 5 with value 1): 1 = the block also owns the tile `rows/2` further down (natural noise
+// PAIR (SPEC 2 and 7, and SPEC 5 with value 1): 1 = the block also owns the tile `rows/2` further down (natural noise
 // layout), 2 = the tile `cols/2` further right (noise counters of the transposed tensor); the
 // two tiles' elements share threefry blocks.
 // ROWMAX (no PAIR; every tile interior): the block also finds, for each of its 128 rows, the largest |q| among its 64
@@ -857,7 +870,7 @@ __global__ __launch_bounds__(256) void quant_tile_kernel(const QArgs a_in) {
               }
             } else if constexpr (PAIR) {
               const uint32_t i = (uint32_t)((r0[0] + rg * 4 + j) * a.nsr + (c0[0] + cc * 8 + e) * a.nsc);
-              pair_quant(x[0][e], inv[0][e], x[1][e], inv[1][e], i, a, qv[0], qv[1]);
+              pair_quant<SPEC>(x[0][e], inv[0][e], x[1][e], inv[1][e], i, a, qv[0], qv[1]);
             } else if constexpr (ROWMAX) {
               float tc;
               qv[0] = spec_quant_mag<SPEC>(x[0][e], inv[0][e], 0, a, tc);
@@ -1038,9 +1051,9 @@ int spec_of(const QArgs& a, int partitionable) {
       return 5;  // neighbouring elements draw from one word, starting at an even counter
     return 0;
   }
-  if (!(a.cbf && a.sbf && (a.out_dtype == AQTX_I8 || a.out_dtype == AQTX_I4))) return 0;
-  if (a.noise == AQTX_NOISE_NONE) return 1;
-  if (a.noise == AQTX_NOISE_JAX_UNIFORM && !partitionable) return 2;
+  if (a.cbf != a.sbf || !(a.out_dtype == AQTX_I8 || a.out_dtype == AQTX_I4)) return 0;
+  if (a.noise == AQTX_NOISE_NONE) return a.cbf ? 1 : 6;
+  if (a.noise == AQTX_NOISE_JAX_UNIFORM && !partitionable) return a.cbf ? 2 : 7;
   return 0;
 }
 
@@ -1090,7 +1103,7 @@ int launch_rows_spec(const QArgs& a, hipStream_t st) {
   if (L <= 2048) AQTX_ROWS(256, 1)
   if (L <= 4096) AQTX_ROWS(256, 2)
   if (L <= 8192) AQTX_ROWS(256, 4)
-  if (SPEC == 2 && sizeof(TIn) == 2) AQTX_ROWS(512, 4)
+  if (SPEC == 2 && sizeof(TIn) == 2 || SPEC == 7) AQTX_ROWS(512, 4)
   AQTX_ROWS(256, 8)
 #undef AQTX_ROWS
 }
@@ -1108,22 +1121,23 @@ int launch_rows(const QArgs& a, int partitionable, hipStream_t st) {
     return 0;
   }
   const int spec = spec_of(a, partitionable);
-  if (a.oa_out != nullptr) {  // (the caller has checked rows_colmax_ok: noise none, so spec is 1 or 0)
-    if (spec == 1) return launch_rows_colmax<TIn, 1>(a, st);
-    return launch_rows_colmax<TIn, 0>(a, st);
+  // one threefry block serves elements i and i + total/2: pair whole rows when the noise counters follow the
+  // natural [batch*rows, cols] order
+  const bool natural = a.nsc == 1 && a.nsr == a.cols && (a.batch == 1 || a.nsb == a.rows * a.cols) &&
+                       L == a.cols && (a.nseg % 2 == 0);
+  // (oa_out: the caller has checked rows_colmax_ok: noise none, so spec is 1, 6 or 0; float input is held in the
+  // compute dtype, so the bf16 pipelines never meet float32 input nor the float32 ones bf16 input)
+  if constexpr (sizeof(TIn) != 4) {
+    if (spec == 1) return a.oa_out != nullptr ? launch_rows_colmax<TIn, 1>(a, st) : launch_rows_spec<TIn, 1, false>(a, st);
+    if (spec == 2) return natural ? launch_rows_spec<TIn, 2, true>(a, st) : launch_rows_spec<TIn, 2, false>(a, st);
+    if (spec == 3) return launch_rows_spec<TIn, 3, false>(a, st);
+    if (spec == 5) return launch_rows_spec<TIn, 5, false>(a, st);
   }
-  if (spec == 1) return launch_rows_spec<TIn, 1, false>(a, st);
-  if (spec == 3) return launch_rows_spec<TIn, 3, false>(a, st);
-  if (spec == 5) return launch_rows_spec<TIn, 5, false>(a, st);
-  if (spec == 2) {
-    // one threefry block serves elements i and i + total/2: pair whole rows when the noise
-    // counters follow the natural [batch*rows, cols] order
-    const bool natural = a.nsc == 1 && a.nsr == a.cols && (a.batch == 1 || a.nsb == a.rows * a.cols) &&
-                         L == a.cols && (a.nseg % 2 == 0);
-    if (natural) return launch_rows_spec<TIn, 2, true>(a, st);
-    return launch_rows_spec<TIn, 2, false>(a, st);
+  if constexpr (sizeof(TIn) != 2) {
+    if (spec == 6) return a.oa_out != nullptr ? launch_rows_colmax<TIn, 6>(a, st) : launch_rows_spec<TIn, 6, false>(a, st);
+    if (spec == 7) return natural ? launch_rows_spec<TIn, 7, true>(a, st) : launch_rows_spec<TIn, 7, false>(a, st);
   }
-  return launch_rows_spec<TIn, 0, false>(a, st);
+  return a.oa_out != nullptr ? launch_rows_colmax<TIn, 0>(a, st) : launch_rows_spec<TIn, 0, false>(a, st);
 }
 
 // Whether the tile kernel can leave row maxima of |q| behind for this plan: one scale per column over whole
@@ -1180,30 +1194,52 @@ int launch_tiles(const QArgs& a, int reduce, int partitionable, int64_t nscales,
     return dim3((unsigned)((cols + kTileC - 1) / kTileC), (unsigned)((rows + kTileR - 1) / kTileR),
                 (unsigned)a.batch);
   };
-  if (a.oa_out != nullptr) {  // (the caller has checked tiles_rowmax_ok: noise none, so spec is 1 or 0)
-    if (spec == 1) quant_tile_kernel<TIn, 1, 0, true><<<grid_for(0), 256, 0, st>>>(a);
-    else quant_tile_kernel<TIn, 0, 0, true><<<grid_for(0), 256, 0, st>>>(a);
-  } else if (spec == 1) {
-    quant_tile_kernel<TIn, 1, 0><<<grid_for(0), 256, 0, st>>>(a);
-  } else if (spec == 3) {
-    quant_tile_kernel<TIn, 3, 0><<<grid_for(0), 256, 0, st>>>(a);
-  } else if (spec == 5) {
-    // half of a threefry block would be thrown away unless the tile rows/2 further down, whose
-    // elements draw from the other half, is quantized by the same workgroup
-    const bool natural = a.batch == 1 && a.nsr == a.cols && (a.rows % 2 == 0) && (a.cols % 8 == 0);
-    if (natural) quant_tile_kernel<TIn, 5, 1><<<grid_for(1), 256, 0, st>>>(a);
-    else quant_tile_kernel<TIn, 5, 0><<<grid_for(0), 256, 0, st>>>(a);
-  } else if (spec == 2) {
-    // pair the two elements of each threefry block: i and i + total/2 lie rows/2 apart when the
-    // noise counters are row-major over [rows, cols], cols/2 apart when over [cols, rows]
+#define AQTX_TILE(SPEC, PAIR, ...) quant_tile_kernel<TIn, SPEC, PAIR, ##__VA_ARGS__><<<grid_for(PAIR), 256, 0, st>>>(a)
+  // pair the two elements of each threefry block: i and i + total/2 lie rows/2 apart when the noise counters are
+  // row-major over [rows, cols], cols/2 apart when over [cols, rows]
+  auto uniform = [&](auto tag) {
+    constexpr int S = decltype(tag)::value;
     const bool natural = a.batch == 1 && a.nsc == 1 && a.nsr == a.cols && (a.rows % 2 == 0);
     const bool transposed = a.batch == 1 && a.nsr == 1 && a.nsc == a.rows && (a.cols % 16 == 0);
-    if (natural) quant_tile_kernel<TIn, 2, 1><<<grid_for(1), 256, 0, st>>>(a);
-    else if (transposed) quant_tile_kernel<TIn, 2, 2><<<grid_for(2), 256, 0, st>>>(a);
-    else quant_tile_kernel<TIn, 2, 0><<<grid_for(0), 256, 0, st>>>(a);
-  } else {
-    quant_tile_kernel<TIn, 0, 0><<<grid_for(0), 256, 0, st>>>(a);
+    if (natural) AQTX_TILE(S, 1);
+    else if (transposed) AQTX_TILE(S, 2);
+    else AQTX_TILE(S, 0);
+  };
+  bool done = false;  // (oa_out: the caller has checked tiles_rowmax_ok: noise none, so spec is 1, 6 or 0)
+  if constexpr (sizeof(TIn) != 4) {  // the bf16 pipelines
+    done = true;
+    if (spec == 1 && a.oa_out != nullptr) {
+      AQTX_TILE(1, 0, true);
+    } else if (spec == 1) {
+      AQTX_TILE(1, 0);
+    } else if (spec == 2) {
+      uniform(std::integral_constant<int, 2>{});
+    } else if (spec == 3) {
+      AQTX_TILE(3, 0);
+    } else if (spec == 5) {
+      // half of a threefry block would be thrown away unless the tile rows/2 further down, whose elements draw
+      // from the other half, is quantized by the same workgroup
+      const bool natural = a.batch == 1 && a.nsr == a.cols && (a.rows % 2 == 0) && (a.cols % 8 == 0);
+      if (natural) AQTX_TILE(5, 1);
+      else AQTX_TILE(5, 0);
+    } else {
+      done = false;
+    }
   }
+  if constexpr (sizeof(TIn) != 2) {  // the float32 ones
+    if (!done) {
+      done = true;
+      if (spec == 6 && a.oa_out != nullptr) AQTX_TILE(6, 0, true);
+      else if (spec == 6) AQTX_TILE(6, 0);
+      else if (spec == 7) uniform(std::integral_constant<int, 7>{});
+      else done = false;
+    }
+  }
+  if (!done) {
+    if (a.oa_out != nullptr) AQTX_TILE(0, 0, true);
+    else AQTX_TILE(0, 0);
+  }
+#undef AQTX_TILE
   AQTX_HIP_CHECK_LAUNCH("quant_tile_kernel");
   return 0;
 }

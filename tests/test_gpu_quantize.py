@@ -311,3 +311,34 @@ def test_nan_row_gives_nan_outputs(gpu):
   for m in (2, 48):
     o, xs = ops.decode(lhs[6:6 + m].contiguous(), wq, ws, quant_bound=127.5, clip_bound=127.0)
     assert bool(torch.isnan(xs[1])) and bool(torch.isnan(o[1]).all()) and not bool(torch.isnan(o[0]).any())
+
+
+@pytest.mark.parametrize('reduce,rows,cols', [
+    # whole rows, two of them sharing the blocks of the generator: the smallest and largest of every launch shape
+    (L.REDUCE_COLS, 2, 8), (L.REDUCE_COLS, 6, 128), (L.REDUCE_COLS, 4, 136), (L.REDUCE_COLS, 2, 2048),
+    (L.REDUCE_COLS, 2, 2056), (L.REDUCE_COLS, 2, 8192), (L.REDUCE_COLS, 2, 8200), (L.REDUCE_COLS, 2, 16384),
+    (L.REDUCE_COLS, 5, 1000),                           # an odd number of rows: one block an element
+    # tiles: rows / 2 apart, with remainders in both directions; cols / 2 apart; an odd number of rows
+    (L.REDUCE_ROWS, 256, 64), (L.REDUCE_ROWS, 258, 200), (L.REDUCE_ROWS, 130, 13), (L.REDUCE_ROWS, 77, 64),
+])
+@pytest.mark.parametrize('noise', [None, 'jax.uniform'])
+def test_float32_pipelines_match_the_oracle(gpu, reduce, rows, cols, noise):
+  """float32 values and scales: rows and tiles, and the re-quantization of int8 values in float32 arithmetic, with
+  noise counters in memory order and in the order of the transposed tensor."""
+  key = prng.prng_key(31)
+  q = R.QuantizerCfg(bits=8, noise=noise, key=key)
+  qb, cb = U.bounds(q)
+  by_row = reduce == L.REDUCE_COLS
+  kw = dict(reduce=reduce, out_dtype=L.I8, quant_bound=qb, clip_bound=cb, noise=U.NOISE[noise], key=key,
+            transpose_out=not by_row)
+  x = U.rand((1, rows, cols), 'f32', seed=rows + cols, outliers=True)
+  qt = R.quantize(x, 'f32', q, [2 if by_row else 1])
+  qg, sg = ops.quantize(U.to_dev(x, 'f32', gpu), **kw)
+  _check(qt, qg.cpu().numpy(), sg.cpu().numpy(), q, transpose=not by_row)
+  if by_row:
+    return
+  w = np.random.default_rng(rows).integers(-127, 128, size=(cols, rows)).astype(np.int8)  # logical [cols, rows]
+  qt = R.quantize(w.astype(np.float32)[None], 'f32', q, [2])
+  qg, sg = ops.quantize(torch.from_numpy(np.ascontiguousarray(w.T)[None]).to(gpu), compute_dtype=torch.float32,
+                        noise_strides=(rows * cols, 1, rows), noise_total=rows * cols, **kw)
+  _check(qt, qg.cpu().numpy(), sg.cpu().numpy(), q)
