@@ -292,6 +292,17 @@ int aqtx_gemm_i8(const aqtx_gemm_plan* plan, const void* a, const void* b,
 int aqtx_gemm_i8_k_slices(const aqtx_gemm_plan* plan);
 
 /*
+ * aqtx_pad_rows: byte rows [batch][rows][k] of one or two contraction operands (b_out NULL: of `a` alone), rows `ld`
+ * and batch entries `stride` bytes apart and aligned in any way, copied to [batch][rows][16 * ceil(k / 16)] with zeros
+ * behind k: operands of aqtx_gemm_i8 / aqtx_gemm_fp8 whose k, leading dimensions or addresses are no multiples of
+ * 16 become ones that its matrix instructions take (k padded; a zero byte is the value 0 in int8 and both fp8 types), instead of one
+ * thread per output element.  No counterpart in the reference (XLA pads its own operands).
+ *   a_out, b_out : 16-byte aligned, batch * rows * 16 * ceil(k / 16) bytes
+ */
+int aqtx_pad_rows(int64_t batch, int64_t k, const void* a, int64_t rows_a, int64_t lda, int64_t stride_a, void* a_out,
+                  const void* b, int64_t rows_b, int64_t ldb, int64_t stride_b, void* b_out, void* stream);
+
+/*
  * aqtx_gemm_weight_only: c[m, n] = bf16(bf16(sum_k a[m, k] * float(b[n, k])) * col_scale[n]) for bf16
  * activations that are NOT quantized and an int8 (or int4 in int8 containers) weight, any m.  Replaces
  * _qtensor_dot_general with an unquantized lhs (aqt/jax/v2/aqt_dot_general.py:843-958: the quantized rhs is

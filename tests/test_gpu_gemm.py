@@ -549,3 +549,37 @@ def test_weight_only_gemm_fragment_ordered_b(gpu):
   want = ops.gemm_weight_only(a, b, cs)
   got = ops.gemm_weight_only(a, ops.tile_weight(b[0], L.I8), cs, b_layout=L.W_FRAGMENTS)
   assert torch.equal(got, want)  # the same products added in the same order
+
+
+@pytest.mark.parametrize('batch,m,n,k', [(1, 257, 129, 129), (1, 64, 65, 1), (2, 70, 66, 65), (1, 300, 1, 1007), (1, 1, 301, 2047),
+                                         (1, 513, 259, 4096 + 15), (1, 259, 1031, 144)])
+@pytest.mark.parametrize('kind', ['i8', 'e4m3', 'e5m2'])
+@pytest.mark.parametrize('view', ['dense', 'wide_rows', 'off_by_one'])
+def test_operands_the_mfma_kernels_cannot_load_are_padded(gpu, batch, m, n, k, kind, view):
+  """k, row pitches and addresses that are no multiples of 16, with bytes around the rows that must not be read as part of
+  them; small integers, whose sums every format and order of summation holds exactly.  Output rows of odd length."""
+  rng = np.random.default_rng(batch + m + n + k)
+  pitch = k + (3 if view == 'wide_rows' else 0)
+  off = 1 if view == 'off_by_one' else 0
+  dt = {'i8': L.I8, 'e4m3': L.E4M3, 'e5m2': L.E5M2}[kind]
+
+  def operand(rows):
+    v = rng.integers(-2, 3, size=(batch, rows, k)).astype(np.int8)
+    buf = torch.full((off + batch * rows * pitch + 16,), 0x3F, dtype=torch.uint8, device=gpu)
+    t = torch.from_numpy(v).to(gpu)
+    t = t if kind == 'i8' else t.float().to({'e4m3': torch.float8_e4m3fn, 'e5m2': torch.float8_e5m2}[kind])
+    buf[off:off + batch * rows * pitch].view(batch, rows, pitch)[:, :, :k] = t.view(torch.uint8)
+    x = buf[off:off + batch * rows * pitch].view(batch, rows, pitch)[:, :, :k]
+    return v, x.view(torch.int8) if kind == 'i8' else x
+
+  a, ta = operand(m)
+  b, tb = operand(n)
+  acc = _ref_acc(a, b)
+  assert np.abs(acc).max() < 2 ** 24
+  rs = np.exp2(rng.integers(-3, 4, size=(batch, m))).astype(np.float32)
+  cs = np.exp2(rng.integers(-3, 4, size=(batch, n))).astype(np.float32)
+  for out in (torch.float32, torch.bfloat16):
+    c = ops.gemm(ta, tb, row_scale=torch.from_numpy(rs).to(gpu), col_scale=torch.from_numpy(cs).to(gpu), out_dtype=out,
+                 a_dtype=dt, b_dtype=dt)
+    want = torch.from_numpy(acc.astype(np.float32)).to(out).float() * torch.from_numpy(rs)[:, :, None] * torch.from_numpy(cs)[:, None, :]
+    assert torch.equal(c.float().cpu(), want), out
