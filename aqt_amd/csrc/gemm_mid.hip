@@ -588,7 +588,7 @@ void gemm_mid_kernel(const GemmArgs g_in) {
   }
 
   // ---- epilogue: lane holds C[m = wm*32*IM + im*32 + lr][n = wn*32*IN + ni*32 + 8q + 4lh + e], register 4q + e of tile (im, ni)
-  // Where rows of C start 16-byte aligned, a wave passes its part of the tile through LDS (a region of its own
+  // Unless the raw accumulators are asked for as well, a wave passes its part of the tile through LDS (a region of its own
   // in the stage buffers, which nobody reads any more) so that the stores are 16 bytes a lane along whole row
   // segments: straight from the accumulator layout a store instruction touches 16 bytes in each of 32 rows.
   if constexpr (!SLAB) {
@@ -599,8 +599,7 @@ void gemm_mid_kernel(const GemmArgs g_in) {
     constexpr bool kStagedFits = DIRECT ? ((S::kWaves + NB - 1) / (DIRECT ? NB : 1)) * kWaveBytes <= kStage
                                         : S::kWaves * kWaveBytes <= NBUF * kStage;
     static_assert(DIRECT || kStagedFits, "the staged tile fits the stage buffers");
-    const bool staged = kStagedFits && g.acc_out == nullptr && ((g.ldc * kEsz) % 16) == 0 && ((g.stride_c * kEsz) % 16) == 0 &&
-                        ((uintptr_t)g.c % 16) == 0 && ((n0 * kEsz) % 16) == 0;
+    const bool staged = kStagedFits && g.acc_out == nullptr;
     if (staged) {
       lds_barrier();
       uint8_t* mine = DIRECT ? ring(wave % (DIRECT ? NB : 1)) + (wave / (DIRECT ? NB : 1)) * kWaveBytes : stage_mem + wave * kWaveBytes;
@@ -661,7 +660,7 @@ void gemm_mid_kernel(const GemmArgs g_in) {
         if (mm >= g.m || nn >= g.n) continue;
         uint8_t* dst = reinterpret_cast<uint8_t*>(g.c) + (bz * g.stride_c + mm * g.ldc + nn) * kEsz;
         if (nn + kPerLane <= g.n) {
-          *reinterpret_cast<v4i*>(dst) = val;
+          *reinterpret_cast<v4i_unaligned*>(dst) = val;
         } else {
           for (int e = 0; e < kPerLane && nn + e < g.n; ++e) {
             if constexpr (kEsz == 2) reinterpret_cast<uint16_t*>(dst)[e] = (uint16_t)((uint32_t)val[e >> 1] >> (16 * (e & 1)));
