@@ -342,3 +342,41 @@ def test_float32_pipelines_match_the_oracle(gpu, reduce, rows, cols, noise):
   qg, sg = ops.quantize(torch.from_numpy(np.ascontiguousarray(w.T)[None]).to(gpu), compute_dtype=torch.float32,
                         noise_strides=(rows * cols, 1, rows), noise_total=rows * cols, **kw)
   _check(qt, qg.cpu().numpy(), sg.cpu().numpy(), q)
+
+
+@pytest.mark.parametrize('rows,cols', [
+    # around the pieces of 8, the launch shapes of the rows kernel and the 128 x 64 tiles (halved where two tiles share
+    # the blocks of the generator); fewer than a piece or a tile
+    (3, 7), (2, 9), (130, 63), (127, 65), (128, 129), (257, 130), (258, 67), (254, 126), (6, 511), (4, 2049), (2, 4099), (3, 8193),
+    (2, 16383), (9, 1),
+])
+@pytest.mark.parametrize('bits,noise', [(8, None), (8, 'jax.uniform'), ('e5m2', 'sr'), ('e4m3', None)])
+@pytest.mark.parametrize('dt', ['bf16', 'f32'])
+def test_sizes_that_are_no_multiples_of_anything(gpu, dt, bits, noise, rows, cols):
+  """Scales by row, by column and by tensor, written in the input's order and transposed, two batch entries where the
+  noise does not pair tiles, and a prescale along the other axis."""
+  key = prng.prng_key(rows * 7 + cols)
+  q = R.QuantizerCfg(bits=bits, key=key)
+  if noise == 'sr':
+    q.fp8_sr = True
+  elif noise:
+    q.noise = noise
+  kn = {None: L.NOISE_NONE, 'sr': L.NOISE_FP8_MANTISSA}.get(noise, U.NOISE.get(noise))
+  qb, cb = U.bounds(q)
+  kw = dict(out_dtype=U.OUT_DT[bits], quant_bound=qb, clip_bound=cb, noise=kn, key=key)
+  for batch in (1, 2):
+    x = U.rand((batch, rows, cols), dt, seed=rows + cols, outliers=True)
+    xd = U.to_dev(x, dt, gpu)
+    for reduce, axes, transpose in ((L.REDUCE_COLS, [2], False), (L.REDUCE_ROWS, [1], False), (L.REDUCE_ROWS, [1], True),
+                                    (L.REDUCE_ALL, [1, 2], True)):
+      qg, sg = ops.quantize(xd, reduce=reduce, transpose_out=transpose, **kw)
+      _check(R.quantize(x, dt, q, axes), qg.cpu().numpy(), sg.cpu().numpy(), q, transpose=transpose)
+  ps = nm.cast(np.abs(U.rand((cols,), 'f32', 3, 0.03)) + np.float32(1e-3), dt)
+  x = x[:1]
+  qg, sg = ops.quantize(xd[:1].contiguous(), reduce=L.REDUCE_COLS, prescale=torch.from_numpy(ps).to(gpu),
+                        prescale_mode=L.PRESCALE_PER_COL, **kw)
+  _check(_oracle_quant(x, dt, q, [2], ps, 2), qg.cpu().numpy(), sg.cpu().numpy(), q)
+  ps = nm.cast(np.abs(U.rand((rows,), 'f32', 4, 0.03)) + np.float32(1e-3), dt)
+  qg, sg = ops.quantize(xd[:1].contiguous(), reduce=L.REDUCE_ROWS, transpose_out=True, prescale=torch.from_numpy(ps).to(gpu),
+                        prescale_mode=L.PRESCALE_PER_ROW, **kw)
+  _check(_oracle_quant(x, dt, q, [1], ps, 1), qg.cpu().numpy(), sg.cpu().numpy(), q, transpose=True)
