@@ -247,6 +247,10 @@ extern "C" int aqtx_quantize(const aqtx_quant_plan* p, const void* x, const floa
       a.G = p->rows; a.ngroups = 1;
       a.ssb = p->reduce == AQTX_REDUCE_ALL ? 1 : 0; a.ssg = 0; a.ssc = 0;
     }
+    // Room behind the abs-max words of a kept workspace (zero like them): the arrival counts of the abs-max blocks, one
+    // column group of its blocks, or one per batch entry
+    const int64_t groups = p->reduce == AQTX_REDUCE_ROWS ? p->batch * a.ngroups * absmax_col_groups(p->cols) : p->batch;
+    if (p->workspace_zeroed && (int64_t)(workspace_bytes / 8) >= nscales + groups) a.ws_arrived = a.ws_absmax + (workspace_bytes / 8) - groups;
     const int64_t grid_y = p->reduce != AQTX_REDUCE_ROWS
                                ? (p->rows + kTileR - 1) / kTileR
                                : a.ngroups * ((a.G + kAbsRowChunk - 1) / kAbsRowChunk);

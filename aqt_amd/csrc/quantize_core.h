@@ -33,6 +33,9 @@ struct QArgs {
   uint16_t* scale_bf16;  // optional second copy of the computed scales as bf16 elements
   uint32_t* ws_absmax;
   float* ws_inv;
+  // Arrival counts of the abs-max blocks, zero on entry and exit, one per group of blocks that share scales: the last
+  // block of a group turns its maxima into scales.  NULL: finalize_scales_kernel does, in a launch of its own.
+  uint32_t* ws_arrived;
   int64_t batch, rows, cols;
   int64_t L;        // rows kernel: segment length
   int64_t nseg;     // rows kernel: number of segments
@@ -67,6 +70,13 @@ struct QArgs {
 constexpr int64_t kColmaxBlocks = 7 * 256;
 
 constexpr int kTileR = 128, kTileC = 64, kTilePad = 132;
+
+// Column abs-max: a block takes 64 lanes x 8 columns (1 where there are fewer than 8) and 64 rows of them.
+constexpr int kAbsRowChunk = 64, kAbsColLanes = 64;
+inline int64_t absmax_col_groups(int64_t cols) {
+  const int64_t width = kAbsColLanes * (cols >= 8 ? 8 : 1);
+  return (cols + width - 1) / width;
+}
 
 // Launches the passes of one plan for one input type.
 int launch_quantize_f32(const QArgs& a, int reduce, int partitionable, int64_t nscales, hipStream_t st);
@@ -608,18 +618,57 @@ __global__ void fill_u32_kernel(uint32_t* p, int64_t n, uint32_t v) {
   if (i < n) p[i] = v;
 }
 
-constexpr int kAbsRowChunk = 64;
 
-// Column abs-max: block = 4 waves x (64 lanes x VEC cols); the waves interleave
+// What the last block of a group finds out: whether every block of it has merged its maxima.  The atomics are
+// read-modify-writes, carried out at the memory side of the per-XCD L2s, and every thread has waited for the value its
+// own returned before the barrier in front of the count, so the exchange needs no fence (each of the group's words is
+// read by one more read-modify-write).
+__device__ __forceinline__ bool last_arrival(uint32_t* arrived, uint32_t blocks, int* flag) {
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const uint32_t before = __hip_atomic_fetch_add(arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    *flag = before + 1u == blocks;
+    if (before + 1u == blocks) __hip_atomic_fetch_and(arrived, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __syncthreads();
+  return *flag != 0;
+}
+
+// Merges one maximum; the wait for the returned value orders it before last_arrival's count.
+__device__ __forceinline__ void merge_absmax(uint32_t* word, float m) {
+  const uint32_t before = __hip_atomic_fetch_max(word, __float_as_uint(m), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  asm volatile("" ::"v"(before));
+}
+
+// Scale (output) and reciprocal scale (workspace) of index i from the merged maximum, whose word goes back to zero.
+__device__ __forceinline__ void finalize_merged(const QArgs& a, int64_t i) {
+  const uint32_t w = __hip_atomic_fetch_and(a.ws_absmax + i, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  float scale, inv;
+  scale_from_absmax(__uint_as_float(w), a, scale, inv);
+  store_scale(a, i, scale);
+  a.ws_inv[i] = inv;
+}
+
+// Column abs-max: block = WAVES waves x (64 lanes x VEC cols); the waves interleave
 // over the rows of one chunk, partial maxima meet in LDS and leave through one
 // atomic max per column (|x| >= 0, so the float bit pattern orders like a uint).
-template <typename TIn, int VEC>
-__global__ __launch_bounds__(256) void absmax_cols_kernel(const QArgs a) {
-  __shared__ float smem[4][64 * VEC];
+// Bound by HBM bytes on large inputs, by the latency of loads, atomics and launches on small ones.  A wave requests four
+// rows before it uses the first (bf16 without a prescale).  FOLD, for launches of few blocks: 16 waves in each, whose one
+// round of requests is the whole chunk, and the last block of a column group to arrive computes its scales (QArgs::ws_arrived),
+// which spares finalize_scales_kernel, 4 to 5 us mostly of gap: 512 to 2048 columns take 6-12 us instead of 9-14 and that
+// launch.  On a chip full of blocks both cost more than they give, as blocks wait at barriers and for the atomics' returns:
+// 8192 x 14336 with a prescale 61-88 us against 57 and the launch.  Chunks of 16 rows, for more blocks, take four times the
+// atomics (4096 x 2048 float32: 22 us against 12).
+template <typename TIn, int VEC, bool FOLD>
+__global__ __launch_bounds__(FOLD ? 1024 : 256) void absmax_cols_kernel(const QArgs a) {
+  constexpr int WAVES = FOLD ? 16 : 4;
+  constexpr int WIDTH = kAbsColLanes * VEC;
+  __shared__ float smem[WAVES][WIDTH];
+  __shared__ int last;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   // a lane's columns; where eight would hang over the end, the last eight of the row (met twice: same maximum)
   auto columns_at = [&](int64_t l) -> int64_t {
-    const int64_t c = ((int64_t)blockIdx.x * 64 + l) * VEC;
+    const int64_t c = (int64_t)blockIdx.x * WIDTH + l * VEC;
     return c >= a.cols ? a.cols : c + VEC <= a.cols ? c : a.cols - VEC;
   };
   const int64_t c0 = columns_at(lane);
@@ -630,50 +679,91 @@ __global__ __launch_bounds__(256) void absmax_cols_kernel(const QArgs a) {
   const int64_t r_begin = g * a.G + chunk * kAbsRowChunk;
   int64_t r_end = r_begin + kAbsRowChunk;
   if (r_end > (g + 1) * a.G) r_end = (g + 1) * a.G;
+  constexpr int AHEAD = 4;  // rows of a wave in flight
   float m[VEC];
 #pragma unroll
   for (int e = 0; e < VEC; ++e) m[e] = 0.0f;
   if (c0 < a.cols) {
-    float ps[VEC];
-#pragma unroll
-    for (int e = 0; e < VEC; ++e) ps[e] = 1.0f;
-    if (a.ps_mode == AQTX_PRESCALE_PER_COL) {
-#pragma unroll
-      for (int e = 0; e < VEC; ++e) ps[e] = a.prescale[b * a.psb + c0 + e];
-    }
     const TIn* xb = reinterpret_cast<const TIn*>(a.x) + b * a.rows * a.cols + c0;
-    for (int64_t r = r_begin + wave; r < r_end; r += 4) {
-      float v[VEC];
-      if constexpr (VEC == 8) Loader<TIn>::load8(xb + r * a.cols, v);
-      else v[0] = Loader<TIn>::load1(xb + r * a.cols);
-      if (a.ps_mode == AQTX_PRESCALE_PER_ROW) {
-        const float rp = a.prescale[b * a.psb + r];
+    bool done = false;
+    if constexpr (VEC == 8 && sizeof(TIn) == 2) {
+      if (a.ps_mode == AQTX_PRESCALE_NONE) {  // bf16 magnitudes order like unsigned integers, two per instruction
+        done = true;
+        uint32_t mw[4] = {0u, 0u, 0u, 0u};
+        auto meet = [&](const uint4& w) {
+          mw[0] = packed_absmax(mw[0], w.x); mw[1] = packed_absmax(mw[1], w.y);
+          mw[2] = packed_absmax(mw[2], w.z); mw[3] = packed_absmax(mw[3], w.w);
+        };
+        int64_t r = r_begin + wave;
+        for (; r + WAVES * (AHEAD - 1) < r_end; r += WAVES * AHEAD) {
+          uint4 w[AHEAD];
 #pragma unroll
-        for (int e = 0; e < VEC; ++e) v[e] = apply_prescale(v[e], rp, a);
-      } else if (a.ps_mode == AQTX_PRESCALE_PER_COL) {
+          for (int u = 0; u < AHEAD; ++u) w[u] = load_unaligned<uint4>(xb + (r + WAVES * u) * a.cols);
 #pragma unroll
-        for (int e = 0; e < VEC; ++e) v[e] = apply_prescale(v[e], ps[e], a);
+          for (int u = 0; u < AHEAD; ++u) meet(w[u]);
+        }
+        for (; r < r_end; r += WAVES) meet(load_unaligned<uint4>(xb + r * a.cols));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          m[2 * i] = __uint_as_float(mw[i] << 16);
+          m[2 * i + 1] = __uint_as_float(mw[i] & 0xFFFF0000u);
+        }
       }
+    }
+    if (!done) {
+      float ps[VEC];
 #pragma unroll
-      for (int e = 0; e < VEC; ++e) m[e] = absmax_step(m[e], v[e]);
+      for (int e = 0; e < VEC; ++e) ps[e] = 1.0f;
+      if (a.ps_mode == AQTX_PRESCALE_PER_COL) {
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) ps[e] = a.prescale[b * a.psb + c0 + e];
+      }
+      for (int64_t r = r_begin + wave; r < r_end; r += WAVES) {
+        float v[VEC];
+        if constexpr (VEC == 8) Loader<TIn>::load8(xb + r * a.cols, v);
+        else v[0] = Loader<TIn>::load1(xb + r * a.cols);
+        if (a.ps_mode == AQTX_PRESCALE_PER_ROW) {
+          const float rp = a.prescale[b * a.psb + r];
+#pragma unroll
+          for (int e = 0; e < VEC; ++e) v[e] = apply_prescale(v[e], rp, a);
+        } else if (a.ps_mode == AQTX_PRESCALE_PER_COL) {
+#pragma unroll
+          for (int e = 0; e < VEC; ++e) v[e] = apply_prescale(v[e], ps[e], a);
+        }
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) m[e] = absmax_step(m[e], v[e]);
+      }
     }
   }
 #pragma unroll
   for (int e = 0; e < VEC; ++e) smem[wave][lane * VEC + e] = m[e];
   __syncthreads();
-  for (int i = threadIdx.x; i < 64 * VEC; i += 256) {
+  for (int i = threadIdx.x; i < WIDTH; i += 64 * WAVES) {
     const int64_t first = columns_at(i / VEC), c = first + i % VEC;
-    if (first < a.cols) {
-      const float mm = nanmax(nanmax(smem[0][i], smem[1][i]), nanmax(smem[2][i], smem[3][i]));
-      atomicMax(a.ws_absmax + b * a.ssb + g * a.ssg + c * a.ssc, __float_as_uint(mm));
+    // (columns a last group of fewer than eight borrows from the group before it belong to that one's blocks)
+    if (first < a.cols && c >= (int64_t)blockIdx.x * WIDTH) {
+      float mm = smem[0][i];
+#pragma unroll
+      for (int w = 1; w < WAVES; ++w) mm = nanmax(mm, smem[w][i]);
+      uint32_t* word = a.ws_absmax + b * a.ssb + g * a.ssg + c * a.ssc;
+      if constexpr (FOLD) merge_absmax(word, mm);
+      else atomicMax(word, __float_as_uint(mm));
     }
+  }
+  if constexpr (FOLD) {
+    if (!last_arrival(a.ws_arrived + (b * a.ngroups + g) * gridDim.x + blockIdx.x, (uint32_t)chunks_per_group, &last)) return;
+    const int64_t end = (int64_t)(blockIdx.x + 1) * WIDTH;
+    for (int64_t c = (int64_t)blockIdx.x * WIDTH + threadIdx.x; c < end && c < a.cols; c += 64 * WAVES)
+      finalize_merged(a, b * a.ssb + g * a.ssg + c * a.ssc);
   }
 }
 
-// Whole-tensor abs-max per batch entry.
+// Whole-tensor abs-max per batch entry (one entry for the whole batch where the batch shares its scale).
+constexpr int kAbsThreads = 1024;
 template <typename TIn>
-__global__ __launch_bounds__(256) void absmax_all_kernel(const QArgs a) {
-  __shared__ float smem[4];
+__global__ __launch_bounds__(kAbsThreads) void absmax_all_kernel(const QArgs a) {
+  __shared__ float smem[kAbsThreads / 64];
+  __shared__ int last;
   const int64_t b = blockIdx.y;
   const int64_t n = a.rows * a.cols;
   const TIn* xb = reinterpret_cast<const TIn*>(a.x) + b * n;
@@ -681,36 +771,64 @@ __global__ __launch_bounds__(256) void absmax_all_kernel(const QArgs a) {
   if (n >= 8 && (a.ps_mode == AQTX_PRESCALE_NONE || a.cols % 8 == 0)) {
     // 8 elements per lane and load (with a prescale: of one row); the last eight of the entry are met twice where their
     // number is no multiple of 8
-    const int64_t stride = (int64_t)gridDim.x * 256 * 8;
+    const int64_t stride = (int64_t)gridDim.x * kAbsThreads * 8;
+    const int64_t j0 = ((int64_t)blockIdx.x * kAbsThreads + threadIdx.x) * 8;
+    bool done = false;
+    if constexpr (sizeof(TIn) == 2) {
+      if (a.ps_mode == AQTX_PRESCALE_NONE) {
+        done = true;
+        uint32_t mw[4] = {0u, 0u, 0u, 0u};
 #pragma unroll 4
-    for (int64_t j = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 8; j < n; j += stride) {
-      const int64_t i = j + 8 <= n ? j : n - 8;
-      float v[8];
-      Loader<TIn>::load8(xb + i, v);
-      if (a.ps_mode == AQTX_PRESCALE_PER_ROW) {
-        const float rp = a.prescale[b * a.psb + i / a.cols];
+        for (int64_t j = j0; j < n; j += stride) {
+          const uint4 w = load_unaligned<uint4>(xb + (j + 8 <= n ? j : n - 8));
+          mw[0] = packed_absmax(mw[0], w.x); mw[1] = packed_absmax(mw[1], w.y);
+          mw[2] = packed_absmax(mw[2], w.z); mw[3] = packed_absmax(mw[3], w.w);
+        }
 #pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = apply_prescale(v[e], rp, a);
-      } else if (a.ps_mode == AQTX_PRESCALE_PER_COL) {
-        const float* pc = a.prescale + b * a.psb + i % a.cols;
-        float ps[8];
-        Loader<float>::load8(pc, ps);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = apply_prescale(v[e], ps[e], a);
+        for (int i = 0; i < 4; ++i)
+          m = nanmax(m, nanmax(__uint_as_float(mw[i] << 16), __uint_as_float(mw[i] & 0xFFFF0000u)));
       }
+    }
+    if (!done) {
+#pragma unroll 4
+      for (int64_t j = j0; j < n; j += stride) {
+        const int64_t i = j + 8 <= n ? j : n - 8;
+        float v[8];
+        Loader<TIn>::load8(xb + i, v);
+        if (a.ps_mode == AQTX_PRESCALE_PER_ROW) {
+          const float rp = a.prescale[b * a.psb + i / a.cols];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) m = absmax_step(m, v[e]);
+          for (int e = 0; e < 8; ++e) v[e] = apply_prescale(v[e], rp, a);
+        } else if (a.ps_mode == AQTX_PRESCALE_PER_COL) {
+          float ps[8];
+          Loader<float>::load8(a.prescale + b * a.psb + i % a.cols, ps);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) v[e] = apply_prescale(v[e], ps[e], a);
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) m = absmax_step(m, v[e]);
+      }
     }
   } else {
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
+    for (int64_t i = (int64_t)blockIdx.x * kAbsThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kAbsThreads) {
       float v = Loader<TIn>::load1(xb + i);
       if (a.ps_mode == AQTX_PRESCALE_PER_ROW) v = apply_prescale(v, a.prescale[b * a.psb + i / a.cols], a);
       else if (a.ps_mode == AQTX_PRESCALE_PER_COL) v = apply_prescale(v, a.prescale[b * a.psb + i % a.cols], a);
       m = absmax_step(m, v);
     }
   }
-  m = segment_max<256>(m, smem);
-  if (threadIdx.x == 0) atomicMax(a.ws_absmax + b * a.ssb, __float_as_uint(m));
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) m = nanmax(m, __shfl_xor(m, off, 64));
+  if ((threadIdx.x & 63) == 0) smem[threadIdx.x >> 6] = m;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int w = 1; w < kAbsThreads / 64; ++w) m = nanmax(m, smem[w]);
+    merge_absmax(a.ws_absmax + b * a.ssb, m);
+  }
+  if (a.ws_arrived == nullptr) return;
+  const uint32_t blocks = a.ssb != 0 ? gridDim.x : gridDim.x * gridDim.y;
+  if (last_arrival(a.ws_arrived + b * a.ssb, blocks, &last) && threadIdx.x == 0) finalize_merged(a, b * a.ssb);
 }
 
 // abs-max bit patterns -> scale (output) and reciprocal scale (workspace).
@@ -820,6 +938,19 @@ __global__ __launch_bounds__(256) void quant_tile_kernel(const QArgs a_in) {
   // Tiles that lie wholly inside the tensor (and inside the first half of a paired axis) take a
   // branch-free path with vector loads of the reciprocal scales and the pre-scale factors.
   const bool interior = (r0[0] + kTileR <= row_lim) && (c0[0] + kTileC <= col_lim) && a.ssc <= 1;
+  // Given scales: the tile's reciprocals are computed here (LDS), where the rows of a column share one
+  __shared__ float inv_lds[NSET][kTileC];
+  const bool inv_here = a.scale_given && a.ngroups == 1;
+  if (inv_here) {
+    if (tid < kTileC) {
+#pragma unroll
+      for (int s = 0; s < NSET; ++s) {
+        const int64_t c = c0[s] + tid;
+        inv_lds[s][tid] = c < a.cols ? inv_of_scale(a.scale[b * a.ssb + c * a.ssc], a) : 1.0f;
+      }
+    }
+    __syncthreads();
+  }
   uint32_t rowmax = 0u;  // ROWMAX: byte j = largest |q| of row r0 + 4 * rg + j among the tile's 64 columns
   auto rows = [&](auto fast_tag) {
     constexpr bool FAST = decltype(fast_tag)::value;
@@ -859,7 +990,10 @@ __global__ __launch_bounds__(256) void quant_tile_kernel(const QArgs a_in) {
               else if (e < nvalid) x[s][e] = spec_prescale<SPEC>(x[s][e], a.prescale[b * a.psb + c + e], a);
             }
           }
-          if constexpr (FAST) {
+          if (inv_here) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) inv[s][e] = inv_lds[s][cc * 8 + e];
+          } else if constexpr (FAST) {
             if (a.ssc == 0) {
               const float v = a.ws_inv[sbase];
 #pragma unroll
@@ -1076,39 +1210,41 @@ int launch_tiles(const QArgs& a, int reduce, int partitionable, int64_t nscales,
     finalize_partials_kernel<<<dim3((unsigned)(nscales / 16)), 256, 0, st>>>(a, nscales);
     AQTX_HIP_CHECK_LAUNCH("finalize_partials_kernel");
   } else {
+  bool folded = false;  // the abs-max launch leaves the scales itself
   if (!a.scale_given) {
     if (!a.ws_zeroed) {
       fill_u32_kernel<<<dim3((unsigned)((nscales + 255) / 256)), 256, 0, st>>>(a.ws_absmax, nscales, 0u);
       AQTX_HIP_CHECK_LAUNCH("fill_u32_kernel");
     }
     if (reduce == AQTX_REDUCE_ALL || reduce == AQTX_REDUCE_ALL_BATCH) {
-      int64_t nblk = (a.rows * a.cols + 256 * 16 - 1) / (256 * 16);
-      // Every block ends in one atomic max.  Atomics on one address take turns (about 10 ns each,
-      // measured), and so do those on the neighbouring words of the batch entries, which share a
-      // cache line: 32 entries x 98 blocks took 31 us for 26 MB.  So the launch as a whole gets at
-      // most one block per 48 KiB of input (the time to stream that much), between 256 and 2048.
+      // Every block ends in two atomics (its maximum and its arrival).  Atomics on one address take turns (about 10 ns
+      // each, measured), and so do those on the neighbouring words of the batch entries, which share a cache line: 32
+      // entries x 98 blocks took 31 us for 26 MB.  So the launch as a whole gets at most one block per 96 KiB of input
+      // (the time to stream that much), and no more than two of them, 16 waves each, on a CU.
+      int64_t nblk = (a.rows * a.cols + kAbsThreads * 8 - 1) / (kAbsThreads * 8);
       const int64_t total_bytes = a.batch * a.rows * a.cols * (int64_t)sizeof(TIn);
-      int64_t cap_total = total_bytes / (48 << 10);
-      cap_total = cap_total < 256 ? 256 : cap_total > 2048 ? 2048 : cap_total;
+      int64_t cap_total = total_bytes / (96 << 10);
+      cap_total = cap_total < 64 ? 64 : cap_total > 512 ? 512 : cap_total;
       const int64_t cap = a.batch >= cap_total ? 1 : cap_total / a.batch;
       if (nblk > cap) nblk = cap;
       if (nblk < 1) nblk = 1;
-      absmax_all_kernel<TIn><<<dim3((unsigned)nblk, (unsigned)a.batch), 256, 0, st>>>(a);
+      folded = a.ws_arrived != nullptr;
+      absmax_all_kernel<TIn><<<dim3((unsigned)nblk, (unsigned)a.batch), kAbsThreads, 0, st>>>(a);
       AQTX_HIP_CHECK_LAUNCH("absmax_all_kernel");
     } else {
-      const int64_t chunks = a.ngroups * ((a.G + kAbsRowChunk - 1) / kAbsRowChunk);
-      if (a.cols >= 8) {
-        dim3 grid((unsigned)((a.cols + 511) / 512), (unsigned)chunks, (unsigned)a.batch);
-        absmax_cols_kernel<TIn, 8><<<grid, 256, 0, st>>>(a);
-      } else {
-        dim3 grid((unsigned)((a.cols + 63) / 64), (unsigned)chunks, (unsigned)a.batch);
-        absmax_cols_kernel<TIn, 1><<<grid, 256, 0, st>>>(a);
-      }
+      const dim3 grid((unsigned)absmax_col_groups(a.cols), (unsigned)(a.ngroups * ((a.G + kAbsRowChunk - 1) / kAbsRowChunk)), (unsigned)a.batch);
+      folded = a.ws_arrived != nullptr && a.cols >= 8 && (int64_t)grid.x * grid.y * grid.z < 1024;
+      if (a.cols < 8) absmax_cols_kernel<TIn, 1, false><<<grid, 256, 0, st>>>(a);
+      else if (folded) absmax_cols_kernel<TIn, 8, true><<<grid, 1024, 0, st>>>(a);
+      else absmax_cols_kernel<TIn, 8, false><<<grid, 256, 0, st>>>(a);
       AQTX_HIP_CHECK_LAUNCH("absmax_cols_kernel");
     }
   }
-  finalize_scales_kernel<<<dim3((unsigned)((nscales + 255) / 256)), 256, 0, st>>>(a, nscales);
-  AQTX_HIP_CHECK_LAUNCH("finalize_scales_kernel");
+  // (given scales shared by whole columns: the tile kernel takes their reciprocals itself)
+  if (a.scale_given ? a.ngroups != 1 : !folded) {
+    finalize_scales_kernel<<<dim3((unsigned)((nscales + 255) / 256)), 256, 0, st>>>(a, nscales);
+    AQTX_HIP_CHECK_LAUNCH("finalize_scales_kernel");
+  }
   }
   const int spec = spec_of(a, partitionable);
   auto grid_for = [&](int pair) {

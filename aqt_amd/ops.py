@@ -112,8 +112,9 @@ def private_workspaces(store: dict):
 def _quantize_workspace(nbytes: int, device) -> torch.Tensor:
   key = (device.index, torch.cuda.current_stream(device).cuda_stream)
   ws = _QUANT_WS.get(key)
-  if ws is None or ws.numel() < nbytes:
-    ws = torch.zeros(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
+  if ws is None or ws.numel() < 2 * nbytes:
+    # with room for the arrival counts of the abs-max blocks (at most one per scale)
+    ws = torch.zeros(max(2 * nbytes, 1 << 20), dtype=torch.uint8, device=device)
     _QUANT_WS[key] = ws
   return ws
 

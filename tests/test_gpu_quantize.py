@@ -380,3 +380,39 @@ def test_sizes_that_are_no_multiples_of_anything(gpu, dt, bits, noise, rows, col
   qg, sg = ops.quantize(xd[:1].contiguous(), reduce=L.REDUCE_ROWS, transpose_out=True, prescale=torch.from_numpy(ps).to(gpu),
                         prescale_mode=L.PRESCALE_PER_ROW, **kw)
   _check(_oracle_quant(x, dt, q, [1], ps, 1), qg.cpu().numpy(), sg.cpu().numpy(), q, transpose=True)
+
+
+@pytest.mark.parametrize('reduce,shape,group', [
+    (L.REDUCE_ROWS, (1, 4096, 600), 0), (L.REDUCE_ROWS, (2, 130, 1025), 0), (L.REDUCE_ROWS, (1, 16, 5), 0),
+    (L.REDUCE_ROWS, (2, 256, 513), 64), (L.REDUCE_ALL, (3, 1000, 257), 0), (L.REDUCE_ALL_BATCH, (3, 1000, 257), 0),
+    (L.REDUCE_ALL_BATCH, (1, 3, 2), 0),
+])
+def test_scales_from_the_last_block_equal_those_of_their_own_launch(gpu, reduce, shape, group):
+  """A kept workspace with room for the arrival counts and one without; calls of other sizes in between leave both as
+  they have to be found (zero); and the same scales given instead of computed."""
+  kw = dict(reduce=reduce, out_dtype=L.I8, quant_bound=127.5, clip_bound=127.0, group=group)
+  x = U.to_dev(U.rand(shape, 'bf16', seed=sum(shape), outliers=True), 'bf16', gpu)
+  y = U.to_dev(U.rand((2, 700, 1300), 'bf16', seed=1), 'bf16', gpu)
+  results = []
+  for room in (True, False):
+    if room:
+      with ops.private_workspaces({}) as store:
+        for _ in range(3):
+          results.append(ops.quantize(x, **kw))
+          ops.quantize(y, reduce=L.REDUCE_ROWS, out_dtype=L.I8, quant_bound=127.5, clip_bound=127.0)
+        words = [t for t in store.values()]
+      assert len(words) == 1 and not bool(words[0][:words[0].numel() // 2].any())
+    else:
+      n = results[0][1].numel()
+      ws = torch.zeros(8 * n, dtype=torch.uint8, device=gpu)
+      with pytest.MonkeyPatch.context() as mp:
+        mp.setattr(ops, '_quantize_workspace', lambda nbytes, device: ws)
+        results.append(ops.quantize(x, **kw))
+      assert not bool(ws[:4 * n].any())
+  results.append(ops.quantize(x, scale=results[0][1], **kw))
+  for q, s in results[1:]:
+    assert torch.equal(q, results[0][0]) and torch.equal(s, results[0][1])
+  want = x.float().abs()
+  want = {L.REDUCE_ROWS: lambda: want.reshape(shape[0], -1, group or shape[1], shape[2]).amax(2), L.REDUCE_ALL: lambda: want.amax((1, 2)),
+          L.REDUCE_ALL_BATCH: lambda: want.amax().reshape(1)}[reduce]()
+  assert torch.equal(results[0][1], (want / 127.5).to(torch.bfloat16).float())
