@@ -41,6 +41,7 @@ class QuantPlan(ctypes.Structure):
       ('out_k_order', ctypes.c_int32),
       ('other_axis_absmax', ctypes.c_void_p),
       ('absmax_partials', ctypes.c_void_p), ('absmax_parts', ctypes.c_int64),
+      ('scale_only', ctypes.c_int32),
   ]
 
 
@@ -95,6 +96,7 @@ class DecodePlan(ctypes.Structure):
       ('quant_bound', ctypes.c_float), ('clip_bound', ctypes.c_float),
       ('w_dtype', ctypes.c_int32), ('tuning', ctypes.c_int32), ('w_layout', ctypes.c_int32),
       ('workspace_zeroed', ctypes.c_int32),
+      ('x_scale_typed', ctypes.c_void_p),
   ]
 
 
@@ -150,6 +152,9 @@ SYMBOLS = {
     'aqtx_sum_tiles': (ctypes.c_int, [_vp, _vp, ctypes.c_int64, ctypes.c_int64, ctypes.c_int32, _vp]),
     'aqtx_prng_split_host': (ctypes.c_int, [ctypes.POINTER(ctypes.c_uint32), ctypes.c_int32,
                                             ctypes.c_int32, ctypes.POINTER(ctypes.c_uint32)]),
+    'aqtx_prng_split2_host': (ctypes.c_int, [ctypes.POINTER(ctypes.c_uint32), ctypes.c_int32, ctypes.c_int32,
+                                             ctypes.c_int32, ctypes.POINTER(ctypes.c_uint32)]),
+    'aqtx_prng_split2': (ctypes.c_int, [_vp, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, _vp, _vp]),
     'aqtx_prng_split': (ctypes.c_int, [_vp, ctypes.c_int32, ctypes.c_int32, _vp, _vp]),
     'aqtx_random_bits': (ctypes.c_int, [ctypes.POINTER(ctypes.c_uint32), ctypes.c_int64,
                                         ctypes.c_int32, ctypes.c_int32, _vp, _vp]),

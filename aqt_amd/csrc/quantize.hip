@@ -175,7 +175,9 @@ extern "C" int aqtx_quantize(const aqtx_quant_plan* p, const void* x, const floa
   if (long_rows_as_batches(p, &alt)) return aqtx_quantize(&alt, x, prescale, q, scale, workspace, workspace_bytes, stream);
   const int64_t total = p->batch * p->rows * p->cols;
   if (total == 0) return 0;
-  AQTX_REQUIRE(x != nullptr && q != nullptr && scale != nullptr, "aqtx_quantize: NULL buffer");
+  AQTX_REQUIRE(x != nullptr && (q != nullptr || p->scale_only) && scale != nullptr, "aqtx_quantize: NULL buffer");
+  AQTX_REQUIRE(!p->scale_only || (p->noise == AQTX_NOISE_NONE && !p->scale_given && p->other_axis_absmax == nullptr),
+               "aqtx_quantize: scale_only goes without noise, a given scale and other_axis_absmax");
   AQTX_REQUIRE((p->prescale == AQTX_PRESCALE_NONE) == (prescale == nullptr),
                "aqtx_quantize: prescale pointer does not match plan->prescale");
   AQTX_REQUIRE(p->batch <= 65535, "aqtx_quantize: batch %lld exceeds 65535", (long long)p->batch);
@@ -194,6 +196,7 @@ extern "C" int aqtx_quantize(const aqtx_quant_plan* p, const void* x, const floa
   a.x = x; a.prescale = prescale; a.q = q; a.scale = scale;
   a.scale_bf16 = (p->scale_typed != nullptr && p->scale_dtype == AQTX_BF16 && !p->scale_given)
                      ? reinterpret_cast<uint16_t*>(p->scale_typed) : nullptr;
+  a.scale_only = p->scale_only;
   a.batch = p->batch; a.rows = p->rows; a.cols = p->cols;
   a.nsb = p->noise_stride_batch; a.nsr = p->noise_stride_row; a.nsc = p->noise_stride_col;
   a.quant_bound = p->quant_bound; a.clip_bound = p->clip_bound;
@@ -331,51 +334,69 @@ extern "C" int aqtx_random_bits(const uint32_t key_host[2], int64_t n, int32_t b
 
 namespace aqtx {
 namespace {
-__global__ __launch_bounds__(256) void prng_split_kernel(const uint32_t* __restrict__ key, int num, int partitionable,
-                                                         uint32_t* __restrict__ out) {
-  const int i = (int)(blockIdx.x * 256 + threadIdx.x);  // word i of the 2 * num
-  if (i >= 2 * num) return;
-  const uint32_t k0 = key[0], k1 = key[1];
+// word i of the 2 * num words of jax.random.split(key, num)
+AQTX_HD uint32_t split_word(uint32_t k0, uint32_t k1, uint32_t num, int partitionable, uint32_t i) {
   if (partitionable) {
-    const U2 b = threefry2x32(k0, k1, 0u, (uint32_t)(i >> 1));
-    out[i] = (i & 1) ? b.y : b.x;
-  } else {
-    BitGen g;
-    g.k0 = k0; g.k1 = k1;
-    g.nwords = 2u * (uint32_t)num; g.half = (uint32_t)num;
-    g.partitionable = 0; g.width = 32;
-    out[i] = g.word_original((uint32_t)i);
+    const U2 b = threefry2x32(k0, k1, 0u, i >> 1);
+    return (i & 1) ? b.y : b.x;
   }
+  BitGen g;
+  g.k0 = k0; g.k1 = k1;
+  g.nwords = 2u * num; g.half = num;
+  g.partitionable = 0; g.width = 32;
+  return g.word_original(i);
+}
+
+// word i of the keys of split(split(key, num)[p], inner), p = 0 .. num - 1; inner 0: of split(key, num)
+AQTX_HD uint32_t split2_word(uint32_t k0, uint32_t k1, uint32_t num, uint32_t inner, int partitionable, uint32_t i) {
+  if (inner == 0) return split_word(k0, k1, num, partitionable, i);
+  const uint32_t p = i / (2 * inner);
+  const uint32_t c0 = split_word(k0, k1, num, partitionable, 2 * p), c1 = split_word(k0, k1, num, partitionable, 2 * p + 1);
+  return split_word(c0, c1, inner, partitionable, i % (2 * inner));
+}
+
+// Bound by its launch: the whole fan-out of a step's key (one split and a split of each part) in one instead of four,
+// which spares a recorded step 4 us a launch.
+__global__ __launch_bounds__(256) void prng_split_kernel(const uint32_t* __restrict__ key, int num, int inner, int partitionable,
+                                                         uint32_t* __restrict__ out) {
+  const int i = (int)(blockIdx.x * 256 + threadIdx.x);
+  if (i >= 2 * num * (inner > 0 ? inner : 1)) return;
+  out[i] = split2_word(key[0], key[1], (uint32_t)num, (uint32_t)inner, partitionable, (uint32_t)i);
 }
 }  // namespace
 }  // namespace aqtx
 
-extern "C" int aqtx_prng_split(const uint32_t* key_device, int32_t num, int32_t partitionable, uint32_t* out_device,
-                               void* stream) {
+extern "C" int aqtx_prng_split2(const uint32_t* key_device, int32_t num, int32_t inner, int32_t partitionable,
+                                uint32_t* out_device, void* stream) {
   clear_error();
-  AQTX_REQUIRE(num >= 0 && num <= (1 << 20), "aqtx_prng_split: num outside 0..2^20");
+  AQTX_REQUIRE(num >= 0 && num <= (1 << 20) && inner >= 0 && (int64_t)num * inner <= (1 << 20),
+               "aqtx_prng_split: num or num * inner outside 0..2^20");
   if (num == 0) return 0;
   AQTX_REQUIRE(key_device != nullptr && out_device != nullptr, "aqtx_prng_split: NULL argument");
-  prng_split_kernel<<<(unsigned)((2 * num + 255) / 256), 256, 0, reinterpret_cast<hipStream_t>(stream)>>>(
-      key_device, num, partitionable, out_device);
+  const int words = 2 * num * (inner > 0 ? inner : 1);
+  prng_split_kernel<<<(unsigned)((words + 255) / 256), 256, 0, reinterpret_cast<hipStream_t>(stream)>>>(
+      key_device, num, inner, partitionable, out_device);
   AQTX_HIP_CHECK_LAUNCH("prng_split_kernel");
   return 0;
 }
 
-extern "C" int aqtx_prng_split_host(const uint32_t key_host[2], int32_t num, int32_t partitionable,
-                                    uint32_t* out_host) {
+extern "C" int aqtx_prng_split(const uint32_t* key_device, int32_t num, int32_t partitionable, uint32_t* out_device,
+                               void* stream) {
+  return aqtx_prng_split2(key_device, num, 0, partitionable, out_device, stream);
+}
+
+extern "C" int aqtx_prng_split2_host(const uint32_t key_host[2], int32_t num, int32_t inner, int32_t partitionable,
+                                     uint32_t* out_host) {
   clear_error();
   AQTX_REQUIRE(key_host != nullptr && out_host != nullptr, "aqtx_prng_split_host: NULL argument");
-  AQTX_REQUIRE(num >= 0, "aqtx_prng_split_host: negative num");
-  if (partitionable) {
-    for (int32_t i = 0; i < num; ++i) {
-      U2 b = threefry2x32(key_host[0], key_host[1], 0u, (uint32_t)i);
-      out_host[2 * i] = b.x;
-      out_host[2 * i + 1] = b.y;
-    }
-  } else {
-    BitGen g = make_bitgen(key_host, 2 * (int64_t)num, 32, 0);
-    for (int32_t i = 0; i < 2 * num; ++i) out_host[i] = g.word_original((uint32_t)i);
-  }
+  AQTX_REQUIRE(num >= 0 && inner >= 0, "aqtx_prng_split_host: negative num");
+  const int64_t words = 2 * (int64_t)num * (inner > 0 ? inner : 1);
+  AQTX_REQUIRE(words < (1ll << 31), "aqtx_prng_split_host: too many keys");
+  for (int64_t i = 0; i < words; ++i)
+    out_host[i] = split2_word(key_host[0], key_host[1], (uint32_t)num, (uint32_t)inner, partitionable, (uint32_t)i);
   return 0;
+}
+
+extern "C" int aqtx_prng_split_host(const uint32_t key_host[2], int32_t num, int32_t partitionable, uint32_t* out_host) {
+  return aqtx_prng_split2_host(key_host, num, 0, partitionable, out_host);
 }

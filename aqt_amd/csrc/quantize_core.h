@@ -55,6 +55,7 @@ struct QArgs {
   int sbf;  // scale dtype is bf16
   int scale_given;
   int ws_zeroed;  // the abs-max words of the workspace are zero on entry
+  int scale_only; // the scales are all that is asked for (a calibration on its own): nothing reads or writes q
   int even_odd8;  // rows kernel: bytes of each group of 8 outputs stored as elements 0,2,4,6,1,3,5,7
   // Partial maxima of |q| along the axis that carries the scales, one byte per position of the reduced axis and
   // part (aqtx_quant_plan::other_axis_absmax): written by a launch (oa_out), or read in place of an abs-max pass
@@ -514,6 +515,7 @@ void quant_rows_kernel(const QArgs a_in) {
     }
   }
 
+  if (a.scale_only) return;
   uint8_t* qp0 = reinterpret_cast<uint8_t*>(a.q) + grow[0] * a.cols + col0[0];
   if constexpr (PAIR) {
     uint8_t* qp1 = reinterpret_cast<uint8_t*>(a.q) + grow[1] * a.cols + col0[1];
@@ -603,6 +605,7 @@ __global__ __launch_bounds__(256) void quant_rows_generic_kernel(const QArgs a_i
     scale_from_absmax(amax, a, scale, inv);
     if (lane == 0) store_scale(a, seg, scale);
   }
+  if (a.scale_only) return;
   uint8_t* qp = reinterpret_cast<uint8_t*>(a.q) + grow * a.cols + col0;
   const uint64_t ctr_row = (uint64_t)(b * a.nsb + r * a.nsr + col0 * a.nsc);
   for (int64_t j = lane; j < a.L; j += 64) {
@@ -1246,6 +1249,7 @@ int launch_tiles(const QArgs& a, int reduce, int partitionable, int64_t nscales,
     AQTX_HIP_CHECK_LAUNCH("finalize_scales_kernel");
   }
   }
+  if (a.scale_only) return 0;
   const int spec = spec_of(a, partitionable);
   auto grid_for = [&](int pair) {
     const int64_t rows = pair == 1 ? a.rows / 2 : a.rows, cols = pair == 2 ? a.cols / 2 : a.cols;

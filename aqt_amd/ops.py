@@ -158,6 +158,7 @@ def quantize(
     k_order: int = 0,
     want_other_axis_absmax: bool = False,
     absmax_partials: Optional[torch.Tensor] = None,
+    scale_only: bool = False,
 ):
   """Calibrate (abs-max) and quantize a contiguous [batch, rows, cols] tensor.
 
@@ -176,6 +177,7 @@ def quantize(
   that carries the scales (uint8 [parts, cols] for REDUCE_COLS, [parts, rows] for REDUCE_ROWS) in
   `q.other_axis_absmax`: what a later quantization of q over that axis takes as `absmax_partials` instead of
   reading q for its abs-max (the backward pass re-quantizes the forward residuals that way).
+  scale_only: calibration alone; q comes back as None.
   """
   _require_gpu(x, prescale, scale)
   assert x.dim() == 3 and x.is_contiguous(), 'x must be a contiguous [batch, rows, cols] tensor'
@@ -226,7 +228,8 @@ def quantize(
     assert scale.dtype == torch.float32 and scale.is_contiguous() and tuple(scale.shape) == sshape
   fp8 = out_dtype in (L.E4M3, L.E5M2)
   qshape = (b, c, r) if transpose_out else (b, r, c)
-  q = torch.empty(qshape, dtype=torch.uint8 if fp8 else torch.int8, device=x.device)
+  plan.scale_only = int(scale_only)
+  q = None if scale_only else torch.empty(qshape, dtype=torch.uint8 if fp8 else torch.int8, device=x.device)
   if prescale is not None:
     assert prescale.dtype == torch.float32 and prescale.is_contiguous()
   lib = L.lib()
@@ -480,13 +483,15 @@ def decode_weight_only(x: torch.Tensor, w_q: torch.Tensor, w_scale: torch.Tensor
 
 def decode(x: torch.Tensor, w_q: torch.Tensor, w_scale: torch.Tensor, *, quant_bound: float,
            clip_bound: float, x_scale_dtype=None, w_scale_dtype=torch.float32, want_xq: bool = False,
-           w_dtype: int = L.I8, tuning: int = 0, static_scratch: bool = False, w_layout: int = L.W_ROWS):
+           w_dtype: int = L.I8, tuning: int = 0, static_scratch: bool = False, w_layout: int = L.W_ROWS,
+           want_typed_scale: bool = False):
   """Serving contraction out = dequant(quant(x) @ w_q^T) for x [m <= 64, k], w_q int8 [n, k], or
   uint8 [n, k/2] holding packed int4 (w_dtype=I4P, the pack_i4 layout).
 
   The activations get per-token dynamic int8 quantisation; `w_scale` is float32 [n] holding
   values of `w_scale_dtype`.  Returns (out [m, n] of x.dtype, x_scale float32 [m]) and, with
-  want_xq, the quantized activations as a third element.  With static_scratch the call goes
+  want_xq, the quantized activations as a third element; with want_typed_scale x_scale carries the same scales as a
+  bf16 tensor in `x_scale.typed` (None unless the scale dtype is bf16).  With static_scratch the call goes
   through aqtx_decode_i8_static: the library's built-in device scratch instead of a workspace
   tensor (n, k <= 32768; calls on one GPU must not overlap).
   """
@@ -512,9 +517,12 @@ def decode(x: torch.Tensor, w_q: torch.Tensor, w_scale: torch.Tensor, *, quant_b
   plan.w_dtype = w_dtype
   plan.tuning = tuning  # launch-shape override for measurements; results do not depend on it
   plan.w_layout = w_layout
+  x_scale = torch.empty((m,), dtype=torch.float32, device=x.device)
+  if want_typed_scale:
+    x_scale.typed = torch.empty((m,), dtype=torch.bfloat16, device=x.device) if plan.x_scale_dtype == L.BF16 else None
+    plan.x_scale_typed = x_scale.typed.data_ptr() if x_scale.typed is not None else None
   if static_scratch:
     out = torch.empty((m, n), dtype=x.dtype, device=x.device)
-    x_scale = torch.empty((m,), dtype=torch.float32, device=x.device)
     xq = torch.empty((m, k), dtype=torch.int8, device=x.device) if want_xq else None
     with _timed('decode'):
       L.check(L.lib().aqtx_decode_i8_static(ctypes.byref(plan), _ptr(x), _ptr(w_q), _ptr(w_scale), _ptr(xq),
@@ -526,7 +534,6 @@ def decode(x: torch.Tensor, w_q: torch.Tensor, w_scale: torch.Tensor, *, quant_b
   ws = _decode_workspace(ex_bytes, ws_bytes - ex_bytes, x.device)
   plan.workspace_zeroed = 1
   out = torch.empty((m, n), dtype=x.dtype, device=x.device)
-  x_scale = torch.empty((m,), dtype=torch.float32, device=x.device)
   xq = torch.empty((m, k), dtype=torch.int8, device=x.device) if want_xq else None
   try:
     with _timed('decode'):
@@ -749,20 +756,22 @@ def fp_round(x: torch.Tensor, *, nexp: int, nmant: int, has_subnormals: bool, ke
   return out
 
 
-def prng_split(key, num: int, partitionable: bool = False):
+def prng_split(key, num: int, partitionable: bool = False, inner: int = 0):
   """jax.random.split(key, num) on raw uint32[2] key data: on the host for a numpy key (returns numpy
   [num, 2]); for a key that is a 2-word device tensor, by a kernel, into a device tensor [num, 2] (no host
-  round trip: the split can be recorded into a HIP graph and follows the key's value on every replay)."""
+  round trip: the split can be recorded into a HIP graph and follows the key's value on every replay).
+  With `inner` each of the num keys is split once more, in the same launch: [num, inner, 2]."""
+  shape = (num, inner, 2) if inner else (num, 2)
   if isinstance(key, torch.Tensor):
     _require_gpu(key)
     assert key.numel() == 2 and key.element_size() == 4 and key.is_contiguous()
-    out = torch.empty((num, 2), dtype=key.dtype, device=key.device)
-    L.check(L.lib().aqtx_prng_split(_ptr(key), num, int(partitionable), _ptr(out), _stream()))
+    out = torch.empty(shape, dtype=key.dtype, device=key.device)
+    L.check(L.lib().aqtx_prng_split2(_ptr(key), num, inner, int(partitionable), _ptr(out), _stream()))
     return out
   k = (ctypes.c_uint32 * 2)(int(key[0]), int(key[1]))
-  out = (ctypes.c_uint32 * (2 * num))()
-  L.check(L.lib().aqtx_prng_split_host(k, num, int(partitionable), out))
-  return np.frombuffer(out, dtype=np.uint32).reshape(num, 2).copy()
+  out = (ctypes.c_uint32 * math.prod(shape))()
+  L.check(L.lib().aqtx_prng_split2_host(k, num, inner, int(partitionable), out))
+  return np.frombuffer(out, dtype=np.uint32).reshape(shape).copy()
 
 
 def _host_key(key, who: str):

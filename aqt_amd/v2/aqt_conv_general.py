@@ -22,6 +22,7 @@ from aqt_amd import _lib as L
 from aqt_amd import ops
 from aqt_amd.v2 import aqt_dot_general
 from aqt_amd.v2 import aqt_tensor
+from aqt_amd.v2 import lowering
 
 ConvDimensionNumbers = collections.namedtuple('ConvDimensionNumbers', ['lhs_spec', 'rhs_spec', 'out_spec'])
 
@@ -153,9 +154,9 @@ def _fused_int8_conv(lhs_qt, rhs_qt, out_dtype, window_strides, padding, lhs_dil
     positions = math.prod(out_sizes)
     if positions > 0:
       b = _conv_weight_matrix(rq, k, cout)
-      row_scale = ls.reshape(n, 1).float().expand(n, positions).reshape(n * positions).contiguous()
+      row_scale = lowering.scale_f32(ls).reshape(n, 1).expand(n, positions).reshape(n * positions).contiguous()
       out, out_sizes = ops.conv_i8(lq, b, kernel, strides, pads, dilation, row_scale=row_scale,
-                                   col_scale=rs.reshape(cout).float().contiguous(), out_dtype=out_dtype,
+                                   col_scale=lowering.scale_f32(rs).reshape(cout).contiguous(), out_dtype=out_dtype,
                                    row_scale_dtype=ls.dtype, col_scale_dtype=rs.dtype)
       return out.reshape([n] + list(out_sizes) + [cout])
   a, out_sizes = ops.im2col_i8(lq, kernel, strides, pads, dilation)
@@ -164,8 +165,8 @@ def _fused_int8_conv(lhs_qt, rhs_qt, out_dtype, window_strides, padding, lhs_dil
   if a.shape[0] * cout == 0 or k == 0:
     return None
   b = _conv_weight_matrix(rq, k, cout)
-  row_scale = ls.reshape(n, 1).float().expand(n, positions).reshape(1, n * positions).contiguous()
-  out = ops.gemm(a.contiguous()[None], b[None], row_scale=row_scale, col_scale=rs.reshape(1, cout).float().contiguous(),
+  row_scale = lowering.scale_f32(ls).reshape(n, 1).expand(n, positions).reshape(1, n * positions).contiguous()
+  out = ops.gemm(a.contiguous()[None], b[None], row_scale=row_scale, col_scale=lowering.scale_f32(rs).reshape(1, cout).contiguous(),
                  out_dtype=out_dtype, dequant_dtype=out_dtype, row_scale_dtype=ls.dtype, col_scale_dtype=rs.dtype,
                  a_dtype=L.I8, b_dtype=L.I8)[0]
   return out.reshape([n] + list(out_sizes) + [cout])

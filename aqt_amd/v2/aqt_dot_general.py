@@ -1208,9 +1208,10 @@ class DotGeneralRaw:
                              quant_bound=spec['quant_bound'], clip_bound=spec['clip_bound'],
                              x_scale_dtype=sdt, w_scale_dtype=w_scale.dtype, want_xq=True,
                              w_dtype=L.I4P if packed else L.I4 if rhs_qt.container_dtype is utils.int4 else L.I8,
-                             w_layout=L.W_FRAGMENTS)
+                             w_layout=L.W_FRAGMENTS, want_typed_scale=True)
     out = out.reshape([lhs.shape[a] for a in lra] + [rhs_arr.shape[a] for a in rra])
     qv = lowering.logical_from_brk(xq[None], lv)
+    xs = xs.typed if xs.typed is not None else xs
     sc = lowering.logical_from_brk(xs.reshape(1, M), lv, k_keep=False).to(sdt)
     lhs_qt_out = aqt_tensor.QTensor(qvalue=qv, scale=[sc], scale_t=None, bias=[], dequant_dtype=lhs_dtype)
     lhs_grad = functools.partial(dq.lhs.numerics.vjp_bwd, (None,))
@@ -1550,9 +1551,10 @@ class DotGeneral:
     # (aqtx_quantize writes that order for groups of up to _EVEN_ODD8_MAX_GROUP values; longer tiles stay in k order)
     k_order = (L.K_EVEN_ODD8 if packed and ts <= _EVEN_ODD8_MAX_GROUP and not (with_qt and lhs_qvalue_needed)
                else L.K_NATURAL)
-    lq, lsc = ops.quantize(lhs.reshape(1, M, T * ts), reduce=L.REDUCE_COLS, group=ts, out_dtype=specs[0]['out_dtype'],
-                           quant_bound=specs[0]['quant_bound'], clip_bound=specs[0]['clip_bound'],
-                           compute_dtype=lhs.dtype, scale_dtype=sdt_l, k_order=k_order)
+    lq, lsc, ltyped = ops.quantize(lhs.reshape(1, M, T * ts), reduce=L.REDUCE_COLS, group=ts, want_typed_scale=True,
+                                   out_dtype=specs[0]['out_dtype'],
+                                   quant_bound=specs[0]['quant_bound'], clip_bound=specs[0]['clip_bound'],
+                                   compute_dtype=lhs.dtype, scale_dtype=sdt_l, k_order=k_order)
     if frozen:
       rv = lowering.view_operand(rhs_qt.qvalue, [], rra, [0, 1])
       rq = _kernel_layout_of(rhs_qt.qvalue, rv, pack_int4=packed)     # [1, N, T*ts] (or packed)
@@ -1574,7 +1576,8 @@ class DotGeneral:
       return out
     mk_container = lambda spec: utils.int4 if spec['out_dtype'] == L.I4 else None
     lhs_qt_out = aqt_tensor.QTensor(
-        qvalue=lq.reshape(lhs.shape) if k_order == L.K_NATURAL else None, scale=[lsc.reshape(tuple(lhs.shape[:-1]) + (1,)).to(sdt_l)], scale_t=None,
+        qvalue=lq.reshape(lhs.shape) if k_order == L.K_NATURAL else None, 
+        scale=[(lsc if ltyped is None else ltyped).reshape(tuple(lhs.shape[:-1]) + (1,)).to(sdt_l)], scale_t=None,
         bias=[], dequant_dtype=lhs.dtype, container_dtype=mk_container(specs[0]))
     if frozen:
       rhs_qt_out = rhs_qt

@@ -146,7 +146,7 @@ _OUT_TORCH = {L.I8: torch.int8, L.I4: torch.int8, L.E4M3: torch.float8_e4m3fn, L
 def quantize_view(v: OperandView, *, spec: dict, compute_dtype, scale_dtype, key=None,
                   per_tensor: bool = False, prescale: Optional[torch.Tensor] = None,
                   scale: Optional[torch.Tensor] = None, want_other_axis_absmax: bool = False,
-                  absmax_partials: Optional[torch.Tensor] = None):
+                  absmax_partials: Optional[torch.Tensor] = None, scale_only: bool = False):
   """Runs the quantize kernel on a view.
 
   Returns (q [B, R, K] int8/uint8, scale float32 [B, R] (or [1] per tensor)).
@@ -175,7 +175,7 @@ def quantize_view(v: OperandView, *, spec: dict, compute_dtype, scale_dtype, key
     raise AssertionError('unreachable')
   q, s, typed = ops.quantize(v.mem, reduce=reduce, transpose_out=transpose, scale=scale,
                              want_typed_scale=True, want_other_axis_absmax=want_other_axis_absmax,
-                             absmax_partials=absmax_partials, **kwargs)
+                             absmax_partials=absmax_partials, scale_only=scale_only, **kwargs)
   shape = (-1,) if per_tensor else (v.B, v.R)
   s = s.reshape(shape)
   # the same scales as elements of the scale dtype, written by the kernel (saves a cast launch)
@@ -191,7 +191,7 @@ def absmax_scale(x: torch.Tensor, shared_axes: Sequence[int], numerics_, scale_d
   spec = dict(out_dtype=L.I8, quant_bound=float(numerics_.get_quant_bound()), clip_bound=1.0,
               noise=L.NOISE_NONE)
   sdt = scale_dtype if scale_dtype is not None else x.dtype
-  _, s = quantize_view(v, spec=spec, compute_dtype=x.dtype, scale_dtype=sdt)
+  _, s = quantize_view(v, spec=spec, compute_dtype=x.dtype, scale_dtype=sdt, scale_only=True)
   return scale_in_dtype(s, v, sdt)
 
 
@@ -209,3 +209,11 @@ def scale_in_dtype(s32: torch.Tensor, v: OperandView, sdt) -> torch.Tensor:
   if sdt != torch.float32:
     out.f32_copy = f32  # same values, for kernels that take float32 scale vectors
   return out
+
+
+def scale_f32(scale: torch.Tensor) -> torch.Tensor:
+  """`scale` in float32: the copy the quantize kernels left beside it (scale_in_dtype), unless it was written to since."""
+  src = getattr(scale, 'f32_copy', None)
+  if src is not None and src.shape == scale.shape and not scale.is_inference() and scale._version == 0:
+    return src
+  return scale.float()

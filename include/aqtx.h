@@ -116,6 +116,8 @@ typedef struct aqtx_quant_plan {
   void* other_axis_absmax;
   const void* absmax_partials;
   int64_t absmax_parts;
+  int32_t scale_only;       /* 1: calibration alone: the scales are written, q is not (it may be NULL); noise NONE and no
+                               given scale */
 } aqtx_quant_plan;
 
 /*
@@ -490,6 +492,8 @@ typedef struct aqtx_decode_plan {
                              the scratch lives in the LAST bytes of the workspace: one shared by plans
                              of different shapes must hold the largest exchange size plus the largest
                              (workspace_bytes - exchange_bytes) of those plans.                      */
+  void* x_scale_typed;    /* optional out [m]: the activation scales once more as bf16 elements (aqtx_decode_i8 with
+                             x_scale_dtype AQTX_BF16 only; ignored otherwise)                        */
 } aqtx_decode_plan;
 
 /*
@@ -578,12 +582,22 @@ int aqtx_prng_split_host(const uint32_t key_host[2], int32_t num, int32_t partit
                          uint32_t* out_host);
 
 /*
+ * aqtx_prng_split2_host: the same, and split(., inner) of each of the num keys: out_host uint32[num][inner][2]
+ * (inner = 0: aqtx_prng_split_host).
+ */
+int aqtx_prng_split2_host(const uint32_t key_host[2], int32_t num, int32_t inner, int32_t partitionable,
+                          uint32_t* out_host);
+
+/*
  * aqtx_prng_split: the same split of a key held in DEVICE memory, by a kernel: key_device uint32[2],
  * out_device uint32[num][2].  For keys that are traced arrays under XLA or change between replays of a
  * HIP graph (aqtx_quant_plan.key_device reads the results).
  */
 int aqtx_prng_split(const uint32_t* key_device, int32_t num, int32_t partitionable, uint32_t* out_device,
                     void* stream);
+/* The two levels of aqtx_prng_split2_host in one launch: out_device uint32[num][inner][2]. */
+int aqtx_prng_split2(const uint32_t* key_device, int32_t num, int32_t inner, int32_t partitionable,
+                     uint32_t* out_device, void* stream);
 
 /*
  * aqtx_random_bits: jax.random.bits(key, [n], uint{bit_width}) on the device,

@@ -453,3 +453,16 @@ def test_weight_only_serving_many_tokens_narrow_weight(gpu):
     out, _ = cfg.dg_core(x, torch.zeros_like(w), None, wq, MATMUL)
   want = (x.float() @ (wq.qvalue.float() * wq.scale[0].float())).cpu().numpy()
   np.testing.assert_allclose(out.float().cpu().numpy(), want, rtol=2.0 ** -6, atol=2.0 ** -6 * np.abs(want).max())
+
+
+@pytest.mark.parametrize('m,n,k,tuning', [(1, 64, 4096, 0), (2, 64, 8192, 0), (8, 256, 14336, 0), (33, 128, 1024, 0), (8, 256, 1024, 2 << 16)])
+def test_activation_scales_as_bf16_elements(gpu, m, n, k, tuning):
+  """The second copy of the scales, from each of the kernels that quantize activations."""
+  g = torch.Generator(device=gpu).manual_seed(m)
+  x = torch.randn(m, k, generator=g, device=gpu).to(torch.bfloat16)
+  w = torch.randint(-127, 128, (n, k), generator=g, device=gpu, dtype=torch.int8)
+  ws = torch.rand(n, generator=g, device=gpu)
+  _, xs = ops.decode(x, w, ws, quant_bound=127.5, clip_bound=127.0, tuning=tuning, want_typed_scale=True)
+  assert xs.typed.dtype == torch.bfloat16 and torch.equal(xs.typed.float(), xs)
+  _, xs = ops.decode(x, w, ws, quant_bound=127.5, clip_bound=127.0, x_scale_dtype=torch.float32, want_typed_scale=True)
+  assert xs.typed is None

@@ -416,3 +416,26 @@ def test_scales_from_the_last_block_equal_those_of_their_own_launch(gpu, reduce,
   want = {L.REDUCE_ROWS: lambda: want.reshape(shape[0], -1, group or shape[1], shape[2]).amax(2), L.REDUCE_ALL: lambda: want.amax((1, 2)),
           L.REDUCE_ALL_BATCH: lambda: want.amax().reshape(1)}[reduce]()
   assert torch.equal(results[0][1], (want / 127.5).to(torch.bfloat16).float())
+
+
+@pytest.mark.parametrize('reduce,shape', [(L.REDUCE_COLS, (1, 5, 3000)), (L.REDUCE_COLS, (1, 3, 5)), (L.REDUCE_COLS, (2, 2, 20000)),
+                                          (L.REDUCE_ROWS, (1, 300, 72)), (L.REDUCE_ALL, (2, 100, 64))])
+def test_calibration_alone_gives_the_scales_of_the_quantization(gpu, reduce, shape):
+  x = U.to_dev(U.rand(shape, 'bf16', seed=9, outliers=True), 'bf16', gpu)
+  kw = dict(reduce=reduce, out_dtype=L.I8, quant_bound=127.5, clip_bound=127.0, want_typed_scale=True)
+  _, s, t = ops.quantize(x, **kw)
+  q, s1, t1 = ops.quantize(x, scale_only=True, **kw)
+  assert q is None and torch.equal(s, s1) and torch.equal(t, t1)
+  with pytest.raises(L.AqtxError, match='scale_only'):
+    ops.quantize(x, reduce=reduce, out_dtype=L.I8, quant_bound=127.5, clip_bound=127.0, scale_only=True, scale=s)
+
+
+@pytest.mark.parametrize('partitionable', [False, True])
+@pytest.mark.parametrize('num,inner', [(1, 1), (3, 2), (2, 5)])
+def test_two_levels_of_key_splits_in_one_call(gpu, num, inner, partitionable):
+  key = prng.prng_key(77)
+  want = np.stack([prng.split(k, inner, partitionable) for k in prng.split(key, num, partitionable)])
+  np.testing.assert_array_equal(ops.prng_split(key, num, partitionable, inner=inner), want)
+  dev = torch.from_numpy(key.view(np.int32).copy()).to(gpu)
+  got = ops.prng_split(dev, num, partitionable, inner=inner).cpu().numpy().view(np.uint32)
+  np.testing.assert_array_equal(got, want)
