@@ -11,6 +11,7 @@ canonical one (a plain permute copy, no arithmetic).
 from __future__ import annotations
 
 import dataclasses
+import functools
 import math
 from typing import Any, List, Optional, Sequence, Tuple
 
@@ -53,16 +54,20 @@ class OperandView:
     return _prod(self.shape[a] for a in self.k_axes)
 
 
-def memory_rank(x: torch.Tensor):
-  """Axes of extent > 1 in memory order (outermost first), and whether x is dense."""
-  big = [a for a in range(x.dim()) if x.shape[a] > 1]
-  order = sorted(big, key=lambda a: (-x.stride(a), a))
+def _memory_rank(shape, strides):
+  big = [a for a in range(len(shape)) if shape[a] > 1]
+  order = sorted(big, key=lambda a: (-strides[a], a))
   expect, dense = 1, True
   for a in reversed(order):
-    if x.stride(a) != expect:
+    if strides[a] != expect:
       dense = False
-    expect *= x.shape[a]
+    expect *= shape[a]
   return order, dense
+
+
+def memory_rank(x: torch.Tensor):
+  """Axes of extent > 1 in memory order (outermost first), and whether x is dense."""
+  return _memory_rank(tuple(x.shape), x.stride())
 
 
 def _merged_stride(shape, axes):
@@ -81,11 +86,12 @@ def _merged_stride(shape, axes):
   return ls[big[-1]] if big else 0
 
 
-def view_operand(x: torch.Tensor, ba: Sequence[int], ra: Sequence[int], ca: Sequence[int]) -> OperandView:
-  """3-D view of x with the groups flattened in the listed axis orders."""
-  ba, ra, ca = list(ba), list(ra), list(ca)
-  shape = tuple(x.shape)
-  order, dense = memory_rank(x)
+# A layer sees the same few layouts on every call, and finding one's view costs ten times its permute and reshape.
+@functools.lru_cache(maxsize=4096)
+def _view_plan(shape, strides, ba, ra, ca):
+  """What view_operand does to an operand of this shape and these strides (values alone decide):
+  (permutation, 3-D shape, k_last, noise strides, whether the permutation has to be copied)."""
+  order, dense = _memory_rank(shape, strides)
   group_of = {}
   for a in ba:
     group_of[a] = 'b'
@@ -103,26 +109,25 @@ def view_operand(x: torch.Tensor, ba: Sequence[int], ra: Sequence[int], ca: Sequ
     it = iter(full)
     return all(any(c == f for f in it) for c in p)
 
-  copied = False
-  if dense and within_ok and len(set(pattern)) == len(pattern) and is_subseq(pattern, ['b', 'r', 'k']):
-    k_last = True
-  elif dense and within_ok and len(set(pattern)) == len(pattern) and is_subseq(pattern, ['b', 'k', 'r']):
-    k_last = False
-  else:
-    x = x.permute(tuple(ba + ra + ca)).contiguous()
-    # after the copy the logical axes are renumbered; keep the caller's numbering for shapes only
-    b_n, r_n = len(ba), len(ra)
-    mem = x.reshape(_prod(x.shape[:b_n]), _prod(x.shape[b_n:b_n + r_n]), _prod(x.shape[b_n + r_n:]))
-    copied, k_last = True, True
-    ns = tuple(_merged_stride(shape, g) for g in (ba, ra, ca))
-    return OperandView(mem, k_last, ba, ra, ca, shape, None if None in ns else ns, copied)
-  perm = ba + (ra + ca if k_last else ca + ra)
-  xp = x.permute(tuple(perm))
+  plain = dense and within_ok and len(set(pattern)) == len(pattern)
+  k_last = not (plain and not is_subseq(pattern, ['b', 'r', 'k']) and is_subseq(pattern, ['b', 'k', 'r']))
+  copied = k_last and not (plain and is_subseq(pattern, ['b', 'r', 'k']))
   B, R, K = (_prod(shape[a] for a in g) for g in (ba, ra, ca))
-  mem = xp.reshape(B, R, K) if k_last else xp.reshape(B, K, R)
-  assert mem.is_contiguous()
   ns = tuple(_merged_stride(shape, g) for g in (ba, ra, ca))
-  return OperandView(mem, k_last, ba, ra, ca, shape, None if None in ns else ns, copied)
+  return (ba + (ra + ca if k_last else ca + ra), (B, R, K) if k_last else (B, K, R), k_last,
+          None if None in ns else ns, copied)
+
+
+def view_operand(x: torch.Tensor, ba: Sequence[int], ra: Sequence[int], ca: Sequence[int]) -> OperandView:
+  """3-D view of x with the groups flattened in the listed axis orders."""
+  shape = tuple(x.shape)
+  perm, dims, k_last, ns, copied = _view_plan(shape, x.stride(), tuple(ba), tuple(ra), tuple(ca))
+  mem = x.permute(perm)
+  if copied:
+    mem = mem.contiguous()
+  mem = mem.reshape(dims)
+  assert mem.is_contiguous()
+  return OperandView(mem, k_last, list(ba), list(ra), list(ca), shape, ns, copied)
 
 
 def logical_from_brk(t: torch.Tensor, v: OperandView, k_keep: bool = True) -> torch.Tensor:

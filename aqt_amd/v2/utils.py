@@ -9,6 +9,7 @@ from __future__ import annotations
 import copy
 import dataclasses
 import enum
+import functools
 from typing import Any, Callable, Optional, Sequence, Union
 
 import numpy as np
@@ -122,11 +123,17 @@ def clone_fields(obj):
   """A new object of obj's class holding the same field values (what copy.copy gives for a plain
   dataclass instance, without the pickle protocol round trip that makes it ~20x slower)."""
   fields = getattr(obj, '__dict__', None)
-  if fields is None or hasattr(type(obj), '__slots__'):
+  if fields is None or _has_slots(type(obj)):
     return copy.copy(obj)
   out = object.__new__(type(obj))
   out.__dict__.update(fields)
   return out
+
+
+@functools.lru_cache(maxsize=1024)
+def _has_slots(cls) -> bool:
+  """Whether instances of `cls` hold fields outside their __dict__ (the empty __slots__ of abc.ABC are none)."""
+  return any(c.__dict__.get('__slots__') for c in cls.__mro__)
 
 
 def deepcopy_fields(obj, memo, shared=()):

@@ -339,3 +339,29 @@ def test_set_context_without_copying_the_settings():
                                    for f in dataclasses.fields(other.fwd.dg_quantizer)})
   got = config.set_context(other, None, train_step=None, copy_settings=False)
   assert got.fwd.lhs is not other.fwd.lhs and got.fwd.dg_quantizer.lhs.numerics is not other.fwd.dg_quantizer.lhs.numerics
+
+
+@pytest.mark.parametrize('rank', [1, 2, 3, 4])
+def test_operand_views_over_memory_orders_and_axis_groups(rank):
+  """lowering.view_operand over every memory order of small tensors and every split of their axes into batch, remaining
+  and contraction axes: the 3-D view holds the values of the plain permutation, shares memory unless it says it copied,
+  and never depends on an earlier call with another layout."""
+  import itertools
+  shape = (2, 3, 1, 4)[:rank]
+  base = torch.arange(2 * int(np.prod(shape)))
+  for order in itertools.permutations(range(rank)):
+    dense = base[:base.numel() // 2].reshape([shape[a] for a in order]).permute([order.index(a) for a in range(rank)])
+    gaps = base.reshape([shape[a] for a in order] + [2])[..., 0].permute([order.index(a) for a in range(rank)])
+    for x in (dense, gaps):
+      for groups in itertools.product('brk', repeat=rank):
+        ba, ra, ca = ([a for a in range(rank) if groups[a] == g] for g in 'brk')
+        v = lowering.view_operand(x, ba, ra, ca)
+        want = x.permute(ba + ra + ca).reshape(v.B, v.R, v.K)
+        got = v.mem if v.k_last else v.mem.transpose(1, 2)
+        assert v.mem.is_contiguous() and torch.equal(got, want) and v.shape == tuple(x.shape)
+        assert v.copied == (v.mem.data_ptr() != x.data_ptr())
+        index = torch.arange(x.numel()).reshape(x.shape).permute(ba + ra + ca).reshape(v.B, v.R, v.K)
+        if v.noise_strides is not None:
+          i, j, k = torch.meshgrid(*(torch.arange(n) for n in (v.B, v.R, v.K)), indexing='ij')
+          sb, sr, sk = v.noise_strides
+          assert torch.equal(index, i * sb + j * sr + k * sk)
