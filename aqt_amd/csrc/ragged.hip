@@ -1,0 +1,61 @@
+// Row offsets of a ragged contraction's groups from their sizes, and zeros in the output rows behind the last group.
+// Bound by its launch: one takes the place of five of a few us each (zeros, cumulative sum, copies, clamp), and of a
+// fill of the whole output, 30 us for 8192 x 14336 bf16 values, of which the contraction overwrites the rows of all groups.
+#include "common.h"
+
+namespace aqtx {
+namespace {
+
+__global__ __launch_bounds__(256) void ragged_prepare_kernel(const int32_t* __restrict__ sizes, int64_t groups, int64_t m,
+                                                             int32_t* __restrict__ offsets, uint16_t* __restrict__ c, int64_t row_halves) {
+  __shared__ int64_t covered;
+  if (threadIdx.x < 64) {  // one wave: inclusive sums of 64 sizes at a time; every block finds the covered rows itself
+    const int lane = (int)threadIdx.x;
+    int64_t before = 0, most = 0;
+    if (blockIdx.x == 0 && lane == 0) offsets[0] = 0;
+    for (int64_t g0 = 0; g0 < groups; g0 += 64) {
+      int64_t s = g0 + lane < groups ? (int64_t)sizes[g0 + lane] : 0;
+#pragma unroll
+      for (int off = 1; off < 64; off <<= 1) {
+        const int64_t up = __shfl_up(s, off, 64);
+        if (lane >= off) s += up;
+      }
+      int64_t end = (int64_t)(int32_t)(before + s);
+      if (end > m) end = m;
+      if (blockIdx.x == 0 && g0 + lane < groups) offsets[g0 + lane + 1] = (int32_t)end;
+      if (end > most) most = end;
+      before += __shfl(s, 63, 64);
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+      const int64_t other = __shfl_xor(most, off, 64);
+      most = other > most ? other : most;
+    }
+    if (lane == 0) covered = most;
+  }
+  __syncthreads();
+  const int64_t first = covered * row_halves, total = m * row_halves, stride = (int64_t)gridDim.x * 256;
+  for (int64_t i = first + (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += stride) c[i] = 0;
+}
+
+}  // namespace
+}  // namespace aqtx
+
+using namespace aqtx;
+
+extern "C" int aqtx_ragged_prepare(const int32_t* sizes, int64_t groups, int64_t m, int32_t* offsets, void* c,
+                                   int64_t row_bytes, void* stream) {
+  clear_error();
+  AQTX_REQUIRE(groups >= 0 && m >= 0 && m < (1ll << 31) && row_bytes >= 0 && row_bytes % 2 == 0,
+               "aqtx_ragged_prepare: negative or too large shape, or odd row bytes");
+  AQTX_REQUIRE(offsets != nullptr && (sizes != nullptr || groups == 0) && (c != nullptr || m * row_bytes == 0),
+               "aqtx_ragged_prepare: NULL buffer");
+  AQTX_REQUIRE(((uintptr_t)sizes % 4) == 0 && ((uintptr_t)offsets % 4) == 0 && ((uintptr_t)c % 2) == 0,
+               "aqtx_ragged_prepare: buffers are not element aligned");
+  int64_t blocks = (m * (row_bytes / 2) + 256 * 64 - 1) / (256 * 64);
+  blocks = blocks < 1 ? 1 : blocks > 1024 ? 1024 : blocks;
+  ragged_prepare_kernel<<<dim3((unsigned)blocks), 256, 0, reinterpret_cast<hipStream_t>(stream)>>>(
+      sizes, groups, m, offsets, reinterpret_cast<uint16_t*>(c), row_bytes / 2);
+  AQTX_HIP_CHECK_LAUNCH("ragged_prepare_kernel");
+  return 0;
+}

@@ -315,6 +315,7 @@ def gemm(
     b_dtype: int = L.I8,
     want_acc: bool = False,
     group_offsets: Optional[torch.Tensor] = None,
+    group_sizes: Optional[torch.Tensor] = None,
     a_k_order: int = 0,
     k_split: int = 0,
     b_layout: int = L.W_ROWS,
@@ -337,7 +338,8 @@ def gemm(
   With `group_offsets` (int32 device tensor [groups + 1], ascending): a ragged product.  A is
   [1, m, k], B [groups, n, k]; group g multiplies rows off[g]:off[g+1] of A with B[g] into the
   same rows of C [1, m, n], in one launch; rows outside every group are left as allocated
-  (zero-initialised here).
+  (zero-initialised here).  `group_sizes` (ragged_sizes) in its place: the offsets, and the zeros behind the last group,
+  are made here, in one launch.  col_scale may then be one row [1, n] for all groups.
 
   int8 operands use the int32 MFMA path, fp8 operands (uint8 tensors holding
   e4m3fn/e5m2 bytes) the float32 one.  `scale_dtype` names the dtype of both scale
@@ -347,16 +349,20 @@ def gemm(
   _require_gpu(a, b, row_scale, col_scale)
   batch, m, k = a.shape
   if b_layout == L.W_FRAGMENTS:
-    assert batch == 1 and group_offsets is None and col_scale is not None and b.is_contiguous() and a.stride(2) == 1
+    assert (batch == 1 and group_offsets is None and group_sizes is None and col_scale is not None and b.is_contiguous()
+            and a.stride(2) == 1)
     n = col_scale.shape[-1]
     assert b.numel() * b.element_size() == L.lib().aqtx_tile_weight_bytes(n, k, b_dtype), (b.shape, n, k)
     b_batches, ldb, stride_b = 1, 0, 0
   else:
     assert a.dim() == 3 and b.dim() == 3 and a.shape[2] == (2 * b.shape[2] if b_dtype == L.I4P else b.shape[2])
-    assert a.shape[0] == b.shape[0] or group_offsets is not None
+    assert a.shape[0] == b.shape[0] or group_offsets is not None or group_sizes is not None
     assert a.stride(2) == 1 and b.stride(2) == 1, 'the contraction axis must be contiguous'
     n = b.shape[1]
     b_batches, ldb, stride_b = b.shape[0], b.stride(1), b.stride(0)
+  if group_sizes is not None:
+    assert group_offsets is None and group_sizes.dtype == torch.int32 and group_sizes.is_cuda and group_sizes.is_contiguous()
+    group_offsets = torch.empty(group_sizes.numel() + 1, dtype=torch.int32, device=a.device)
   if group_offsets is not None:
     assert a.shape[0] == 1 and group_offsets.dtype == torch.int32 and group_offsets.is_cuda
     assert group_offsets.numel() == b.shape[0] + 1 and group_offsets.is_contiguous()
@@ -369,8 +375,11 @@ def gemm(
   out_dt = aqtx_dtype(out_dtype)
   dq_dt = aqtx_dtype(dequant_dtype) if dequant_dtype is not None else (out_dt if out_dt != L.I32 else L.F32)
   sc_dt = aqtx_dtype(scale_dtype) if scale_dtype is not None else dq_dt
-  alloc = torch.zeros if group_offsets is not None else torch.empty
+  alloc = torch.zeros if group_offsets is not None and group_sizes is None else torch.empty
   c = alloc((batch, m, n), dtype=_AQTX_TO_TORCH[out_dt], device=a.device)
+  if group_sizes is not None:
+    L.check(L.lib().aqtx_ragged_prepare(_ptr(group_sizes), group_sizes.numel(), m, _ptr(group_offsets), _ptr(c),
+                                        n * c.element_size(), _stream()))
   acc = None
   if want_acc:
     acc = torch.empty((batch, m, n), dtype=torch.float32 if fp8 else torch.int32, device=a.device)
@@ -389,10 +398,11 @@ def gemm(
   plan.a_k_order = a_k_order
   plan.k_split = 1 if fp8 else k_split
   plan.accumulate = (FP8_ACCUMULATE if accumulate is None else accumulate) if fp8 else L.ACC_FAST
-  for s, shape in ((row_scale, (batch, m)), (col_scale, (b_batches, n))):
+  shared_cols = group_sizes is not None and col_scale is not None and col_scale.shape[0] == 1
+  for s, shape in ((row_scale, (batch, m)), (col_scale, (1 if shared_cols else b_batches, n))):
     if s is not None:
       assert s.dtype == torch.float32 and s.is_contiguous() and tuple(s.shape) == shape, (tuple(s.shape), shape)
-  plan.row_scale_stride_b, plan.col_scale_stride_b = m, n
+  plan.row_scale_stride_b, plan.col_scale_stride_b = m, 0 if shared_cols else n
   fn = L.lib().aqtx_gemm_fp8 if fp8 else L.lib().aqtx_gemm_i8
   slabs = None
   if not fp8:
@@ -406,14 +416,10 @@ def gemm(
   return (c, acc) if want_acc else c
 
 
-def ragged_offsets(group_sizes, m: int, device) -> torch.Tensor:
-  """[0, s0, s0+s1, ...] as int32 on the device, clamped to the m rows there are; computed on the
-  device when the sizes live there (no host round trip)."""
+def ragged_sizes(group_sizes, device) -> torch.Tensor:
+  """Group sizes as gemm(group_sizes=...) takes them: int32 on the device (no host round trip where they live there)."""
   sizes = group_sizes if isinstance(group_sizes, torch.Tensor) else torch.tensor(list(group_sizes), dtype=torch.int32)
-  sizes = sizes.to(device=device, dtype=torch.int32)
-  offs = torch.zeros(sizes.numel() + 1, dtype=torch.int32, device=device)
-  offs[1:] = torch.cumsum(sizes, 0)
-  return torch.clamp(offs, max=m)
+  return sizes.to(device=device, dtype=torch.int32).contiguous()
 
 
 def gemm_weight_only(a: torch.Tensor, b: torch.Tensor, col_scale: torch.Tensor, *, col_scale_dtype=torch.float32,

@@ -887,9 +887,9 @@ class DotGeneralRaw:
       if not (K % 16 == 0 and lq.data_ptr() % 16 == 0 and rq3.data_ptr() % 16 == 0 and M * N > 0):
         raise _NotFused('ragged contraction with unaligned operands')
       out = ops.gemm(lq, rq3, row_scale=ls.reshape(1, M) if ls.numel() == M else ls.reshape(1, 1).expand(1, M).contiguous(),
-                     col_scale=rs.reshape(1, -1).expand(G, N).contiguous(), a_dtype=lkd, b_dtype=rkd,
+                     col_scale=rs.reshape(1, -1).expand(1, N).contiguous(), a_dtype=lkd, b_dtype=rkd,
                      row_scale_dtype=lsdt, col_scale_dtype=rsdt, out_dtype=dequant_dtype, dequant_dtype=dequant_dtype,
-                     group_offsets=ops.ragged_offsets(ragged, M, lq.device))
+                     group_sizes=ops.ragged_sizes(ragged, lq.device))
       res = DotGeneralRes(lhs=TensorRes(mt=MultiTensor(x=lhs, qx=lhs_qt_out), quant_grad=lhs_grad),
                           rhs=TensorRes(mt=MultiTensor(x=rhs_arr, qx=rhs_qt_out), quant_grad=rhs_grad))
       return out.reshape(M, N), res

@@ -49,7 +49,7 @@ def lax_ragged_dot(lhs, rhs, group_sizes, precision=None, preferred_element_type
                and a.data_ptr() % 16 == 0 and bt.data_ptr() % 16 == 0)
     if aligned:
       return ops.gemm(a[None], bt, row_scale=None, col_scale=None, out_dtype=torch.int32, a_dtype=L.I8,
-                      b_dtype=L.I8, group_offsets=ops.ragged_offsets(group_sizes, m, lhs.device))[0]
+                      b_dtype=L.I8, group_sizes=ops.ragged_sizes(group_sizes, lhs.device))[0]
   # one contraction per group on row slices (sizes read on the host: a synchronisation when they
   # live on the device)
   sizes = _host_group_sizes(group_sizes)

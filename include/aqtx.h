@@ -296,6 +296,15 @@ int aqtx_gemm_i8(const aqtx_gemm_plan* plan, const void* a, const void* b,
 int aqtx_gemm_i8_k_slices(const aqtx_gemm_plan* plan);
 
 /*
+ * aqtx_ragged_prepare: what a ragged contraction (aqtx_gemm_plan.group_offsets) needs beside its operands:
+ * offsets[0 .. groups] = 0 and the running sums of sizes[0 .. groups - 1], none above m; and zeros in the rows of c
+ * ([m][row_bytes]) behind the last of them, which no group writes.  All pointers on the device: sizes may be computed
+ * there.
+ */
+int aqtx_ragged_prepare(const int32_t* sizes, int64_t groups, int64_t m, int32_t* offsets, void* c, int64_t row_bytes,
+                        void* stream);
+
+/*
  * aqtx_pad_rows: byte rows [batch][rows][k] of one or two contraction operands (b_out NULL: of `a` alone), rows `ld`
  * and batch entries `stride` bytes apart and aligned in any way, copied to [batch][rows][16 * ceil(k / 16)] with zeros
  * behind k: operands of aqtx_gemm_i8 / aqtx_gemm_fp8 whose k, leading dimensions or addresses are no multiples of

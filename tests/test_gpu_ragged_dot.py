@@ -105,3 +105,31 @@ def test_ragged_gemm_one_launch_against_integer_reference(gpu):
   for g, (lo, hi) in enumerate(zip(offs[:-1], offs[1:])):
     want[lo:hi] = a[lo:hi].astype(np.int64) @ b[g].astype(np.int64).T
   np.testing.assert_array_equal(out, want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('groups', [1, 3, 64, 65, 200])
+@pytest.mark.parametrize('left', [0, 1, 300, 4000])
+def test_ragged_gemm_prepares_offsets_and_zeros_from_the_sizes(gpu, groups, left):
+  """Sizes with empty groups, `left` rows behind the last group (negative room: sizes that overrun the rows are cut at
+  m), int32 and bf16 outputs, one row of column scales for all groups: as the offsets made on the host give it."""
+  from aqt_amd import ops
+  rng = np.random.default_rng(groups + left)
+  sizes = rng.integers(0, 40, groups) * rng.integers(0, 2, groups)
+  sizes[-1] += 1
+  total = int(sizes.sum())
+  k, n = 64, 33
+  for m in (total + left, max(1, total - 5)):
+    a = torch.from_numpy(rng.integers(-127, 128, (1, m, k)).astype(np.int8)).to(gpu)
+    b = torch.from_numpy(rng.integers(-127, 128, (groups, n, k)).astype(np.int8)).to(gpu)
+    offs = torch.from_numpy(np.minimum(np.concatenate([[0], np.cumsum(sizes)]), m).astype(np.int32)).to(gpu)
+    ones, cs = torch.ones((1, m), device=gpu), torch.rand((1, n), device=gpu)
+    dev_sizes = ops.ragged_sizes(torch.from_numpy(sizes), gpu)
+    junk = torch.full((2 * m * n * 4,), 0x7F, dtype=torch.uint8, device=gpu)  # what a freed block would leave behind
+    del junk
+    got = ops.gemm(a, b, row_scale=None, col_scale=None, out_dtype=torch.int32, group_sizes=dev_sizes)
+    want = ops.gemm(a, b, row_scale=None, col_scale=None, out_dtype=torch.int32, group_offsets=offs)
+    assert torch.equal(got, want) and not bool(got[0, min(total, m):].any())
+    got = ops.gemm(a, b, row_scale=ones, col_scale=cs, out_dtype=torch.bfloat16, group_sizes=dev_sizes)
+    want = ops.gemm(a, b, row_scale=ones, col_scale=cs.expand(groups, n).contiguous(), out_dtype=torch.bfloat16, group_offsets=offs)
+    assert torch.equal(got, want)
