@@ -154,6 +154,7 @@ struct GemmArgs {
   // Ragged batches: entry b multiplies rows [group_offsets[b], group_offsets[b+1]) of one flat
   // A with B[b] into the same rows of one flat C (m is then an upper bound of a group's rows).
   const int32_t* group_offsets;
+  int groups;       // ragged: entries of the batch (the grid is one row of tiles_m + groups tile rows)
   int a_even_odd8;  // packed int4 B only: A's bytes of every 8 k are stored as k 0,2,4,6,1,3,5,7
   // B in the fragment order of aqtx_tile_weight (batch 1): blocks of 16 rows, b_steps KiB each, a KiB holding
   // 64 bytes of each of the 16 rows (lane r + 16 c of the KiB = bytes 16 c .. 16 c + 15 of row r); rows past n
@@ -292,22 +293,46 @@ void gemm_kernel(const GemmArgs g_in) {
   const int lr = lane & 31, lh = lane >> 5;
 
   int tm, tn;
+  int64_t bz = blockIdx.y;
   if (g_in.group_offsets != nullptr) {
-    // Only the first few tile rows of a group hold work; ids run along n first, so that those
-    // rows are dealt round-robin to all XCDs (the banded walk would leave them to one XCD).
-    tm = (int)(blockIdx.x / (unsigned)g.tiles_n);
-    tn = (int)(blockIdx.x % (unsigned)g.tiles_n);
+    // The groups' tiles follow one another: a wave looks 64 groups up at a time for the one its id falls into, and the
+    // XCD-aware walk covers that group's tiles.  A grid of the largest possible group times the groups is mostly workgroups
+    // that leave at once, and each of those still waits for the LDS of a whole CU: 8192 rows in 8 groups x 4096 x 14336
+    // took 608 us that way, 552 this way; in 16 groups x 1024 x 7168 147 and 123; 700 rows in 16 x 1024 x 4096 39 and 25.
+    int id = (int)blockIdx.x, group = -1, group_tiles_m = 0;
+    for (int first = 0; first < g.groups; first += 64) {
+      int tiles = 0;
+      if (first + lane < g.groups) {
+        const int rows = g_in.group_offsets[first + lane + 1] - g_in.group_offsets[first + lane];
+        tiles = rows > 0 ? (rows + BM - 1) / BM * g.tiles_n : 0;
+      }
+      int sum = tiles;  // inclusive
+#pragma unroll
+      for (int off = 1; off < 64; off <<= 1) {
+        const int up = __shfl_up(sum, off, 64);
+        if (lane >= off) sum += up;
+      }
+      const uint64_t behind = __ballot(sum > id);
+      if (behind != 0) {
+        const int at = __builtin_ctzll(behind);
+        group = first + at;
+        id -= __shfl(sum - tiles, at, 64);
+        group_tiles_m = __shfl(tiles, at, 64) / g.tiles_n;
+        break;
+      }
+      id -= __shfl(sum, 63, 64);
+    }
+    if (group < 0) return;
+    bz = __builtin_amdgcn_readfirstlane(group);
+    tile_of_block(__builtin_amdgcn_readfirstlane(id), __builtin_amdgcn_readfirstlane(group_tiles_m), g.tiles_n, tm, tn);
   } else {
     tile_of_block(blockIdx.x, g.tiles_m, g.tiles_n, tm, tn);
   }
-  const int64_t bz = blockIdx.y;
   int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
   if (g_in.group_offsets != nullptr) {
-    // the group's row range replaces the batch strides of A, C and the row scale; tiles past
-    // the group's last row leave at once (the grid is sized for the largest possible group)
+    // the group's row range replaces the batch strides of A, C and the row scale
     const int64_t row0 = g_in.group_offsets[bz];
     const int64_t rows = g_in.group_offsets[bz + 1] - row0;
-    if (m0 >= rows) return;
     g.m = rows;
     g.a += row0 * g.lda;
     g.c = reinterpret_cast<uint8_t*>(g.c) + row0 * g.ldc * (g.out_dtype == AQTX_BF16 ? 2 : 4);
@@ -906,7 +931,15 @@ inline GemmArgs make_gemm_args(const aqtx_gemm_plan* p, const void* a, const voi
   g.tiles_m = (int)((p->m + BM - 1) / BM);
   g.tiles_n = (int)((p->n + BN - 1) / BN);
   g.group_offsets = p->group_offsets;
+  g.groups = (int)p->batch;
   return g;
+}
+
+// Grid of the 256 x 256 kernel, a workgroup per tile.  Ragged: groups of m rows in all have at most that many tile rows
+// and one begun per group.
+inline dim3 gemm_grid(const GemmArgs& g) {
+  if (g.group_offsets != nullptr) return dim3((unsigned)((int64_t)(g.tiles_m + g.groups) * g.tiles_n), 1);
+  return dim3((unsigned)(g.tiles_m * g.tiles_n), (unsigned)g.groups);
 }
 
 inline bool gemm_vector_shape_ok(const aqtx_gemm_plan* p) {

@@ -57,7 +57,7 @@ extern "C" int aqtx_gemm_fp8(const aqtx_gemm_plan* p, const void* a, const void*
   if (p->k_split <= 1 && gemm_mid_k_slices(p) > 0) return launch_gemm_fp8_mid(p, a, b, row_scale, col_scale, c, acc_out, st);
   AQTX_REQUIRE(p->lda * (int64_t)BM < (1ll << 31) && p->ldb * (int64_t)BN < (1ll << 31),
                "aqtx_gemm_fp8: leading dimension too large for 32-bit tile offsets");
-  dim3 grid((unsigned)(g.tiles_m * g.tiles_n), (unsigned)p->batch);
+  const dim3 grid = gemm_grid(g);
   const int epi = gemm_epilogue_id(p);
   if (epi < 0 || epi == 3)
     return set_error("aqtx_gemm_fp8: unsupported out/dequant/scale dtype combination (%d, %d, %d)",

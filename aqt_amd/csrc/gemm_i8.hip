@@ -106,7 +106,7 @@ extern "C" int aqtx_gemm_i8(const aqtx_gemm_plan* p, const void* a, const void* 
   }
   AQTX_REQUIRE(p->lda * (int64_t)BM < (1ll << 31) && p->ldb * (int64_t)BN < (1ll << 31),
                "aqtx_gemm_i8: leading dimension too large for 32-bit tile offsets");
-  dim3 grid((unsigned)(g.tiles_m * g.tiles_n), (unsigned)p->batch);
+  const dim3 grid = gemm_grid(g);
   const int epi = gemm_epilogue_id(p);
   if (epi < 0)
     return set_error("aqtx_gemm_i8: unsupported out/dequant/scale dtype combination (%d, %d, %d)",
