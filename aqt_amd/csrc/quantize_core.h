@@ -408,13 +408,17 @@ __device__ __forceinline__ uint2 pack8(const uint32_t (&q)[8], int even_odd8) {
 // A block is 256 threads, or 512 (LANES = 512: one long segment per block, half the row values per
 // thread, so that six waves fit a SIMD: the stochastic pipeline is bound by vector instruction
 // issue, and a wave issues one such instruction every ~12 cycles at best).
+// The bound of four waves a SIMD goes to pipelines that fit 128 registers.  int8 values of the bf16 pipelines, held as
+// floats, do not: two paired rows of eight pieces need 182, and spill 196 bytes a lane under the bound (300 rows of 9000
+// with noise: 17.7 us, 12.8 without it; 2048 of 16384: 59 and 55).
 // COLMAX (whole rows as segments, one per block, no PAIR): the grid is smaller than the number of rows, a block
 // walks rows blockIdx.x, + gridDim.x, ... and keeps, per column it owns, the largest |q| it wrote; at the end it
 // stores them as row blockIdx.x of QArgs::oa_out ([gridDim.x][cols] bytes): what a later pass that calibrates the
 // quantized values over the rows needs instead of reading them again.
 template <typename TIn, int LANES, int ITERS, int SPEC, bool PAIR, bool COLMAX = false>
 __global__ __launch_bounds__(LANES == 512 ? 512 : 256,
-                             (COLMAX && ITERS <= 2 && SPEC == 1) ? 7 : LANES == 512 ? 3 : SPEC != 0 && !COLMAX ? 4 : 1)
+                             (COLMAX && ITERS <= 2 && SPEC == 1) ? 7 : LANES == 512 ? 3
+                             : !COLMAX && ((sizeof(TIn) == 2 && SPEC != 0) || spec_is_f32(SPEC)) ? 4 : 1)
 void quant_rows_kernel(const QArgs a_in) {
   const QArgs a = with_device_key(a_in);
   constexpr int VEC = 8;
@@ -1168,8 +1172,8 @@ int launch_rows_spec(const QArgs& a, hipStream_t st) {
   if (L <= 2048) AQTX_ROWS(256, 1)
   if (L <= 4096) AQTX_ROWS(256, 2)
   if (L <= 8192) AQTX_ROWS(256, 4)
-  if (SPEC == 2 && sizeof(TIn) == 2 || SPEC == 7) AQTX_ROWS(512, 4)
-  AQTX_ROWS(256, 8)
+  if constexpr ((SPEC == 2 && sizeof(TIn) == 2) || SPEC == 7) AQTX_ROWS(512, 4)
+  else AQTX_ROWS(256, 8)
 #undef AQTX_ROWS
 }
 
