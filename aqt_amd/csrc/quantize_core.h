@@ -430,11 +430,13 @@ void quant_rows_kernel(const QArgs a_in) {
   const int tid = threadIdx.x;
   const int lane = tid % LANES;
   const int64_t nseg_grid = PAIR ? a.nseg / 2 : a.nseg;
-  // first of the eight values of piece `it`, or a.L behind the segment; a last piece that would hang over the end
-  // starts eight before it (values met twice give the same bytes and the same maximum)
-  auto piece_at = [&](int it) -> int64_t {
-    const int64_t j = (int64_t)(it * LANES + lane) * VEC;
-    return j >= a.L ? a.L : j + VEC <= a.L ? j : a.L - VEC;
+  // A last piece that would hang over the end starts eight before it (values met twice give the same bytes and the same
+  // maximum).  In 32 bits (a segment holds at most 16384 values): one minimum a piece.
+  const int len = (int)a.L;
+  auto has_piece = [&](int it) { return (it * LANES + lane) * VEC < len; };
+  auto piece_at = [&](int it) {
+    const int j = (it * LANES + lane) * VEC;
+    return j < len - VEC ? j : len - VEC;
   };
   float colmax[COLMAX ? ITERS : 1][VEC];  // largest clipped |x / scale| per column (rounded at the end)
   if constexpr (COLMAX) {
@@ -470,8 +472,8 @@ void quant_rows_kernel(const QArgs a_in) {
     uint32_t amax_packed = 0u;
 #pragma clang loop unroll(full)
     for (int it = 0; it < ITERS; ++it) {
-      const int64_t j0 = piece_at(it);
-      if (active && j0 < a.L) {
+      const int j0 = piece_at(it);
+      if (active && has_piece(it)) {
         bool stored = false;
         if constexpr (PACKED) {
           if (a.ps_mode == AQTX_PRESCALE_NONE) {  // the loaded words are the stored form
@@ -526,8 +528,8 @@ void quant_rows_kernel(const QArgs a_in) {
     const uint32_t ctr_row = (uint32_t)(grow[0] * a.cols);  // natural layout: index of (row, 0)
 #pragma clang loop unroll(full)
     for (int it = 0; it < ITERS; ++it) {
-      const int64_t j0 = piece_at(it);
-      if (active && j0 < a.L) {
+      const int j0 = piece_at(it);
+      if (active && has_piece(it)) {
         uint32_t q0[VEC], q1[VEC];
         float t0[VEC], t1[VEC];
         v[0][it].get(t0);
@@ -544,8 +546,8 @@ void quant_rows_kernel(const QArgs a_in) {
     const uint64_t ctr_row = (uint64_t)(b * a.nsb + r * a.nsr + col0[0] * a.nsc);
 #pragma clang loop unroll(full)
     for (int it = 0; it < ITERS; ++it) {
-      const int64_t j0 = piece_at(it);
-      if (active && j0 < a.L) {
+      const int j0 = piece_at(it);
+      if (active && has_piece(it)) {
         uint32_t q[VEC];
         float t[VEC];
         v[0][it].get(t);
@@ -553,10 +555,10 @@ void quant_rows_kernel(const QArgs a_in) {
         for (int e = 0; e < VEC; ++e) {
           if constexpr (COLMAX) {
             float tc;
-            q[e] = spec_quant_mag<SPEC>(t[e], inv[0], ctr_row + (uint64_t)((j0 + e) * a.nsc), a, tc);
+            q[e] = spec_quant_mag<SPEC>(t[e], inv[0], ctr_row + (uint64_t)((int64_t)(j0 + e) * a.nsc), a, tc);
             colmax[it][e] = fmaxf(colmax[it][e], fabsf(tc));
           } else {
-            q[e] = spec_quant<SPEC>(t[e], inv[0], ctr_row + (uint64_t)((j0 + e) * a.nsc), a);
+            q[e] = spec_quant<SPEC>(t[e], inv[0], ctr_row + (uint64_t)((int64_t)(j0 + e) * a.nsc), a);
           }
         }
         store8(qp0 + j0, pack8(q, a.even_odd8));
@@ -569,8 +571,8 @@ void quant_rows_kernel(const QArgs a_in) {
   if constexpr (COLMAX) {
 #pragma clang loop unroll(full)
     for (int it = 0; it < ITERS; ++it) {
-      const int64_t j0 = piece_at(it);
-      if (j0 < a.L) {
+      const int j0 = piece_at(it);
+      if (has_piece(it)) {
         uint32_t m[VEC];
 #pragma unroll
         for (int e = 0; e < VEC; ++e) m[e] = (uint32_t)(int)rintf(colmax[it][e]);
