@@ -1242,7 +1242,14 @@ int launch_tiles(const QArgs& a, int reduce, int partitionable, int64_t nscales,
       AQTX_HIP_CHECK_LAUNCH("absmax_all_kernel");
     } else {
       const dim3 grid((unsigned)absmax_col_groups(a.cols), (unsigned)(a.ngroups * ((a.G + kAbsRowChunk - 1) / kAbsRowChunk)), (unsigned)a.batch);
-      folded = a.ws_arrived != nullptr && a.cols >= 8 && (int64_t)grid.x * grid.y * grid.z < 1024;
+      // Folded up to two blocks of 16 waves a CU, one round of the chip, and float values without a prescale, which are
+      // bound by HBM bytes from there on, below one a CU (calibration and quantization, folded against not: bf16 128
+      // blocks 12.1 and 12.1 us, 256 15.7 and 14.8, 512 24.4 and 21.6, 640 28.5 and 24.1; float32 128 13.7 and 16.7,
+      // 256 19-22 and 21, 512 31.4 and 28.4; bf16 with a prescale 256 18.9 and 21.4, 512 27.3 and 28.4, 576 33.7 and
+      // 31.5; int8 256 16.3 and 17.4, 512 24.1 and 24.1, 640 28.6 and 25.9).
+      const int64_t blocks = (int64_t)grid.x * grid.y * grid.z;
+      folded = a.ws_arrived != nullptr && a.cols >= 8 &&
+               (sizeof(TIn) != 1 && a.ps_mode == AQTX_PRESCALE_NONE ? blocks < 256 : blocks <= 512);
       if (a.cols < 8) absmax_cols_kernel<TIn, 1, false><<<grid, 256, 0, st>>>(a);
       else if (folded) absmax_cols_kernel<TIn, 8, true><<<grid, 1024, 0, st>>>(a);
       else absmax_cols_kernel<TIn, 8, false><<<grid, 256, 0, st>>>(a);

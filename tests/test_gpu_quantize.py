@@ -418,6 +418,23 @@ def test_scales_from_the_last_block_equal_those_of_their_own_launch(gpu, reduce,
   assert torch.equal(results[0][1], (want / 127.5).to(torch.bfloat16).float())
 
 
+@pytest.mark.parametrize('rows,cols', [(8128, 512), (8192, 512), (8193, 1024), (16384, 1024), (16385, 1024)])
+@pytest.mark.parametrize('dt,prescaled', [('bf16', False), ('bf16', True), ('f32', False), ('i8', False)])
+def test_column_scales_on_both_sides_of_the_fold(gpu, dt, prescaled, rows, cols):
+  """Blocks of 64 rows x 512 columns: 127 to 514, with the launch for the scales and without it."""
+  x = torch.randn((1, rows, cols), generator=torch.Generator().manual_seed(rows)) * 20
+  x = {'bf16': x.to(torch.bfloat16), 'f32': x, 'i8': x.to(torch.int8)}[dt].to(gpu)
+  compute = torch.float32 if dt == 'f32' else torch.bfloat16
+  kw, want = {}, x.to(compute).float()
+  if prescaled:
+    ps = torch.exp2(torch.arange(rows, device=gpu) % 5 - 2.0)  # powers of two: the products are exact
+    kw, want = dict(prescale=ps, prescale_mode=L.PRESCALE_PER_ROW), want * ps[None, :, None]
+  q, s = ops.quantize(x, reduce=L.REDUCE_ROWS, compute_dtype=compute, out_dtype=L.I8, quant_bound=128.0, clip_bound=127.0, **kw)
+  assert torch.equal(s, (want.abs().amax(1, keepdim=True) / 128.0).to(compute).float())
+  assert torch.equal(ops.quantize(x, reduce=L.REDUCE_ROWS, compute_dtype=compute, out_dtype=L.I8, quant_bound=128.0, clip_bound=127.0,
+                                  scale=s, **kw)[0], q)
+
+
 @pytest.mark.parametrize('reduce,shape', [(L.REDUCE_COLS, (1, 5, 3000)), (L.REDUCE_COLS, (1, 3, 5)), (L.REDUCE_COLS, (2, 2, 20000)),
                                           (L.REDUCE_ROWS, (1, 300, 72)), (L.REDUCE_ALL, (2, 100, 64))])
 def test_calibration_alone_gives_the_scales_of_the_quantization(gpu, reduce, shape):
