@@ -695,8 +695,16 @@ void gemm_kernel(const GemmArgs g_in) {
     // Tiles that lie wholly inside C skip every bounds check.
     const bool interior = (em0 + BM <= g.m) && (en0 + BN <= g.n);
 
-    auto epilogue = [&](auto checked_tag) {
-      constexpr bool kChecked = decltype(checked_tag)::value;
+    // 4-byte outputs whose rows start between 16-byte boundaries go through the L2, which makes whole lines of the pieces
+    // two workgroups write of one; past it, such a piece is a partial write to memory: 2048 x 8190 float32 over k = 512
+    // 28 against 53 us, 4096 x 4099 over 1024 50 against 73.  (2-byte ones are level or ahead past it, 3000 x 3001 over
+    // 1040 26.5 against 28.8; and so are outputs beyond the 256 MB of the cache behind the L2s, 8192 x 14335 float32 over
+    // 4096 598 against 624.)
+    const bool through_l2 = kEsz == 4 && (((g.ldc * kEsz) % 16) != 0 || ((uintptr_t)cbase % 16) != 0) &&
+                            g_in.m * g.ldc * kEsz * (int64_t)gridDim.y <= (256ll << 20);
+
+    auto epilogue = [&](auto checked_tag, auto l2_tag) {
+      constexpr bool kChecked = decltype(checked_tag)::value, kThroughL2 = decltype(l2_tag)::value;
 #pragma unroll
       for (int pass = 0; pass < kPasses; ++pass) {
 #pragma unroll
@@ -760,11 +768,15 @@ void gemm_kernel(const GemmArgs g_in) {
           // Non-temporal: the output is not read again by this launch, and kept out of the L2 it leaves the
           // operand panels there (measured: 0.7 % off the launch, 1.4 % off the training step)
           const v4i vo = v4i{(int)v.x, (int)v.y, (int)v.z, (int)v.w};
+          auto store = [&] {
+            if constexpr (kThroughL2) *reinterpret_cast<v4i_unaligned*>(dst) = vo;
+            else __builtin_nontemporal_store(vo, reinterpret_cast<v4i_unaligned*>(dst));
+          };
           if constexpr (!kChecked) {
-            __builtin_nontemporal_store(vo, reinterpret_cast<v4i_unaligned*>(dst));
+            store();
           } else if (mrow0 + row < g.m && nn < g.n) {
             if (full) {
-              __builtin_nontemporal_store(vo, reinterpret_cast<v4i_unaligned*>(dst));
+              store();
             } else {
               const uint32_t w[4] = {v.x, v.y, v.z, v.w};
               const int nv = (int)(g.n - nn) < kColsPerPair ? (int)(g.n - nn) : kColsPerPair;
@@ -779,8 +791,10 @@ void gemm_kernel(const GemmArgs g_in) {
         }
       }
     };
-    if (interior && ((uintptr_t)cs % 16) == 0) epilogue(std::false_type{});
-    else epilogue(std::true_type{});
+    if (through_l2) {
+      if constexpr (kEsz == 4) epilogue(std::true_type{}, std::true_type{});
+    } else if (interior && ((uintptr_t)cs % 16) == 0) epilogue(std::false_type{}, std::false_type{});
+    else epilogue(std::true_type{}, std::false_type{});
   }
   if (!more) break;
   __syncthreads();  // the staging rows of the epilogue have been read: the next tile may fill the stages

@@ -583,3 +583,17 @@ def test_operands_the_mfma_kernels_cannot_load_are_padded(gpu, batch, m, n, k, k
                  a_dtype=dt, b_dtype=dt)
     want = torch.from_numpy(acc.astype(np.float32)).to(out).float() * torch.from_numpy(rs)[:, :, None] * torch.from_numpy(cs)[:, None, :]
     assert torch.equal(c.float().cpu(), want), out
+
+
+@pytest.mark.parametrize('n', [3001, 3002, 3004])
+def test_large_tiles_store_rows_that_start_anywhere(gpu, n):
+  """Outputs of the 256 x 256 kernel (144 tiles) whose rows start between 16-byte boundaries, and on them."""
+  m, k = 2900, 48
+  a, b = _ints((1, m, k), 3), _ints((1, n, k), 4)
+  acc = torch.from_numpy(_ref_acc(a, b))
+  ta, tb = torch.from_numpy(a).to(gpu), torch.from_numpy(b).to(gpu)
+  assert torch.equal(ops.gemm(ta, tb, row_scale=None, col_scale=None, out_dtype=torch.int32).cpu().long(), acc)
+  rs, cs = torch.exp2(torch.arange(m) % 7 - 3.0)[None], torch.exp2(torch.arange(n) % 5 - 2.0)[None]
+  for out in (torch.float32, torch.bfloat16):
+    c = ops.gemm(ta, tb, row_scale=rs.to(gpu), col_scale=cs.to(gpu), out_dtype=out)
+    assert torch.equal(c.cpu(), (acc.to(out).float() * rs[:, :, None] * cs[:, None, :]).to(out))
