@@ -434,7 +434,9 @@ void quant_rows_kernel(const QArgs a_in) {
   // maximum).  In 32 bits (a segment holds at most 16384 values): one minimum a piece.
   const int len = (int)a.L;
   auto has_piece = [&](int it) { return (it * LANES + lane) * VEC < len; };
-  auto piece_at = [&](int it) {
+  // (64 bits on the run-time pipeline, whose noise counters are: 10000 rows of 2048 float32 values to e4m3 23.1 us, 24.8
+  // with its piece positions in 32)
+  auto piece_at = [&](int it) -> std::conditional_t<SPEC == 0, int64_t, int> {
     const int j = (it * LANES + lane) * VEC;
     return j < len - VEC ? j : len - VEC;
   };
@@ -472,7 +474,7 @@ void quant_rows_kernel(const QArgs a_in) {
     uint32_t amax_packed = 0u;
 #pragma clang loop unroll(full)
     for (int it = 0; it < ITERS; ++it) {
-      const int j0 = piece_at(it);
+      const auto j0 = piece_at(it);
       if (active && has_piece(it)) {
         bool stored = false;
         if constexpr (PACKED) {
@@ -528,7 +530,7 @@ void quant_rows_kernel(const QArgs a_in) {
     const uint32_t ctr_row = (uint32_t)(grow[0] * a.cols);  // natural layout: index of (row, 0)
 #pragma clang loop unroll(full)
     for (int it = 0; it < ITERS; ++it) {
-      const int j0 = piece_at(it);
+      const auto j0 = piece_at(it);
       if (active && has_piece(it)) {
         uint32_t q0[VEC], q1[VEC];
         float t0[VEC], t1[VEC];
@@ -546,7 +548,7 @@ void quant_rows_kernel(const QArgs a_in) {
     const uint64_t ctr_row = (uint64_t)(b * a.nsb + r * a.nsr + col0[0] * a.nsc);
 #pragma clang loop unroll(full)
     for (int it = 0; it < ITERS; ++it) {
-      const int j0 = piece_at(it);
+      const auto j0 = piece_at(it);
       if (active && has_piece(it)) {
         uint32_t q[VEC];
         float t[VEC];
@@ -571,7 +573,7 @@ void quant_rows_kernel(const QArgs a_in) {
   if constexpr (COLMAX) {
 #pragma clang loop unroll(full)
     for (int it = 0; it < ITERS; ++it) {
-      const int j0 = piece_at(it);
+      const auto j0 = piece_at(it);
       if (has_piece(it)) {
         uint32_t m[VEC];
 #pragma unroll
