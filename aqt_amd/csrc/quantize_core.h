@@ -584,7 +584,8 @@ void quant_rows_kernel(const QArgs a_in) {
   }
 }
 
-// Generic rows kernel: segments shorter than 8 or longer than 16384; one wave per segment, two reads.
+// Generic rows kernel: segments shorter than 8 or longer than 16384, and others (element_rows_ahead); one wave per
+// segment, two reads.
 template <typename TIn>
 __global__ __launch_bounds__(256) void quant_rows_generic_kernel(const QArgs a_in) {
   const QArgs a = with_device_key(a_in);
@@ -1181,25 +1182,51 @@ int launch_rows_spec(const QArgs& a, hipStream_t st) {
 #undef AQTX_ROWS
 }
 
+// Whether segments whose length is no multiple of 8 go to the kernel with a wave per segment and an element a lane.  Pieces
+// of 8 are ahead where loads and stores are what a row costs (1000 rows of 1001 bf16 values 4.3 us against 9.5) and beyond
+// 2048 values always.  They lose where a lane's eight draws or conversions follow one another with too few rows to hide
+// it, and where rows are many and leave most lanes of a launch shape (128, 512, 2048 values) without a piece.  The lines
+// lie where the two measured alike; pieces / elements in us at either side of them, by pipeline:
+//   typed, no noise     570 values: 1000 rows 4.2 / 6.6, 10000 15.8 / 14.0; 700: 10000 16.0 / 16.9
+//   run time, no noise  20 values: 1000 rows 4.6 / 3.7, 8200 4.6 / 5.7; 129: 40000 24.4 / 23.2; 700: 4000 10.3 / 9.1; 1001: 10.5 / 16.1
+//   noise, paired rows  10 values: 10000 rows 13.5 / 7.5, 30000 14.6 / 16.6; 31: 1000 5.2 / 3.9, 8200 6.1 / 6.9; 100: 1000
+//                       5.2 / 4.4, 4000 5.3 / 5.9; 129: 100 5.3 / 5.1, 4000 6.6 / 7.3; 570: 1000 6.9 / 8.5, 10000 29.2 / 25.4
+//   noise otherwise     10 values: 30000 rows 17.2 / 16.4, 40000 19.6 / 20.9; 31: 10000 8.3 / 7.5, 30000 15.4 / 16.7; 100: 1000
+//                       5.9 / 4.4, 8200 8.0 / 8.8; 300: 10000 19.3 / 16.9; 511: 19.7 / 23.4; 700: 1000 7.6 / 9.8, 4000 19.8 / 15.5
+inline bool element_rows_ahead(const QArgs& a, int spec, bool paired) {
+  const int64_t L = a.L, n = a.nseg;
+  if (L % 8 == 0 || L > 2048 || a.even_odd8) return false;
+  struct Lines {
+    int64_t below16, below64, below128;     // fewer segments than this of a length below 16, 64, 128
+    int64_t mid_length, mid_segments;       // lengths beyond 128 below, and fewer segments than
+    int64_t long_length, long_segments;     // lengths beyond 512 below, and at least so many segments
+  };
+  constexpr int64_t kAny = INT64_MAX;
+  constexpr Lines kTyped{0, 0, 0, 0, 0, 640, 4096}, kRunTime{4096, 4096, 2048, 160, kAny, 800, 2048},
+      kPaired{20480, 6144, 2048, 256, 2048, 640, 4096}, kNoise{32768, 16384, 4096, 400, kAny, 1024, 2048};
+  const Lines& l = a.noise == AQTX_NOISE_NONE ? (spec != 0 ? kTyped : kRunTime) : paired ? kPaired : kNoise;
+  if (L < 128) return n < (L < 16 ? l.below16 : L < 64 ? l.below64 : l.below128);
+  if (L < 512) return L < l.mid_length && n < l.mid_segments;
+  return L < l.long_length && n >= l.long_segments;
+}
+
 template <typename TIn>
 int launch_rows(const QArgs& a, int partitionable, hipStream_t st) {
   const int64_t L = a.L;
   AQTX_REQUIRE(!a.even_odd8 || (L % 8 == 0 && a.cols % 8 == 0 && L <= 16384),
                "aqtx_quantize: out_k_order = EVEN_ODD8 needs cols and group to be multiples of 8 and "
                "segments of at most 16384");
-  // (a length that is no multiple of 8 in one wave per segment, an element a lane: 1999 rows of 1030 bf16 values 14 us, the
-  // same of 3001 with noise 56; in pieces of 8 they take 7 and 23)
-  if (L < 8 || L > 16384) {
-    const int64_t blocks = (a.nseg + 3) / 4;
-    quant_rows_generic_kernel<TIn><<<dim3((unsigned)blocks), 256, 0, st>>>(a);
-    AQTX_HIP_CHECK_LAUNCH("quant_rows_generic_kernel");
-    return 0;
-  }
   const int spec = spec_of(a, partitionable);
   // one threefry block serves elements i and i + total/2: pair whole rows when the noise counters follow the
   // natural [batch*rows, cols] order
   const bool natural = a.nsc == 1 && a.nsr == a.cols && (a.batch == 1 || a.nsb == a.rows * a.cols) &&
                        L == a.cols && (a.nseg % 2 == 0);
+  if (L < 8 || L > 16384 || element_rows_ahead(a, spec, natural && spec_has_uniform_noise(spec))) {
+    const int64_t blocks = (a.nseg + 3) / 4;
+    quant_rows_generic_kernel<TIn><<<dim3((unsigned)blocks), 256, 0, st>>>(a);
+    AQTX_HIP_CHECK_LAUNCH("quant_rows_generic_kernel");
+    return 0;
+  }
   // (oa_out: the caller has checked rows_colmax_ok: noise none, so spec is 1, 6 or 0; float input is held in the
   // compute dtype, so the bf16 pipelines never meet float32 input nor the float32 ones bf16 input)
   if constexpr (sizeof(TIn) != 4) {

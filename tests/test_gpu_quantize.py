@@ -382,6 +382,28 @@ def test_sizes_that_are_no_multiples_of_anything(gpu, dt, bits, noise, rows, col
   _check(_oracle_quant(x, dt, q, [1], ps, 1), qg.cpu().numpy(), sg.cpu().numpy(), q, transpose=True)
 
 
+@pytest.mark.parametrize('rows,cols,dt,bits,noise', [
+    # even row counts share the generator's blocks between rows, odd ones do not; either side of a line where it matters
+    (20478, 9, 'bf16', 8, 'jax.uniform'), (20480, 9, 'bf16', 8, 'jax.uniform'), (6142, 31, 'f32', 8, 'jax.uniform'),
+    (6144, 31, 'f32', 8, 'jax.uniform'), (2046, 129, 'bf16', 8, 'jax.uniform'), (2048, 129, 'bf16', 8, 'jax.uniform'),
+    (4096, 570, 'bf16', 8, 'jax.uniform'), (32769, 10, 'bf16', 8, 'jax.uniform'), (4097, 100, 'f32', 8, 'jax.uniform'),
+    (2049, 399, 'bf16', 8, 'jax.uniform'), (2049, 401, 'bf16', 8, 'jax.uniform'), (2049, 1023, 'f32', 'e5m2', 'sr'),
+    (4096, 639, 'bf16', 8, None), (4096, 641, 'bf16', 8, None), (4095, 20, 'f32', 'e4m3', None), (4096, 20, 'f32', 'e4m3', None),
+    (2048, 799, 'f32', 'e4m3', None),
+])
+def test_row_kernels_on_both_sides_of_their_lines(gpu, rows, cols, dt, bits, noise):
+  q = R.QuantizerCfg(bits=bits, key=prng.prng_key(rows + cols))
+  if noise == 'sr':
+    q.fp8_sr = True
+  elif noise:
+    q.noise = noise
+  qb, cb = U.bounds(q)
+  x = U.rand((1, rows, cols), dt, seed=rows + cols, outliers=True)
+  qg, sg = ops.quantize(U.to_dev(x, dt, gpu), reduce=L.REDUCE_COLS, out_dtype=U.OUT_DT[bits], quant_bound=qb, clip_bound=cb,
+                        noise={None: L.NOISE_NONE, 'sr': L.NOISE_FP8_MANTISSA}.get(noise, U.NOISE.get(noise)), key=q.key)
+  _check(R.quantize(x, dt, q, [2]), qg.cpu().numpy(), sg.cpu().numpy(), q)
+
+
 @pytest.mark.parametrize('reduce,shape,group', [
     (L.REDUCE_ROWS, (1, 4096, 600), 0), (L.REDUCE_ROWS, (2, 130, 1025), 0), (L.REDUCE_ROWS, (1, 16, 5), 0),
     (L.REDUCE_ROWS, (2, 256, 513), 64), (L.REDUCE_ALL, (3, 1000, 257), 0), (L.REDUCE_ALL_BATCH, (3, 1000, 257), 0),
