@@ -950,6 +950,9 @@ __global__ __launch_bounds__(256) void quant_tile_kernel(const QArgs a_in) {
   // Tiles that lie wholly inside the tensor (and inside the first half of a paired axis) take a
   // branch-free path with vector loads of the reciprocal scales and the pre-scale factors.
   const bool interior = (r0[0] + kTileR <= row_lim) && (c0[0] + kTileC <= col_lim) && a.ssc <= 1;
+  // Every lane of the tile that has values has eight: one decision for the tile, before each lane's own (64 x 64 values
+  // with noise and one scale 15.3 us; 18.8 with the lanes' decision alone).
+  const bool whole = a.cols % 8 == 0 && col_lim % 8 == 0;
   // Given scales: the tile's reciprocals are computed here (LDS), where the rows of a column share one
   __shared__ float inv_lds[NSET][kTileC];
   const bool inv_here = a.scale_given && a.ngroups == 1;
@@ -983,7 +986,9 @@ __global__ __launch_bounds__(256) void quant_tile_kernel(const QArgs a_in) {
 #pragma unroll
         for (int s = 0; s < NSET; ++s) {
           const int64_t r = r0[s] + rg * 4 + j, c = c0[s] + cc * 8;
-          if (FAST || nvalid == 8) {
+          if (FAST || whole) {
+            Loader<TIn>::load8(xb + r * a.cols + c, x[s]);
+          } else if (nvalid == 8) {
             Loader<TIn>::load8(xb + r * a.cols + c, x[s]);
           } else {
 #pragma unroll
@@ -1075,7 +1080,9 @@ __global__ __launch_bounds__(256) void quant_tile_kernel(const QArgs a_in) {
 #pragma unroll
           for (int s = 0; s < NSET; ++s) {
             const int64_t r = r0[s] + rg * 4 + j, c = c0[s] + cc * 8;
-            if (FAST || nvalid == 8) {
+            if (FAST || whole) {
+              store8(qb + r * a.cols + c, make_uint2(w[s][0], w[s][1]));
+            } else if (nvalid == 8) {
               store8(qb + r * a.cols + c, make_uint2(w[s][0], w[s][1]));
             } else {
               for (int e = 0; e < nvalid; ++e)
