@@ -367,16 +367,18 @@ def gemm(
     assert a.shape[0] == 1 and group_offsets.dtype == torch.int32 and group_offsets.is_cuda
     assert group_offsets.numel() == b.shape[0] + 1 and group_offsets.is_contiguous()
   fp8 = a_dtype in (L.E4M3, L.E5M2)
-  if b_layout == L.W_ROWS and b_dtype != L.I4P and group_offsets is None and k_split <= 1 and _pads_rows(a, b, fp8):
+  out_dt = aqtx_dtype(out_dtype)
+  dq_dt = aqtx_dtype(dequant_dtype) if dequant_dtype is not None else (out_dt if out_dt != L.I32 else L.F32)
+  sc_dt = aqtx_dtype(scale_dtype) if scale_dtype is not None else dq_dt
+  # (the MFMA kernels have no epilogue that dequantizes in one float dtype and writes another; the element kernel has)
+  if (b_layout == L.W_ROWS and b_dtype != L.I4P and group_offsets is None and 0 <= k_split <= 1
+      and out_dt in (L.I32, dq_dt) and _pads_rows(a, b, fp8)):
     a, b = _pad_rows(a, b)
     k, ldb, stride_b = a.shape[2], b.stride(1), b.stride(0)
     if fp8:
       # what such operands always had: float32 sums of whole products (relative error against 64 bits, e4m3: 8.2e-9 at
       # k = 129 and 7.8e-8 at 4095, one thread per element 8.6e-9 and 7.9e-8)
       accumulate = L.ACC_F32
-  out_dt = aqtx_dtype(out_dtype)
-  dq_dt = aqtx_dtype(dequant_dtype) if dequant_dtype is not None else (out_dt if out_dt != L.I32 else L.F32)
-  sc_dt = aqtx_dtype(scale_dtype) if scale_dtype is not None else dq_dt
   alloc = torch.zeros if group_offsets is not None and group_sizes is None else torch.empty
   c = alloc((batch, m, n), dtype=_AQTX_TO_TORCH[out_dt], device=a.device)
   if group_sizes is not None:

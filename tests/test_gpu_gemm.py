@@ -597,3 +597,24 @@ def test_large_tiles_store_rows_that_start_anywhere(gpu, n):
   for out in (torch.float32, torch.bfloat16):
     c = ops.gemm(ta, tb, row_scale=rs.to(gpu), col_scale=cs.to(gpu), out_dtype=out)
     assert torch.equal(c.cpu(), (acc.to(out).float() * rs[:, :, None] * cs[:, None, :]).to(out))
+
+
+@pytest.mark.parametrize('kind', ['i8', 'e4m3'])
+@pytest.mark.parametrize('out,dequant', [(torch.float32, torch.bfloat16), (torch.bfloat16, torch.float32)])
+@pytest.mark.parametrize('m,n,k', [(3, 5, 7), (130, 70, 129)])
+def test_unaligned_operands_dequantized_in_another_dtype_than_written(gpu, m, n, k, out, dequant, kind):
+  """A pair of dtypes that only the kernel for unaligned operands has: taken at every size."""
+  a, b = (np.random.default_rng(s).integers(-2, 3, size=(1, r, k)) for s, r in ((1, m), (2, n)))
+  acc = torch.from_numpy(_ref_acc(a, b)).float()
+  rs, cs = torch.exp2(torch.arange(m) % 7 - 3.0)[None], torch.exp2(torch.arange(n) % 5 - 2.0)[None]
+
+  def operand(v):
+    t = torch.from_numpy(v).to(gpu)
+    return t.to(torch.int8) if kind == 'i8' else t.float().to(torch.float8_e4m3fn).view(torch.uint8)
+
+  dt = L.I8 if kind == 'i8' else L.E4M3
+  c = ops.gemm(operand(a), operand(b), row_scale=rs.to(gpu), col_scale=cs.to(gpu), out_dtype=out, dequant_dtype=dequant,
+               a_dtype=dt, b_dtype=dt)
+  want = acc.to(dequant).float() * rs[:, :, None]
+  want = (want.to(dequant).float() * cs[:, None, :]).to(dequant).to(out)
+  assert c.dtype == out and torch.equal(c.cpu(), want)
