@@ -365,3 +365,45 @@ def test_operand_views_over_memory_orders_and_axis_groups(rank):
           i, j, k = torch.meshgrid(*(torch.arange(n) for n in (v.B, v.R, v.K)), indexing='ij')
           sb, sr, sk = v.noise_strides
           assert torch.equal(index, i * sb + j * sr + k * sk)
+
+
+def test_copies_of_settings_ask_the_class():
+  """Configurations are copied field by field; a class with a copy of its own is asked for it, whatever its base."""
+  import abc
+
+  class Base(abc.ABC):
+    def __init__(self):
+      self.n = 1
+
+  class Copies(Base):
+    def __copy__(self):
+      out = type(self)()
+      out.n = self.n + 10
+      return out
+
+  class Restores(Base):
+    def __setstate__(self, state):
+      self.__dict__.update(state)
+      self.restored = True
+
+  class Made(Base):
+    def __new__(cls, *args):
+      out = super().__new__(cls)
+      out.made = True
+      return out
+
+  class Reduced(Base):
+    def __reduce__(self):
+      return (type(self), (), {'n': 5})
+
+  class Slotted(Base):
+    __slots__ = ('more',)
+
+  assert utils.clone_fields(Base()).n == 1
+  assert utils.clone_fields(Copies()).n == 11
+  assert utils.clone_fields(Restores()).restored
+  assert utils.clone_fields(Made()).made
+  assert utils.clone_fields(Reduced()).n == 5
+  x = Slotted()
+  x.more = 3
+  assert utils.clone_fields(x).more == 3 and utils.clone_fields(x).n == 1
