@@ -196,8 +196,8 @@ class Quantizer:
     rest = [a for a in range(x.dim()) if a not in shared]
     v = lowering.view_operand(x, [], rest, shared)
     per_tensor = s.numel() == 1
-    sv = lowering.view_operand(lowering.scale_f32(s), [], rest, shared)
-    s32 = sv.mem.reshape(-1).contiguous()
+    sv = lowering.view_operand(s, [], rest, shared)
+    s32 = sv.mem.reshape(-1).float().contiguous()
     s_in = s32.reshape(1) if per_tensor else s32.reshape(1, v.R, 1) if v.k_last else s32.reshape(1, 1, v.R)
     q, _ = lowering.quantize_view(
         v, spec=spec, compute_dtype=x.dtype, scale_dtype=s.dtype,

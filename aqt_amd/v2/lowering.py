@@ -214,11 +214,3 @@ def scale_in_dtype(s32: torch.Tensor, v: OperandView, sdt) -> torch.Tensor:
   if sdt != torch.float32:
     out.f32_copy = f32  # same values, for kernels that take float32 scale vectors
   return out
-
-
-def scale_f32(scale: torch.Tensor) -> torch.Tensor:
-  """`scale` in float32: the copy the quantize kernels left beside it (scale_in_dtype), unless it was written to since."""
-  src = getattr(scale, 'f32_copy', None)
-  if src is not None and src.shape == scale.shape and not scale.is_inference() and scale._version == 0:
-    return src
-  return scale.float()

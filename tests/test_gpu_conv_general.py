@@ -309,3 +309,25 @@ def test_conv_layer_with_128_features_matches_oracle(gpu):
                                             R.RawCfg(_qcfg(8, po2=False), _qcfg(8, po2=False)), case.get('dil'))
     assert tuple(out.shape) == want.shape
     np.testing.assert_array_equal(out.float().cpu().numpy(), want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('cout', [128, 24])  # with and without a window matrix
+def test_scales_written_past_autograd_are_the_ones_used(gpu, cout):
+  """A scale of a quantized tensor changed through .data (which no version counts) before the tensor is used again."""
+  from aqt_amd.v2 import aqt_conv_general
+  conv = aqt_conv_general.make_conv_general_dilated_with_qt(aqt_conv_general.conv_general_dilated_make(2, 8, 8))
+  x = U.to_dev(_rand_unif((2, 7, 7, 16), 1.0, 1, 'bf16'), 'bf16', gpu)
+  w = U.to_dev(_rand_unif((3, 3, 16, cout), 1.0, 2, 'bf16'), 'bf16', gpu)
+  kw = dict(window_strides=(1, 1), padding='SAME', dimension_numbers=aqt_conv_general.flax_conv_dimension_numbers(x.shape))
+  out, (lq, rq) = conv(x, w, **kw)
+  rq.scale[0].data.mul_(2)
+  lq.scale[0].data = lq.scale[0] * 4
+  assert torch.equal(conv(x, w, lhs_qt=lq, rhs_qt=rq, **kw)[0], out * 8)
+
+  quantizer = aqt_conv_general.conv_general_dilated_make(2, 8, 8).dg_quantizer.rhs
+  qt = quantizer.calibrate(w, calibration_axes=[0, 1, 2])
+  qt.scale[0].data.mul_(2)
+  got, _ = quantizer.calculate_qvalue(w, qt)
+  want = torch.clamp(torch.round((w * (1 / qt.scale[0]))), -127, 127).to(torch.int8)
+  assert torch.equal(got.qvalue, want)
