@@ -41,7 +41,6 @@ class QuantPlan(ctypes.Structure):
       ('out_k_order', ctypes.c_int32),
       ('other_axis_absmax', ctypes.c_void_p),
       ('absmax_partials', ctypes.c_void_p), ('absmax_parts', ctypes.c_int64),
-      ('scale_only', ctypes.c_int32),
   ]
 
 
@@ -96,7 +95,6 @@ class DecodePlan(ctypes.Structure):
       ('quant_bound', ctypes.c_float), ('clip_bound', ctypes.c_float),
       ('w_dtype', ctypes.c_int32), ('tuning', ctypes.c_int32), ('w_layout', ctypes.c_int32),
       ('workspace_zeroed', ctypes.c_int32),
-      ('x_scale_typed', ctypes.c_void_p),
   ]
 
 
@@ -129,6 +127,7 @@ SYMBOLS = {
                                      ctypes.c_size_t, _vp]),
     'aqtx_quantize_workspace_bytes': (ctypes.c_size_t, [ctypes.POINTER(QuantPlan)]),
     'aqtx_quantize_other_axis_parts': (ctypes.c_int64, [ctypes.POINTER(QuantPlan)]),
+    'aqtx_calibrate': (ctypes.c_int, [ctypes.POINTER(QuantPlan), _vp, _vp, _vp, _vp, ctypes.c_size_t, _vp]),
     'aqtx_dequantize': (ctypes.c_int, [ctypes.POINTER(QuantPlan), _vp, _vp, _vp, _vp]),
     'aqtx_scale_cast': (ctypes.c_int, [ctypes.POINTER(ScalePlan), _vp, _vp, _vp, _vp, _vp]),
     'aqtx_gemm_i8': (ctypes.c_int, [ctypes.POINTER(GemmPlan), _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
@@ -140,6 +139,8 @@ SYMBOLS = {
     'aqtx_gemm_weight_only': (ctypes.c_int, [ctypes.POINTER(GemmPlan), _vp, _vp, _vp, _vp, _vp]),
     'aqtx_decode_i8': (ctypes.c_int, [ctypes.POINTER(DecodePlan), _vp, _vp, _vp, _vp, _vp, _vp,
                                       _vp, ctypes.c_size_t, _vp]),
+    'aqtx_decode_i8_typed': (ctypes.c_int, [ctypes.POINTER(DecodePlan), _vp, _vp, _vp, _vp, _vp, _vp, _vp,
+                                            _vp, ctypes.c_size_t, _vp]),
     'aqtx_decode_workspace_bytes': (ctypes.c_size_t, [ctypes.POINTER(DecodePlan)]),
     'aqtx_decode_exchange_bytes': (ctypes.c_size_t, [ctypes.POINTER(DecodePlan)]),
     'aqtx_tile_weight_bytes': (ctypes.c_size_t, [ctypes.c_int64, ctypes.c_int64, ctypes.c_int32]),

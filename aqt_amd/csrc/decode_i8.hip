@@ -1200,7 +1200,7 @@ extern "C" size_t aqtx_decode_exchange_bytes(const aqtx_decode_plan* p) {
 namespace {
 
 int decode_impl(const aqtx_decode_plan* p, const void* x, const void* w, const float* w_scale, void* xq,
-                float* x_scale, void* out, void* workspace, size_t workspace_bytes, void* stream) {
+                float* x_scale, void* x_scale_typed, void* out, void* workspace, size_t workspace_bytes, void* stream) {
   if (p->m == 0 || p->n == 0) return 0;
   AQTX_REQUIRE(x != nullptr && w != nullptr && w_scale != nullptr && x_scale != nullptr && out != nullptr,
                "aqtx_decode_i8: NULL buffer");
@@ -1218,7 +1218,7 @@ int decode_impl(const aqtx_decode_plan* p, const void* x, const void* w, const f
   d.xs_bf16 = p->x_scale_dtype == AQTX_BF16;
   d.ws_bf16 = p->w_scale_dtype == AQTX_BF16;
   d.x = x; d.x_scale_out = x_scale;
-  d.x_scale_typed = d.xs_bf16 ? reinterpret_cast<uint16_t*>(p->x_scale_typed) : nullptr;
+  d.x_scale_typed = reinterpret_cast<uint16_t*>(x_scale_typed);
   d.quant_bound = p->quant_bound; d.clip_bound = p->clip_bound; d.x_bf16 = xbf;
   d.acc_shift = pk ? 4 : 0;
   d.w_frag = p->w_layout == AQTX_W_FRAGMENTS;
@@ -1374,7 +1374,18 @@ extern "C" int aqtx_decode_i8(const aqtx_decode_plan* p, const void* x, const vo
                               void* workspace, size_t workspace_bytes, void* stream) {
   clear_error();
   if (int rc = validate_decode(p)) return rc;
-  return decode_impl(p, x, w, w_scale, xq, x_scale, out, workspace, workspace_bytes, stream);
+  return decode_impl(p, x, w, w_scale, xq, x_scale, nullptr, out, workspace, workspace_bytes, stream);
+}
+
+extern "C" int aqtx_decode_i8_typed(const aqtx_decode_plan* p, const void* x, const void* w,
+                                    const float* w_scale, void* xq, float* x_scale, void* x_scale_typed, void* out,
+                                    void* workspace, size_t workspace_bytes, void* stream) {
+  clear_error();
+  if (int rc = validate_decode(p)) return rc;
+  AQTX_REQUIRE(p->x_scale_dtype == AQTX_BF16, "aqtx_decode_i8_typed: x_scale_dtype must be bf16, got %d", p->x_scale_dtype);
+  AQTX_REQUIRE(p->m == 0 || p->n == 0 || (x_scale_typed != nullptr && ((uintptr_t)x_scale_typed % 2) == 0),
+               "aqtx_decode_i8_typed: x_scale_typed is NULL or not element aligned");
+  return decode_impl(p, x, w, w_scale, xq, x_scale, x_scale_typed, out, workspace, workspace_bytes, stream);
 }
 
 extern "C" int aqtx_decode_i8_check(void* workspace, size_t workspace_bytes, void* stream) {
@@ -1410,7 +1421,7 @@ extern "C" int aqtx_decode_i8_static(const aqtx_decode_plan* p, const void* x, c
   // cleared by its first kernel, never assumed to be zero.
   aqtx_decode_plan plan = *p;
   plan.workspace_zeroed = 0;
-  return decode_impl(&plan, x, w, w_scale, xq, x_scale, out, ws, kStaticScratchBytes, stream);
+  return decode_impl(&plan, x, w, w_scale, xq, x_scale, nullptr, out, ws, kStaticScratchBytes, stream);
 }
 
 extern "C" size_t aqtx_tile_weight_bytes(int64_t n, int64_t k, int32_t w_dtype) {

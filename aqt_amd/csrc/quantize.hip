@@ -146,8 +146,6 @@ static bool long_rows_as_batches(const aqtx_quant_plan* p, aqtx_quant_plan* q) {
   return true;
 }
 
-static bool long_rows_as_batches(const aqtx_quant_plan* p, aqtx_quant_plan* q);
-
 extern "C" int64_t aqtx_quantize_other_axis_parts(const aqtx_quant_plan* p) {
   aqtx_quant_plan alt;
   if (p == nullptr || p->scale_given || long_rows_as_batches(p, &alt)) return 0;
@@ -166,18 +164,18 @@ extern "C" size_t aqtx_quantize_workspace_bytes(const aqtx_quant_plan* p) {
   return (size_t)scale_count(p) * 8;
 }
 
-extern "C" int aqtx_quantize(const aqtx_quant_plan* p, const void* x, const float* prescale,
-                             void* q, float* scale, void* workspace, size_t workspace_bytes,
-                             void* stream) {
-  clear_error();
+// scale_only: q is neither read nor written (aqtx_calibrate).
+static int quantize_impl(const aqtx_quant_plan* p, const void* x, const float* prescale, void* q, float* scale, bool scale_only,
+                         void* workspace, size_t workspace_bytes, void* stream) {
   if (int rc = validate(p)) return rc;
   aqtx_quant_plan alt;
-  if (long_rows_as_batches(p, &alt)) return aqtx_quantize(&alt, x, prescale, q, scale, workspace, workspace_bytes, stream);
+  if (long_rows_as_batches(p, &alt))
+    return quantize_impl(&alt, x, prescale, q, scale, scale_only, workspace, workspace_bytes, stream);
   const int64_t total = p->batch * p->rows * p->cols;
   if (total == 0) return 0;
-  AQTX_REQUIRE(x != nullptr && (q != nullptr || p->scale_only) && scale != nullptr, "aqtx_quantize: NULL buffer");
-  AQTX_REQUIRE(!p->scale_only || (p->noise == AQTX_NOISE_NONE && !p->scale_given && p->other_axis_absmax == nullptr),
-               "aqtx_quantize: scale_only goes without noise, a given scale and other_axis_absmax");
+  AQTX_REQUIRE(x != nullptr && (q != nullptr || scale_only) && scale != nullptr, "aqtx_quantize: NULL buffer");
+  AQTX_REQUIRE(!scale_only || (p->noise == AQTX_NOISE_NONE && !p->scale_given && p->other_axis_absmax == nullptr),
+               "aqtx_calibrate (scale_only) goes without noise, a given scale and other_axis_absmax");
   AQTX_REQUIRE((p->prescale == AQTX_PRESCALE_NONE) == (prescale == nullptr),
                "aqtx_quantize: prescale pointer does not match plan->prescale");
   AQTX_REQUIRE(p->batch <= 65535, "aqtx_quantize: batch %lld exceeds 65535", (long long)p->batch);
@@ -196,7 +194,7 @@ extern "C" int aqtx_quantize(const aqtx_quant_plan* p, const void* x, const floa
   a.x = x; a.prescale = prescale; a.q = q; a.scale = scale;
   a.scale_bf16 = (p->scale_typed != nullptr && p->scale_dtype == AQTX_BF16 && !p->scale_given)
                      ? reinterpret_cast<uint16_t*>(p->scale_typed) : nullptr;
-  a.scale_only = p->scale_only;
+  a.scale_only = scale_only;
   a.batch = p->batch; a.rows = p->rows; a.cols = p->cols;
   a.nsb = p->noise_stride_batch; a.nsr = p->noise_stride_row; a.nsc = p->noise_stride_col;
   a.quant_bound = p->quant_bound; a.clip_bound = p->clip_bound;
@@ -265,6 +263,19 @@ extern "C" int aqtx_quantize(const aqtx_quant_plan* p, const void* x, const floa
     case AQTX_BF16: return launch_quantize_bf16(a, p->reduce, p->partitionable, nscales, st);
     default: return launch_quantize_i8(a, p->reduce, p->partitionable, nscales, st);
   }
+}
+
+extern "C" int aqtx_quantize(const aqtx_quant_plan* p, const void* x, const float* prescale,
+                             void* q, float* scale, void* workspace, size_t workspace_bytes,
+                             void* stream) {
+  clear_error();
+  return quantize_impl(p, x, prescale, q, scale, false, workspace, workspace_bytes, stream);
+}
+
+extern "C" int aqtx_calibrate(const aqtx_quant_plan* p, const void* x, const float* prescale, float* scale, void* workspace,
+                              size_t workspace_bytes, void* stream) {
+  clear_error();
+  return quantize_impl(p, x, prescale, nullptr, scale, true, workspace, workspace_bytes, stream);
 }
 
 extern "C" int aqtx_dequantize(const aqtx_quant_plan* p, const void* q, const float* scale,

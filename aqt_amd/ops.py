@@ -233,7 +233,6 @@ def quantize(
     assert scale.dtype == torch.float32 and scale.is_contiguous() and tuple(scale.shape) == sshape
   fp8 = out_dtype in (L.E4M3, L.E5M2)
   qshape = (b, c, r) if transpose_out else (b, r, c)
-  plan.scale_only = int(scale_only)
   q = None if scale_only else torch.empty(qshape, dtype=torch.uint8 if fp8 else torch.int8, device=x.device)
   if prescale is not None:
     assert prescale.dtype == torch.float32 and prescale.is_contiguous()
@@ -253,8 +252,11 @@ def quantize(
   ws = _quantize_workspace(ws_bytes, x.device) if ws_bytes else None
   plan.workspace_zeroed = int(ws is not None)
   try:
-    L.check(lib.aqtx_quantize(ctypes.byref(plan), _ptr(x), _ptr(prescale), _ptr(q), _ptr(scale),
-                              _ptr(ws), ws.numel() if ws is not None else 0, _stream()))
+    tail = (_ptr(scale), _ptr(ws), ws.numel() if ws is not None else 0, _stream())
+    if scale_only:
+      L.check(lib.aqtx_calibrate(ctypes.byref(plan), _ptr(x), _ptr(prescale), *tail))
+    else:
+      L.check(lib.aqtx_quantize(ctypes.byref(plan), _ptr(x), _ptr(prescale), _ptr(q), *tail))
   except Exception:
     _QUANT_WS.clear()  # a failed launch sequence may have left abs-max words behind
     raise
@@ -535,13 +537,14 @@ def decode(x: torch.Tensor, w_q: torch.Tensor, w_scale: torch.Tensor, *, quant_b
   x_scale = torch.empty((m,), dtype=torch.float32, device=x.device)
   if want_typed_scale:
     x_scale.typed = torch.empty((m,), dtype=torch.bfloat16, device=x.device) if plan.x_scale_dtype == L.BF16 else None
-    plan.x_scale_typed = x_scale.typed.data_ptr() if x_scale.typed is not None else None
   if static_scratch:
     out = torch.empty((m, n), dtype=x.dtype, device=x.device)
     xq = torch.empty((m, k), dtype=torch.int8, device=x.device) if want_xq else None
     with _timed('decode'):
       L.check(L.lib().aqtx_decode_i8_static(ctypes.byref(plan), _ptr(x), _ptr(w_q), _ptr(w_scale), _ptr(xq),
                                             _ptr(x_scale), _ptr(out), _stream()))
+    if want_typed_scale and x_scale.typed is not None:
+      x_scale.typed.copy_(x_scale)
     return (out, x_scale, xq) if want_xq else (out, x_scale)
   ws_bytes = int(L.lib().aqtx_decode_workspace_bytes(ctypes.byref(plan)))
   ex_bytes = int(L.lib().aqtx_decode_exchange_bytes(ctypes.byref(plan)))
@@ -552,8 +555,12 @@ def decode(x: torch.Tensor, w_q: torch.Tensor, w_scale: torch.Tensor, *, quant_b
   xq = torch.empty((m, k), dtype=torch.int8, device=x.device) if want_xq else None
   try:
     with _timed('decode'):
-      L.check(L.lib().aqtx_decode_i8(ctypes.byref(plan), _ptr(x), _ptr(w_q), _ptr(w_scale), _ptr(xq),
-                                     _ptr(x_scale), _ptr(out), _ptr(ws), ws.numel(), _stream()))
+      operands = (ctypes.byref(plan), _ptr(x), _ptr(w_q), _ptr(w_scale), _ptr(xq), _ptr(x_scale))
+      tail = (_ptr(out), _ptr(ws), ws.numel(), _stream())
+      if want_typed_scale and x_scale.typed is not None:
+        L.check(L.lib().aqtx_decode_i8_typed(*operands, _ptr(x_scale.typed), *tail))
+      else:
+        L.check(L.lib().aqtx_decode_i8(*operands, *tail))
   except Exception:
     _QUANT_WS.clear()  # a failed launch sequence may have left partial sums behind
     raise

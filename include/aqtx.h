@@ -116,8 +116,6 @@ typedef struct aqtx_quant_plan {
   void* other_axis_absmax;
   const void* absmax_partials;
   int64_t absmax_parts;
-  int32_t scale_only;       /* 1: calibration alone: the scales are written, q is not (it may be NULL); noise NONE and no
-                               given scale */
 } aqtx_quant_plan;
 
 /*
@@ -137,6 +135,13 @@ typedef struct aqtx_quant_plan {
 int aqtx_quantize(const aqtx_quant_plan* plan, const void* x, const float* prescale,
                   void* q, float* scale, void* workspace, size_t workspace_bytes,
                   void* stream);
+
+/*
+ * aqtx_calibrate: the scales aqtx_quantize would write for the plan, and nothing else (AbsMaxCalibration on its own,
+ * aqt/jax/v2/calibration.py:117-157): noise AQTX_NOISE_NONE, no given scale and no other_axis_absmax.
+ */
+int aqtx_calibrate(const aqtx_quant_plan* plan, const void* x, const float* prescale, float* scale, void* workspace,
+                   size_t workspace_bytes, void* stream);
 
 /* Scratch bytes aqtx_quantize needs for `plan` (0 for single-pass plans). */
 size_t aqtx_quantize_workspace_bytes(const aqtx_quant_plan* plan);
@@ -501,8 +506,6 @@ typedef struct aqtx_decode_plan {
                              the scratch lives in the LAST bytes of the workspace: one shared by plans
                              of different shapes must hold the largest exchange size plus the largest
                              (workspace_bytes - exchange_bytes) of those plans.                      */
-  void* x_scale_typed;    /* optional out [m]: the activation scales once more as bf16 elements (aqtx_decode_i8 with
-                             x_scale_dtype AQTX_BF16 only; ignored otherwise)                        */
 } aqtx_decode_plan;
 
 /*
@@ -526,6 +529,10 @@ typedef struct aqtx_decode_plan {
 int aqtx_decode_i8(const aqtx_decode_plan* plan, const void* x, const void* w,
                    const float* w_scale, void* xq, float* x_scale, void* out,
                    void* workspace, size_t workspace_bytes, void* stream);
+/* The same, and the activation scales once more as bf16 elements [m] in x_scale_typed (x_scale_dtype AQTX_BF16). */
+int aqtx_decode_i8_typed(const aqtx_decode_plan* plan, const void* x, const void* w,
+                         const float* w_scale, void* xq, float* x_scale, void* x_scale_typed, void* out,
+                         void* workspace, size_t workspace_bytes, void* stream);
 size_t aqtx_decode_workspace_bytes(const aqtx_decode_plan* plan);
 /* Leading bytes of the workspace that hold the partial-sum exchange and the control words (see workspace_zeroed). */
 size_t aqtx_decode_exchange_bytes(const aqtx_decode_plan* plan);

@@ -26,6 +26,24 @@ def test_library_exports_every_declared_symbol():
   assert lib.aqtx_version() == 1
 
 
+def test_plans_end_where_they_did_before():
+  """A plan carries no size of its own, so a caller built against an earlier header of this version has plans of that
+  header's length: what is new comes as an entry point, not as a field behind the last one."""
+  sizes = dict(QuantPlan=184, ScalePlan=96, GemmPlan=176, GroupedGemmPlan=88, DecodePlan=64, Im2colPlan=88, FpRoundPlan=48)
+  for name, size in sizes.items():
+    assert ctypes.sizeof(getattr(L, name)) == size, name
+
+
+def test_nothing_behind_a_plan_is_read():
+  """A plan in memory whose next bytes are somebody else's: a NULL q is refused whatever they hold."""
+  plan = _qplan()
+  for fill in (0x00, 0x01, 0xFF):
+    memory = (ctypes.c_uint8 * (184 + 64))(*([fill] * (184 + 64)))
+    ctypes.memmove(memory, ctypes.byref(plan), 184)
+    rc = L.lib().aqtx_quantize(ctypes.cast(memory, ctypes.POINTER(L.QuantPlan)), FAKE, None, None, FAKE, None, 0, None)
+    assert 'NULL buffer' in _err(rc), fill
+
+
 def _err(status):
   assert status != 0
   return L.lib().aqtx_last_error().decode()
