@@ -278,16 +278,33 @@ FP8_ACCUMULATE = L.ACC_F32 if os.environ.get('AQTX_FP8_ACCUMULATE', '').lower() 
 
 def _pads_rows(a: torch.Tensor, b: torch.Tensor, fp8: bool) -> bool:
   """Whether gemm() copies A [batch, m, k] and B [batch, n, k] to rows the MFMA kernels can load: what they cannot load is
-  k, strides or addresses that are no multiples of 16.  The kernel with one thread per output element keeps what is
-  smaller than a second launch (128 x 128 x 129: 8 us copied against 12 in int8, 10 against 36 in fp8; 64 x 64 x 33: 8
-  against 5 in int8; 16 x 16 x 17: 8 against 7 in fp8), empty operands, and a k with which the MFMA kernels' 32-bit
-  tile offsets would overflow."""
-  k = a.shape[2]
+  k, strides or addresses that are no multiples of 16.  The kernel with one thread per output element, 256 columns a block,
+  keeps empty operands, a k with which the MFMA kernels' 32-bit tile offsets would overflow, and what it does in less."""
+  batch, m, k = a.shape
+  if not (k | a.stride(1) | b.stride(1) | a.stride(0) | b.stride(0) | a.data_ptr() | b.data_ptr()) % 16:
+    return False
+  n = b.shape[1]
   if not (a.element_size() == b.element_size() == 1 and 0 < k < 2 ** 22 and a.numel() and b.numel()):
     return False
-  if k <= (16 if fp8 else 64) and a.shape[1] * b.shape[1] <= 4096:
-    return False
-  return bool((k | a.stride(1) | b.stride(1) | a.stride(0) | b.stride(0) | a.data_ptr() | b.data_ptr()) % 16)
+  if m > 65535:  # more rows than the kernel with one thread per element takes
+    return True
+  # The two launches take 7 us (8 in fp8) where nothing else does.  One thread an element takes 3 us and 0.06 a k (0.22 in
+  # fp8) on one block a CU, and more the more waves there are.  Copied / one thread an element, us:
+  #   int8  64 x 64 x 65 7.0 / 7.2, 500 x 64 x 63 8.0 / 7.1, 300 x 1 x 64 x 65 10.4 / 7.2, 300 x 4 x 4 x 70 9.8 / 7.3, 32 x 33 x 33 x 33 7.7 / 5.1
+  #         64 x 1000 x 63 8.1 / 7.2; 129 x 257 x 33 7.4 / 6.5, x 63 8.0 / 10.2; 129 x 1000 x 23 7.5 / 5.5, x 33 7.5 / 8.7
+  #         500 x 257 x 20 7.5 / 6.3, x 33 7.5 / 10.9; 500 x 1000 x 12 7.8 / 6.5, x 17 7.5 / 8.4; 35000 x 8 x 9 10.1 / 18.7
+  #   fp8   16 x 16 x 20 7.6 / 7.3, x 33 7.5 / 10.2; 500 x 257 x 17 8.4 / 8.3, x 20 8.4 / 9.2; 500 x 1000 x 7 8.7 / 6.9,
+  #         x 17 8.6 / 11.4; 300 x 16 x 16 x 17 9.5 / 13.0
+  blocks, waves = batch * m * -(-n // 256), batch * m * -(-n // 64)
+  if fp8:
+    most = 20 if waves <= 1000 else 17 if waves <= 3000 else 8 if waves <= 8000 else 0
+  elif n <= 64 and blocks <= 1200:
+    most = 76 if blocks <= 600 or n <= 16 else 45
+  elif blocks <= 256:
+    most = 64
+  else:
+    most = 40 if waves <= 1000 else 23 if waves <= 2100 else 20 if waves <= 5000 else 12 if waves <= 8000 else 0
+  return k > most
 
 
 def _pad_rows(a: torch.Tensor, b: torch.Tensor):
@@ -378,8 +395,7 @@ def gemm(
     a, b = _pad_rows(a, b)
     k, ldb, stride_b = a.shape[2], b.stride(1), b.stride(0)
     if fp8:
-      # what such operands always had: float32 sums of whole products (relative error against 64 bits, e4m3: 8.2e-9 at
-      # k = 129 and 7.8e-8 at 4095, one thread per element 8.6e-9 and 7.9e-8)
+      # what such operands always had: float32 sums of whole products
       accumulate = L.ACC_F32
   alloc = torch.zeros if group_offsets is not None and group_sizes is None else torch.empty
   c = alloc((batch, m, n), dtype=_AQTX_TO_TORCH[out_dt], device=a.device)
