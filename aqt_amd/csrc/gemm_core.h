@@ -152,7 +152,7 @@ struct GemmArgs {
   int p2_bf16;    // the second product is rounded to bf16
   int col_first;  // scale order
   // Ragged batches: entry b multiplies rows [group_offsets[b], group_offsets[b+1]) of one flat
-  // A with B[b] into the same rows of one flat C (m is then an upper bound of a group's rows).
+  // A with B[b] into the same rows of one flat C: offsets that ascend, m rows in all (gemm_grid counts on both).
   const int32_t* group_offsets;
   int groups;       // ragged: entries of the batch (the grid is one row of tiles_m + groups tile rows)
   int a_even_odd8;  // packed int4 B only: A's bytes of every 8 k are stored as k 0,2,4,6,1,3,5,7

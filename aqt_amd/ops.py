@@ -118,7 +118,7 @@ def _quantize_workspace(nbytes: int, device) -> torch.Tensor:
   key = (device.index, _raw_stream(device.index))
   ws = _QUANT_WS.get(key)
   if ws is None or ws.numel() < 2 * nbytes:
-    # with room for the arrival counts of the abs-max blocks (at most one per scale)
+    # twice what the scales need: room for the arrival counts of the abs-max blocks (aqtx_quant_plan.workspace_zeroed)
     ws = torch.zeros(max(2 * nbytes, 1 << 20), dtype=torch.uint8, device=device)
     _QUANT_WS[key] = ws
   return ws
@@ -436,6 +436,15 @@ def gemm(
     L.check(fn(ctypes.byref(plan), _ptr(a), _ptr(b), _ptr(row_scale), _ptr(col_scale), _ptr(c),
                _ptr(acc), _stream()))
   return (c, acc) if want_acc else c
+
+
+def ragged_offsets(group_sizes, m: int, device) -> torch.Tensor:
+  """[0, s0, s0+s1, ...] as gemm(group_offsets=...) takes them: int32 on the device, clamped to the m rows there are, computed
+  there when the sizes live there (no host round trip).  gemm(group_sizes=...) makes them in its own first launch; these serve
+  several contractions over the same groups."""
+  offs = torch.zeros(len(group_sizes) + 1, dtype=torch.int32, device=device)
+  offs[1:] = torch.cumsum(ragged_sizes(group_sizes, device), 0)
+  return torch.clamp(offs, max=m)
 
 
 def ragged_sizes(group_sizes, device) -> torch.Tensor:

@@ -133,3 +133,29 @@ def test_ragged_gemm_prepares_offsets_and_zeros_from_the_sizes(gpu, groups, left
     got = ops.gemm(a, b, row_scale=ones, col_scale=cs, out_dtype=torch.bfloat16, group_sizes=dev_sizes)
     want = ops.gemm(a, b, row_scale=ones, col_scale=cs.expand(groups, n).contiguous(), out_dtype=torch.bfloat16, group_offsets=offs)
     assert torch.equal(got, want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('groups', [63, 64, 65, 130, 200])
+def test_ragged_gemm_of_many_groups_against_integer_reference(gpu, groups):
+  """Groups on both sides of the 64 a wave looks up at a time, some of several 256-row tiles, some empty, n of two tiles:
+  every group meets its own B.  Sizes and offsets made on the host, on the device and by the contraction itself."""
+  from aqt_amd import ops
+  rng = np.random.default_rng(groups)
+  sizes = rng.integers(0, 30, groups) * rng.integers(0, 2, groups)
+  for g, rows in ((2, 600), (61, 257), (62, 512), (64, 300), (65, 1), (groups - 1, 513)):
+    if g < groups:
+      sizes[g] = rows
+  m, k, n = int(sizes.sum()) + 7, 32, 300
+  a = rng.integers(-127, 128, (m, k)).astype(np.int8)
+  b = rng.integers(-127, 128, (groups, n, k)).astype(np.int8)
+  want, at = np.zeros((m, n)), 0
+  for g, rows in enumerate(sizes):
+    want[at:at + rows] = a[at:at + rows].astype(np.float64) @ b[g].astype(np.float64).T
+    at += rows
+  ta, tb = torch.from_numpy(a).to(gpu)[None], torch.from_numpy(b).to(gpu)
+  on_device = torch.from_numpy(sizes.astype(np.int32)).to(gpu)
+  for kw in (dict(group_sizes=ops.ragged_sizes(sizes.tolist(), gpu)), dict(group_offsets=ops.ragged_offsets(sizes.tolist(), m, gpu)),
+             dict(group_offsets=ops.ragged_offsets(on_device, m, gpu))):
+    out = ops.gemm(ta, tb, row_scale=None, col_scale=None, out_dtype=torch.int32, **kw)[0]
+    np.testing.assert_array_equal(out.cpu().numpy(), want)
