@@ -248,9 +248,11 @@ static int quantize_impl(const aqtx_quant_plan* p, const void* x, const float* p
       a.G = p->rows; a.ngroups = 1;
       a.ssb = p->reduce == AQTX_REDUCE_ALL ? 1 : 0; a.ssg = 0; a.ssc = 0;
     }
-    // Room behind the abs-max words of a kept workspace (zero like them): the arrival counts of the abs-max blocks, one
-    // column group of its blocks, or one per batch entry
-    const int64_t groups = p->reduce == AQTX_REDUCE_ROWS ? p->batch * a.ngroups * absmax_col_groups(p->cols) : p->batch;
+    // Room behind the abs-max words of a kept workspace (zero like them): the arrival counts of the abs-max blocks, one per
+    // set of scales that they share: a column group of its blocks, a batch entry, or the whole batch
+    const int64_t groups = p->reduce == AQTX_REDUCE_ROWS  ? p->batch * a.ngroups * absmax_col_groups(p->cols)
+                           : p->reduce == AQTX_REDUCE_ALL ? p->batch
+                                                          : 1;
     if (p->workspace_zeroed && (int64_t)(workspace_bytes / 8) >= nscales + groups) a.ws_arrived = a.ws_absmax + (workspace_bytes / 8) - groups;
     const int64_t grid_y = p->reduce != AQTX_REDUCE_ROWS
                                ? (p->rows + kTileR - 1) / kTileR

@@ -1264,8 +1264,9 @@ int launch_tiles(const QArgs& a, int reduce, int partitionable, int64_t nscales,
     if (reduce == AQTX_REDUCE_ALL || reduce == AQTX_REDUCE_ALL_BATCH) {
       // Every block ends in two atomics (its maximum and its arrival).  Atomics on one address take turns (about 10 ns
       // each, measured), and so do those on the neighbouring words of the batch entries, which share a cache line: 32
-      // entries x 98 blocks took 31 us for 26 MB.  So the launch as a whole gets at most one block per 96 KiB of input
-      // (the time to stream that much), and no more than two of them, 16 waves each, on a CU.
+      // entries x 98 blocks took 31 us for 26 MB.  So the launch as a whole aims at one block per 96 KiB of input (the
+      // time to stream that much), but at least 64 where there are values for them (small tensors are bound by latency)
+      // and at most 512, two of 16 waves on each CU; a batch of more entries has one block for each.
       int64_t nblk = (a.rows * a.cols + kAbsThreads * 8 - 1) / (kAbsThreads * 8);
       const int64_t total_bytes = a.batch * a.rows * a.cols * (int64_t)sizeof(TIn);
       int64_t cap_total = total_bytes / (96 << 10);

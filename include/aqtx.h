@@ -95,9 +95,11 @@ typedef struct aqtx_quant_plan {
                             (written for AQTX_BF16 only; NULL or F32: `scale` is all there is)   */
   int32_t workspace_zeroed; /* 1: the caller keeps one workspace across calls on one stream, passes its
                             whole size as workspace_bytes, and its first half is zero on entry;
-                            aqtx_quantize returns it zeroed and skips its own clearing launch.  Twice
-                            aqtx_quantize_workspace_bytes or more spares another launch: the room in the
-                            first half holds counts with which the last abs-max block computes the scales */
+                            aqtx_quantize returns it zeroed and skips its own clearing launch.  With twice
+                            aqtx_quantize_workspace_bytes or more the room in the first half holds counts
+                            with which the last abs-max block computes the scales, where that is faster than
+                            a launch of its own: one scale per tensor or batch entry always, scales per
+                            column up to some hundred blocks of 64 rows x 512 columns, from 8 columns on  */
   const uint32_t* key_device; /* optional DEVICE pointer to the two key words; when not NULL the kernels
                             read the key there and `key` above is ignored (a key that is a traced
                             array under XLA, or one updated on the device between HIP graph replays) */

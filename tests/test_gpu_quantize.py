@@ -440,6 +440,24 @@ def test_scales_from_the_last_block_equal_those_of_their_own_launch(gpu, reduce,
   assert torch.equal(results[0][1], (want / 127.5).to(torch.bfloat16).float())
 
 
+@pytest.mark.parametrize('reduce,shape,scales', [(L.REDUCE_ALL_BATCH, (3, 300, 70), 1), (L.REDUCE_ALL, (3, 300, 70), 3),
+                                                 (L.REDUCE_ROWS, (2, 300, 70), 140), (L.REDUCE_ROWS, (2, 64, 9), 18)])
+def test_a_workspace_of_twice_the_bytes_holds_the_counts(gpu, reduce, shape, scales):
+  """The smallest workspace with room for the arrival counts: nothing beside it is touched, its first half stays zero."""
+  x = U.to_dev(U.rand(shape, 'bf16', seed=5, outliers=True), 'bf16', gpu)
+  kw = dict(reduce=reduce, out_dtype=L.I8, quant_bound=127.5, clip_bound=127.0)
+  want = ops.quantize(x, **kw)
+  buf = torch.full((16 * scales + 64,), 0x5A, dtype=torch.uint8, device=gpu)
+  ws = buf[:16 * scales]
+  ws[:8 * scales] = 0
+  with pytest.MonkeyPatch.context() as mp:
+    mp.setattr(ops, '_quantize_workspace', lambda nbytes, device: ws if nbytes == 8 * scales else None)
+    for _ in range(3):
+      got = ops.quantize(x, **kw)
+      assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+      assert not bool(ws[:8 * scales].any()) and bool((buf[16 * scales:] == 0x5A).all())
+
+
 @pytest.mark.parametrize('rows,cols', [(8128, 512), (8192, 512), (8193, 1024), (16384, 1024), (16385, 1024)])
 @pytest.mark.parametrize('dt,prescaled', [('bf16', False), ('bf16', True), ('f32', False), ('i8', False)])
 def test_column_scales_on_both_sides_of_the_fold(gpu, dt, prescaled, rows, cols):
