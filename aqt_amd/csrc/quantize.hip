@@ -164,16 +164,17 @@ extern "C" size_t aqtx_quantize_workspace_bytes(const aqtx_quant_plan* p) {
   return (size_t)scale_count(p) * 8;
 }
 
-// scale_only: q is neither read nor written (aqtx_calibrate).
+// scale_only: q is neither read nor written (aqtx_calibrate).  given_bf16: the given scales (aqtx_quantize_given).
 static int quantize_impl(const aqtx_quant_plan* p, const void* x, const float* prescale, void* q, float* scale, bool scale_only,
-                         void* workspace, size_t workspace_bytes, void* stream) {
+                         const uint16_t* given_bf16, void* workspace, size_t workspace_bytes, void* stream) {
   if (int rc = validate(p)) return rc;
   aqtx_quant_plan alt;
   if (long_rows_as_batches(p, &alt))
-    return quantize_impl(&alt, x, prescale, q, scale, scale_only, workspace, workspace_bytes, stream);
+    return quantize_impl(&alt, x, prescale, q, scale, scale_only, given_bf16, workspace, workspace_bytes, stream);
   const int64_t total = p->batch * p->rows * p->cols;
   if (total == 0) return 0;
-  AQTX_REQUIRE(x != nullptr && (q != nullptr || scale_only) && scale != nullptr, "aqtx_quantize: NULL buffer");
+  AQTX_REQUIRE(x != nullptr && (q != nullptr || scale_only) && (scale != nullptr || given_bf16 != nullptr),
+               "aqtx_quantize: NULL buffer");
   AQTX_REQUIRE(!scale_only || (p->noise == AQTX_NOISE_NONE && !p->scale_given && p->other_axis_absmax == nullptr),
                "aqtx_calibrate (scale_only) goes without noise, a given scale and other_axis_absmax");
   AQTX_REQUIRE((p->prescale == AQTX_PRESCALE_NONE) == (prescale == nullptr),
@@ -195,6 +196,7 @@ static int quantize_impl(const aqtx_quant_plan* p, const void* x, const float* p
   a.scale_bf16 = (p->scale_typed != nullptr && p->scale_dtype == AQTX_BF16 && !p->scale_given)
                      ? reinterpret_cast<uint16_t*>(p->scale_typed) : nullptr;
   a.scale_only = scale_only;
+  a.given_bf16 = given_bf16;
   a.batch = p->batch; a.rows = p->rows; a.cols = p->cols;
   a.nsb = p->noise_stride_batch; a.nsr = p->noise_stride_row; a.nsc = p->noise_stride_col;
   a.quant_bound = p->quant_bound; a.clip_bound = p->clip_bound;
@@ -271,13 +273,25 @@ extern "C" int aqtx_quantize(const aqtx_quant_plan* p, const void* x, const floa
                              void* q, float* scale, void* workspace, size_t workspace_bytes,
                              void* stream) {
   clear_error();
-  return quantize_impl(p, x, prescale, q, scale, false, workspace, workspace_bytes, stream);
+  return quantize_impl(p, x, prescale, q, scale, false, nullptr, workspace, workspace_bytes, stream);
+}
+
+extern "C" int aqtx_quantize_given(const aqtx_quant_plan* p, const void* x, const float* prescale, void* q,
+                                   const void* scale, void* workspace, size_t workspace_bytes, void* stream) {
+  clear_error();
+  AQTX_REQUIRE(p != nullptr && p->scale_given, "aqtx_quantize_given: plan is NULL or has no scale_given");
+  if (p->scale_dtype != AQTX_BF16)
+    return quantize_impl(p, x, prescale, q, reinterpret_cast<float*>(const_cast<void*>(scale)), false, nullptr, workspace,
+                         workspace_bytes, stream);
+  AQTX_REQUIRE(((uintptr_t)scale % 2) == 0, "aqtx_quantize_given: scale is not element aligned");
+  return quantize_impl(p, x, prescale, q, nullptr, false, reinterpret_cast<const uint16_t*>(scale), workspace, workspace_bytes,
+                       stream);
 }
 
 extern "C" int aqtx_calibrate(const aqtx_quant_plan* p, const void* x, const float* prescale, float* scale, void* workspace,
                               size_t workspace_bytes, void* stream) {
   clear_error();
-  return quantize_impl(p, x, prescale, nullptr, scale, true, workspace, workspace_bytes, stream);
+  return quantize_impl(p, x, prescale, nullptr, scale, true, nullptr, workspace, workspace_bytes, stream);
 }
 
 extern "C" int aqtx_dequantize(const aqtx_quant_plan* p, const void* q, const float* scale,

@@ -54,6 +54,7 @@ struct QArgs {
   int cbf;  // compute dtype is bf16
   int sbf;  // scale dtype is bf16
   int scale_given;
+  const uint16_t* given_bf16;  // given scales as bf16 elements, read where they lie (NULL: in `scale`)
   int ws_zeroed;  // the abs-max words of the workspace are zero on entry
   int scale_only; // the scales are all that is asked for (a calibration on its own): nothing reads or writes q
   int even_odd8;  // rows kernel: bytes of each group of 8 outputs stored as elements 0,2,4,6,1,3,5,7
@@ -102,6 +103,11 @@ __device__ __forceinline__ QArgs with_device_key(const QArgs& in) {
 __device__ __forceinline__ void store_scale(const QArgs& a, int64_t i, float v) {
   a.scale[i] = v;
   if (a.scale_bf16 != nullptr) a.scale_bf16[i] = (uint16_t)(__float_as_uint(v) >> 16);
+}
+
+// A scale the caller gives.
+__device__ __forceinline__ float given_scale(const QArgs& a, int64_t i) {
+  return a.given_bf16 != nullptr ? __uint_as_float((uint32_t)a.given_bf16[i] << 16) : a.scale[i];
 }
 
 // ---- typed vector loads ------------------------------------------------------
@@ -515,7 +521,7 @@ void quant_rows_kernel(const QArgs a_in) {
       amax = nanmax(amax, nanmax(__uint_as_float(amax_packed << 16), __uint_as_float(amax_packed & 0xFFFF0000u)));
     amax = segment_max<LANES>(amax, smem[s]);
     if (a.scale_given) {
-      scale[s] = active ? a.scale[seg] : 1.0f;
+      scale[s] = active ? given_scale(a, seg) : 1.0f;
       inv[s] = inv_of_scale(scale[s], a);
     } else {
       spec_scale_from_absmax<SPEC>(amax, a, scale[s], inv[s]);
@@ -608,7 +614,7 @@ __global__ __launch_bounds__(256) void quant_rows_generic_kernel(const QArgs a_i
   amax = segment_max<64>(amax, nullptr);
   float scale, inv;
   if (a.scale_given) {
-    scale = a.scale[seg];
+    scale = given_scale(a, seg);
     inv = inv_of_scale(scale, a);
   } else {
     scale_from_absmax(amax, a, scale, inv);
@@ -849,7 +855,7 @@ __global__ void finalize_scales_kernel(const QArgs a, int64_t n) {
   if (i >= n) return;
   float scale, inv;
   if (a.scale_given) {
-    scale = a.scale[i];
+    scale = given_scale(a, i);
     inv = inv_of_scale(scale, a);
   } else {
     scale_from_absmax(__uint_as_float(a.ws_absmax[i]), a, scale, inv);
@@ -961,7 +967,7 @@ __global__ __launch_bounds__(256) void quant_tile_kernel(const QArgs a_in) {
 #pragma unroll
       for (int s = 0; s < NSET; ++s) {
         const int64_t c = c0[s] + tid;
-        inv_lds[s][tid] = c < a.cols ? inv_of_scale(a.scale[b * a.ssb + c * a.ssc], a) : 1.0f;
+        inv_lds[s][tid] = c < a.cols ? inv_of_scale(given_scale(a, b * a.ssb + c * a.ssc), a) : 1.0f;
       }
     }
     __syncthreads();

@@ -183,6 +183,7 @@ def quantize(
   `q.other_axis_absmax`: what a later quantization of q over that axis takes as `absmax_partials` instead of
   reading q for its abs-max (the backward pass re-quantizes the forward residuals that way).
   scale_only: calibration alone; q comes back as None.
+  `scale`, given scales: float32 holding values of scale_dtype, or elements of scale_dtype.
   """
   _require_gpu(x, prescale, scale)
   assert x.dim() == 3 and x.is_contiguous(), 'x must be a contiguous [batch, rows, cols] tensor'
@@ -230,7 +231,8 @@ def quantize(
       typed = torch.empty(sshape, dtype=torch.bfloat16, device=x.device)
       plan.scale_typed = typed.data_ptr()
   else:
-    assert scale.dtype == torch.float32 and scale.is_contiguous() and tuple(scale.shape) == sshape
+    assert (scale.dtype == torch.float32 or (scale.dtype == torch.bfloat16 and scale_dt == L.BF16)), scale.dtype
+    assert scale.is_contiguous() and tuple(scale.shape) == sshape
   fp8 = out_dtype in (L.E4M3, L.E5M2)
   qshape = (b, c, r) if transpose_out else (b, r, c)
   q = None if scale_only else torch.empty(qshape, dtype=torch.uint8 if fp8 else torch.int8, device=x.device)
@@ -256,7 +258,8 @@ def quantize(
     if scale_only:
       L.check(lib.aqtx_calibrate(ctypes.byref(plan), _ptr(x), _ptr(prescale), *tail))
     else:
-      L.check(lib.aqtx_quantize(ctypes.byref(plan), _ptr(x), _ptr(prescale), _ptr(q), *tail))
+      fn = lib.aqtx_quantize_given if scale.dtype == torch.bfloat16 else lib.aqtx_quantize
+      L.check(fn(ctypes.byref(plan), _ptr(x), _ptr(prescale), _ptr(q), *tail))
   except Exception:
     _QUANT_WS.clear()  # a failed launch sequence may have left abs-max words behind
     raise

@@ -197,8 +197,8 @@ class Quantizer:
     v = lowering.view_operand(x, [], rest, shared)
     per_tensor = s.numel() == 1
     sv = lowering.view_operand(s, [], rest, shared)
-    s32 = sv.mem.reshape(-1).float().contiguous()
-    s_in = s32.reshape(1) if per_tensor else s32.reshape(1, v.R, 1) if v.k_last else s32.reshape(1, 1, v.R)
+    flat = sv.mem.reshape(-1).contiguous()
+    s_in = flat.reshape(1) if per_tensor else flat.reshape(1, v.R, 1) if v.k_last else flat.reshape(1, 1, v.R)
     q, _ = lowering.quantize_view(
         v, spec=spec, compute_dtype=x.dtype, scale_dtype=s.dtype,
         key=None if self.context is None else self.context.key, per_tensor=per_tensor, scale=s_in)

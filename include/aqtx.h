@@ -144,6 +144,9 @@ int aqtx_quantize(const aqtx_quant_plan* plan, const void* x, const float* presc
  */
 int aqtx_calibrate(const aqtx_quant_plan* plan, const void* x, const float* prescale, float* scale, void* workspace,
                    size_t workspace_bytes, void* stream);
+/* aqtx_quantize with scale_given, the scales being elements of plan->scale_dtype (bf16 ones are read where they lie). */
+int aqtx_quantize_given(const aqtx_quant_plan* plan, const void* x, const float* prescale, void* q, const void* scale,
+                        void* workspace, size_t workspace_bytes, void* stream);
 
 /* Scratch bytes aqtx_quantize needs for `plan` (0 for single-pass plans). */
 size_t aqtx_quantize_workspace_bytes(const aqtx_quant_plan* plan);

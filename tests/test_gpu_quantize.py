@@ -440,6 +440,24 @@ def test_scales_from_the_last_block_equal_those_of_their_own_launch(gpu, reduce,
   assert torch.equal(results[0][1], (want / 127.5).to(torch.bfloat16).float())
 
 
+@pytest.mark.parametrize('reduce,shape,group', [
+    (L.REDUCE_COLS, (2, 5, 3000), 0), (L.REDUCE_COLS, (1, 9, 20), 4), (L.REDUCE_COLS, (1, 2, 20000), 0), (L.REDUCE_COLS, (1, 30, 96), 32),
+    (L.REDUCE_ROWS, (1, 300, 72), 0), (L.REDUCE_ROWS, (2, 256, 130), 64), (L.REDUCE_ALL, (2, 100, 64), 0), (L.REDUCE_ALL_BATCH, (2, 7, 9), 0),
+])
+@pytest.mark.parametrize('dt', ['bf16', 'i8', 'f32'])
+def test_scales_given_as_bf16_elements(gpu, dt, reduce, shape, group):
+  """Read where they lie, in every kernel that takes given scales: the same bytes as from a float32 copy of them."""
+  x = U.rand(shape, 'f32', seed=3, outliers=True)
+  x = torch.from_numpy(x * 20).to({'bf16': torch.bfloat16, 'i8': torch.int8, 'f32': torch.float32}[dt]).to(gpu)
+  kw = dict(reduce=reduce, group=group, out_dtype=L.I8, quant_bound=127.5, clip_bound=127.0, scale_dtype=torch.bfloat16,
+            compute_dtype=torch.float32 if dt == 'f32' else torch.bfloat16)
+  _, s = ops.quantize(x, **kw)
+  s = s * 0.5  # clipping, and no maximum of its own to fall back on
+  want, _ = ops.quantize(x, scale=s, **kw)
+  got, same = ops.quantize(x, scale=s.to(torch.bfloat16), **kw)
+  assert torch.equal(got, want) and same.dtype == torch.bfloat16
+
+
 @pytest.mark.parametrize('reduce,shape,scales', [(L.REDUCE_ALL_BATCH, (3, 300, 70), 1), (L.REDUCE_ALL, (3, 300, 70), 3),
                                                  (L.REDUCE_ROWS, (2, 300, 70), 140), (L.REDUCE_ROWS, (2, 64, 9), 18)])
 def test_a_workspace_of_twice_the_bytes_holds_the_counts(gpu, reduce, shape, scales):
