@@ -120,6 +120,8 @@ class FpRoundPlan(ctypes.Structure):
 FP_NEAREST, FP_NOISE_JAX_BITS, FP_NOISE_INDEX = 0, 1, 2
 
 SYMBOLS = {
+    'aqtx_conv_scales': (ctypes.c_int, [_vp, ctypes.c_int32, ctypes.c_int64, ctypes.c_int64, _vp, _vp, ctypes.c_int32,
+                                        ctypes.c_int64, _vp, _vp]),
     'aqtx_im2col_i8': (ctypes.c_int, [ctypes.POINTER(Im2colPlan), _vp, _vp, _vp]),
     'aqtx_conv_i8': (ctypes.c_int, [ctypes.POINTER(Im2colPlan), ctypes.POINTER(GemmPlan), _vp, _vp, _vp, _vp, _vp, _vp]),
     'aqtx_fp_round': (ctypes.c_int, [ctypes.POINTER(FpRoundPlan), _vp, _vp, ctypes.POINTER(ctypes.c_uint32), _vp]),

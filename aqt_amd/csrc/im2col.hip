@@ -52,10 +52,46 @@ __global__ __launch_bounds__(256) void im2col_kernel(const Im2colArgs a) {
   }
 }
 
+struct ConvScalesArgs {
+  const void *row, *col;
+  float *row_out, *col_out;
+  int64_t rows, positions, cols;
+  int row_bf16, col_bf16;
+};
+
+// Bound by its launch, which takes the place of a cast of each scale and of the copy that spreads one over the positions.
+__global__ __launch_bounds__(256) void conv_scales_kernel(const ConvScalesArgs a) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  auto at = [](const void* p, int bf16, int64_t j) {
+    return bf16 ? __uint_as_float((uint32_t)reinterpret_cast<const uint16_t*>(p)[j] << 16) : reinterpret_cast<const float*>(p)[j];
+  };
+  if (i < a.rows) a.row_out[i] = at(a.row, a.row_bf16, i / a.positions);
+  else if (i - a.rows < a.cols) a.col_out[i - a.rows] = at(a.col, a.col_bf16, i - a.rows);
+}
+
 }  // namespace
 }  // namespace aqtx
 
 using namespace aqtx;
+
+extern "C" int aqtx_conv_scales(const void* row, int32_t row_dtype, int64_t images, int64_t positions, float* row_out,
+                                const void* col, int32_t col_dtype, int64_t features, float* col_out, void* stream) {
+  clear_error();
+  AQTX_REQUIRE(is_float_dtype(row_dtype) && is_float_dtype(col_dtype), "aqtx_conv_scales: scales must be bf16 or f32");
+  AQTX_REQUIRE(images >= 0 && positions >= 0 && features >= 0 && images < (1ll << 31) && positions < (1ll << 31) &&
+                   features < (1ll << 31), "aqtx_conv_scales: extent outside 0..2^31-1");
+  ConvScalesArgs a{row, col, row_out, col_out, images * positions, positions, features, row_dtype == AQTX_BF16, col_dtype == AQTX_BF16};
+  const int64_t blocks = (a.rows + a.cols + 255) / 256;
+  if (blocks == 0) return 0;
+  AQTX_REQUIRE((a.rows == 0 || (row != nullptr && row_out != nullptr)) && (a.cols == 0 || (col != nullptr && col_out != nullptr)),
+               "aqtx_conv_scales: NULL buffer");
+  AQTX_REQUIRE(((uintptr_t)row % (a.row_bf16 ? 2 : 4)) == 0 && ((uintptr_t)col % (a.col_bf16 ? 2 : 4)) == 0 &&
+                   ((uintptr_t)row_out % 4) == 0 && ((uintptr_t)col_out % 4) == 0, "aqtx_conv_scales: buffers are not element aligned");
+  AQTX_REQUIRE(blocks < (1ll << 31), "aqtx_conv_scales: too many positions for one launch");
+  conv_scales_kernel<<<(unsigned)blocks, 256, 0, reinterpret_cast<hipStream_t>(stream)>>>(a);
+  AQTX_HIP_CHECK_LAUNCH("conv_scales_kernel");
+  return 0;
+}
 
 extern "C" int aqtx_im2col_i8(const aqtx_im2col_plan* p, const void* x, void* out, void* stream) {
   clear_error();

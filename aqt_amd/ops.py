@@ -734,6 +734,20 @@ def im2col_i8(x: torch.Tensor, kernel, strides, pads, dilation):
   return out, out_sizes
 
 
+def conv_scales(row: torch.Tensor, col: torch.Tensor, positions: int):
+  """The scales of images and of output features (one each, bf16 or float32) as the float32 vectors of conv_i8 and gemm:
+  [images * positions] and [features]."""
+  _require_gpu(row, col)
+  row, col = row.reshape(-1).contiguous(), col.reshape(-1).contiguous()
+  n, features = row.numel(), col.numel()
+  start = -(-features // 64) * 64  # both vectors at the boundaries the contractions load pieces from
+  out = torch.empty((start + n * positions,), dtype=torch.float32, device=row.device)
+  rows, cols = out[start:], out[:features]
+  L.check(L.lib().aqtx_conv_scales(_ptr(row), aqtx_dtype(row.dtype), n, positions, _ptr(rows), _ptr(col), aqtx_dtype(col.dtype),
+                                   features, _ptr(cols), _stream()))
+  return rows, cols
+
+
 def conv_i8_supported(x: torch.Tensor) -> bool:
   """Whether conv_i8 takes this input: features a multiple of 128, less than 2 GiB."""
   return x.shape[-1] > 0 and x.shape[-1] % 128 == 0 and x.numel() < 2 ** 31

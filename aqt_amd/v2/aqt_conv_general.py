@@ -118,11 +118,6 @@ def lax_conv_general_dilated(lhs, rhs, window_strides, padding, lhs_dilation=Non
   return out.reshape([n] + list(out_sizes) + [cout])
 
 
-def _scale_of_positions(scale, n: int, positions: int):
-  """The scale of each of n images at each of its output positions, float32 [n, positions]: cast and copied in one launch."""
-  return scale.reshape(n, 1).expand(n, positions).to(torch.float32, memory_format=torch.contiguous_format).contiguous()
-
-
 def _fused_int8_conv(lhs_qt, rhs_qt, out_dtype, window_strides, padding, lhs_dilation, rhs_dilation,
                      feature_group_count, batch_group_count, preferred_element_type):
   """int8 x int8 with one scale per batch element and one per output feature: the contraction
@@ -158,9 +153,9 @@ def _fused_int8_conv(lhs_qt, rhs_qt, out_dtype, window_strides, padding, lhs_dil
     positions = math.prod(out_sizes)
     if positions > 0:
       b = _conv_weight_matrix(rq, k, cout)
-      row_scale = _scale_of_positions(ls, n, positions).reshape(n * positions)
+      row_scale, col_scale = ops.conv_scales(ls, rs, positions)
       out, out_sizes = ops.conv_i8(lq, b, kernel, strides, pads, dilation, row_scale=row_scale,
-                                   col_scale=rs.reshape(cout).float().contiguous(), out_dtype=out_dtype,
+                                   col_scale=col_scale, out_dtype=out_dtype,
                                    row_scale_dtype=ls.dtype, col_scale_dtype=rs.dtype)
       return out.reshape([n] + list(out_sizes) + [cout])
   a, out_sizes = ops.im2col_i8(lq, kernel, strides, pads, dilation)
@@ -169,8 +164,8 @@ def _fused_int8_conv(lhs_qt, rhs_qt, out_dtype, window_strides, padding, lhs_dil
   if a.shape[0] * cout == 0 or k == 0:
     return None
   b = _conv_weight_matrix(rq, k, cout)
-  row_scale = _scale_of_positions(ls, n, positions).reshape(1, n * positions)
-  out = ops.gemm(a.contiguous()[None], b[None], row_scale=row_scale, col_scale=rs.reshape(1, cout).float().contiguous(),
+  row_scale, col_scale = ops.conv_scales(ls, rs, positions)
+  out = ops.gemm(a.contiguous()[None], b[None], row_scale=row_scale[None], col_scale=col_scale[None],
                  out_dtype=out_dtype, dequant_dtype=out_dtype, row_scale_dtype=ls.dtype, col_scale_dtype=rs.dtype,
                  a_dtype=L.I8, b_dtype=L.I8)[0]
   return out.reshape([n] + list(out_sizes) + [cout])

@@ -425,6 +425,14 @@ typedef struct aqtx_im2col_plan {
 int aqtx_im2col_i8(const aqtx_im2col_plan* plan, const void* x, void* out, void* stream);
 
 /*
+ * aqtx_conv_scales: the float32 scale vectors of a convolution's contraction from the quantized operands' scales, bf16
+ * or f32 elements: row_out[images * positions] holds row[image] at each of an image's output positions, col_out[features]
+ * col.  What the broadcasts of QTensor.dequant (aqt_tensor.py:161-200) are in the reference.
+ */
+int aqtx_conv_scales(const void* row, int32_t row_dtype, int64_t images, int64_t positions, float* row_out,
+                     const void* col, int32_t col_dtype, int64_t features, float* col_out, void* stream);
+
+/*
  * aqtx_conv_i8: the same convolution in one launch, the windows read in place instead of gathered:
  * C[images * positions][n] = dequant(windows(x) * B^T), i.e. aqtx_im2col_i8(window, x) followed by
  * aqtx_gemm_i8(plan, ., b, ...) without the [images * positions][taps * c] matrix in between (same bits).

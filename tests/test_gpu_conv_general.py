@@ -331,3 +331,15 @@ def test_scales_written_past_autograd_are_the_ones_used(gpu, cout):
   got, _ = quantizer.calculate_qvalue(w, qt)
   want = torch.clamp(torch.round((w * (1 / qt.scale[0]))), -127, 127).to(torch.int8)
   assert torch.equal(got.qvalue, want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('n,positions,features', [(1, 1, 1), (3, 49, 24), (32, 100, 128), (2, 1, 300), (5, 0, 7)])
+@pytest.mark.parametrize('rdt,cdt', [(torch.bfloat16, torch.bfloat16), (torch.float32, torch.bfloat16), (torch.bfloat16, torch.float32)])
+def test_conv_scales(gpu, rdt, cdt, n, positions, features):
+  from aqt_amd import ops
+  row = torch.rand((n, 1, 1, 1), device=gpu).to(rdt)
+  col = torch.rand((1, 1, 1, 2 * features), device=gpu).to(cdt)[..., ::2]  # not contiguous
+  rows, cols = ops.conv_scales(row, col, positions)
+  assert torch.equal(rows, row.float().reshape(n, 1).expand(n, positions).reshape(-1)) and torch.equal(cols, col.float().reshape(-1))
+  assert rows.data_ptr() % 16 == 0 and cols.data_ptr() % 16 == 0
