@@ -1272,7 +1272,9 @@ int launch_tiles(const QArgs& a, int reduce, int partitionable, int64_t nscales,
       // each, measured), and so do those on the neighbouring words of the batch entries, which share a cache line: 32
       // entries x 98 blocks took 31 us for 26 MB.  So the launch as a whole aims at one block per 96 KiB of input (the
       // time to stream that much), but at least 64 where there are values for them (small tensors are bound by latency)
-      // and at most 512, two of 16 waves on each CU; a batch of more entries has one block for each.
+      // and at most 512, two of 16 waves on each CU; a batch of more entries has one block for each.  (Calibrated and
+      // quantized, against blocks of 4 waves for 48 KiB each, 256 to 2048 of them, and a launch for the scales: bf16 64 x
+      // 64 9.6 and 10.3 us, 2048 x 2048 10.6 and 13.4, 8192 x 4096 33.7 and 45.4, 256 entries of 64 x 64 10.9 and 11.0.)
       int64_t nblk = (a.rows * a.cols + kAbsThreads * 8 - 1) / (kAbsThreads * 8);
       const int64_t total_bytes = a.batch * a.rows * a.cols * (int64_t)sizeof(TIn);
       int64_t cap_total = total_bytes / (96 << 10);
@@ -1285,14 +1287,18 @@ int launch_tiles(const QArgs& a, int reduce, int partitionable, int64_t nscales,
       AQTX_HIP_CHECK_LAUNCH("absmax_all_kernel");
     } else {
       const dim3 grid((unsigned)absmax_col_groups(a.cols), (unsigned)(a.ngroups * ((a.G + kAbsRowChunk - 1) / kAbsRowChunk)), (unsigned)a.batch);
-      // Folded up to two blocks of 16 waves a CU, one round of the chip, and float values without a prescale, which are
-      // bound by HBM bytes from there on, below one a CU (calibration and quantization, folded against not: bf16 128
-      // blocks 12.1 and 12.1 us, 256 15.7 and 14.8, 512 24.4 and 21.6, 640 28.5 and 24.1; float32 128 13.7 and 16.7,
-      // 256 19-22 and 21, 512 31.4 and 28.4; bf16 with a prescale 256 18.9 and 21.4, 512 27.3 and 28.4, 576 33.7 and
-      // 31.5; int8 256 16.3 and 17.4, 512 24.1 and 24.1, 640 28.6 and 25.9).
-      const int64_t blocks = (int64_t)grid.x * grid.y * grid.z;
-      folded = a.ws_arrived != nullptr && a.cols >= 8 &&
-               (sizeof(TIn) != 1 && a.ps_mode == AQTX_PRESCALE_NONE ? blocks < 256 : blocks <= 512);
+      // Folded up to two blocks of 16 waves a CU, one round of the chip, and small inputs up to four.  Float values without a
+      // prescale are bound by HBM bytes from 8 million on: there only where few blocks share a set of scales.  Calibration and
+      // quantization, folded / not, us:
+      //   bf16           8192 x 512 12.1 / 12.1, 2048 x 4096 15.7 / 14.8, 4096 x 4096 24.4 / 21.6 (groups of 64 rows 20.5 / 22.3),
+      //                  512 x 32768 21.3 / 21.7, 4096 x 5120 28.5 / 24.1
+      //   float32        8192 x 512 13.7 / 16.7, 256 x 64 x 64 11.7 / 14.5, 8192 x 1024 21.5 / 21.2, 513 x 16383 24.3 / 26.5,
+      //                  4096 x 4096 31.4 / 28.4
+      //   bf16 prescaled 2048 x 4096 18.9 / 21.4, 4096 x 4096 27.3 / 28.4, 4608 x 4096 33.7 / 31.5; 50000 x 64 27.1 / 31.0
+      //   int8           2048 x 4096 16.3 / 17.4, 4096 x 4096 24.1 / 24.1, 4096 x 5120 28.6 / 25.9; 50000 x 64 24.7 / 27.0
+      const int64_t blocks = (int64_t)grid.x * grid.y * grid.z, values = a.batch * a.rows * a.cols;
+      const bool bytes_bound = sizeof(TIn) != 1 && a.ps_mode == AQTX_PRESCALE_NONE && values >= (8 << 20) && a.G > 16 * kAbsRowChunk;
+      folded = a.ws_arrived != nullptr && a.cols >= 8 && !bytes_bound && blocks <= (values < (4 << 20) ? 1023 : 512);
       if (a.cols < 8) absmax_cols_kernel<TIn, 1, false><<<grid, 256, 0, st>>>(a);
       else if (folded) absmax_cols_kernel<TIn, 8, true><<<grid, 1024, 0, st>>>(a);
       else absmax_cols_kernel<TIn, 8, false><<<grid, 256, 0, st>>>(a);
