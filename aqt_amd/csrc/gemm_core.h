@@ -154,7 +154,7 @@ struct GemmArgs {
   // Ragged batches: entry b multiplies rows [group_offsets[b], group_offsets[b+1]) of one flat
   // A with B[b] into the same rows of one flat C: offsets that ascend, m rows in all (gemm_grid counts on both).
   const int32_t* group_offsets;
-  int groups;       // ragged: entries of the batch (the grid is one row of tiles_m + groups tile rows)
+  int groups;       // ragged: entries of the batch (gemm_grid)
   int a_even_odd8;  // packed int4 B only: A's bytes of every 8 k are stored as k 0,2,4,6,1,3,5,7
   // B in the fragment order of aqtx_tile_weight (batch 1): blocks of 16 rows, b_steps KiB each, a KiB holding
   // 64 bytes of each of the 16 rows (lane r + 16 c of the KiB = bytes 16 c .. 16 c + 15 of row r); rows past n
@@ -295,32 +295,69 @@ void gemm_kernel(const GemmArgs g_in) {
   int tm, tn;
   int64_t bz = blockIdx.y;
   if (g_in.group_offsets != nullptr) {
-    // The groups' tiles follow one another: a wave looks 64 groups up at a time for the one its id falls into, and the
-    // XCD-aware walk covers that group's tiles.  A grid of the largest possible group times the groups is mostly workgroups
-    // that leave at once, and each of those still waits for the LDS of a whole CU: 8192 rows in 8 groups x 4096 x 14336
-    // took 608 us that way, 552 this way; in 16 groups x 1024 x 7168 147 and 123; 700 rows in 16 x 1024 x 4096 39 and 25.
+    // The groups' tiles follow one another: a wave looks the one up that its id falls into, and the XCD-aware walk covers
+    // that group's tiles.  A grid of the largest possible group times the groups is mostly workgroups that leave at once, and
+    // each of those still waits for the LDS of a whole CU: 8192 rows in 8 groups x 4096 x 14336 took 608 us that way, 552 this
+    // way; in 16 groups x 1024 x 7168 147 and 123; 700 rows in 16 x 1024 x 4096 39 and 25.
     int id = (int)blockIdx.x, group = -1, group_tiles_m = 0;
-    for (int first = 0; first < g.groups; first += 64) {
-      int tiles = 0;
-      if (first + lane < g.groups) {
-        const int rows = g_in.group_offsets[first + lane + 1] - g_in.group_offsets[first + lane];
-        tiles = rows > 0 ? (rows + BM - 1) / BM * g.tiles_n : 0;
-      }
-      int sum = tiles;  // inclusive
+    auto inclusive = [&](int sum) {
 #pragma unroll
       for (int off = 1; off < 64; off <<= 1) {
         const int up = __shfl_up(sum, off, 64);
         if (lane >= off) sum += up;
       }
-      const uint64_t behind = __ballot(sum > id);
-      if (behind != 0) {
-        const int at = __builtin_ctzll(behind);
-        group = first + at;
-        id -= __shfl(sum - tiles, at, 64);
-        group_tiles_m = __shfl(tiles, at, 64) / g.tiles_n;
-        break;
+      return sum;
+    };
+    auto tile_rows_of = [&](int rows) { return rows > 0 ? (rows + BM - 1) / BM : 0; };
+    if (g.groups <= 128) {  // a group a lane
+      for (int first = 0; first < g.groups; first += 64) {
+        const int at = first + lane;
+        const int tile_rows = at < g.groups ? tile_rows_of(g_in.group_offsets[at + 1] - g_in.group_offsets[at]) : 0;
+        const int tiles = tile_rows * g.tiles_n, sum = inclusive(tiles);
+        const uint64_t behind = __ballot(sum > id);
+        if (behind != 0) {
+          const int of = __builtin_ctzll(behind);
+          group = first + of;
+          id -= __shfl(sum - tiles, of, 64);
+          group_tiles_m = __shfl(tile_rows, of, 64);
+          break;
+        }
+        id -= __shfl(sum, 63, 64);
       }
-      id -= __shfl(sum, 63, 64);
+    } else if (id < (int64_t)(g_in.group_offsets[g.groups] - g_in.group_offsets[0]) * g.tiles_n) {  // (no more tile rows than rows)
+      // Eight groups a lane, 512 at a time: 64 at a time are a chain of loads and sums for each workgroup, 20000 rows in
+      // 10000 groups x 32 x 64 1868 us (one workgroup per group and tile 1320, this way 1284), 500 in 2000 empty ones 221 (34; 9).
+      constexpr int kPer = 8;
+      for (int first = 0; first < g.groups; first += 64 * kPer) {
+        int off[kPer + 1], tile_rows[kPer], tiles = 0;
+#pragma unroll
+        for (int u = 0; u <= kPer; ++u) {
+          const int at = first + lane * kPer + u;
+          off[u] = g_in.group_offsets[at < g.groups ? at : g.groups];
+        }
+#pragma unroll
+        for (int u = 0; u < kPer; ++u) {
+          tile_rows[u] = tile_rows_of(off[u + 1] - off[u]);
+          tiles += tile_rows[u] * g.tiles_n;
+        }
+        const int sum = inclusive(tiles);
+        const uint64_t behind = __ballot(sum > id);
+        if (behind != 0) {
+          const int at = __builtin_ctzll(behind);
+          id -= __shfl(sum - tiles, at, 64);
+#pragma unroll
+          for (int u = 0; u < kPer; ++u) {
+            const int rows = __shfl(tile_rows[u], at, 64);
+            if (group < 0 && id < rows * g.tiles_n) {
+              group = first + at * kPer + u;
+              group_tiles_m = rows;
+            }
+            if (group < 0) id -= rows * g.tiles_n;
+          }
+          break;
+        }
+        id -= __shfl(sum, 63, 64);
+      }
     }
     if (group < 0) return;
     bz = __builtin_amdgcn_readfirstlane(group);
@@ -950,9 +987,12 @@ inline GemmArgs make_gemm_args(const aqtx_gemm_plan* p, const void* a, const voi
 }
 
 // Grid of the 256 x 256 kernel, a workgroup per tile.  Ragged: groups of m rows in all have at most that many tile rows
-// and one begun per group.
+// and one begun per group, and no more than rows.
 inline dim3 gemm_grid(const GemmArgs& g) {
-  if (g.group_offsets != nullptr) return dim3((unsigned)((int64_t)(g.tiles_m + g.groups) * g.tiles_n), 1);
+  if (g.group_offsets != nullptr) {
+    const int64_t tile_rows = (int64_t)g.tiles_m + g.groups;
+    return dim3((unsigned)((tile_rows < g.m ? tile_rows : g.m) * g.tiles_n), 1);
+  }
   return dim3((unsigned)(g.tiles_m * g.tiles_n), (unsigned)g.groups);
 }
 

@@ -8,34 +8,66 @@
 namespace aqtx {
 namespace {
 
+// Every block finds the covered rows itself.  Up to 128 groups: inclusive sums over one wave, 64 at a time.  More: eight sizes a thread, 2048
+// at a time (64 at a time are a chain of a load and seven sums for each 64, 16 us for 2000 groups).
+template <bool MANY>
 __global__ __launch_bounds__(256) void ragged_prepare_kernel(const int32_t* __restrict__ sizes, int64_t groups, int64_t m,
                                                              int32_t* __restrict__ offsets, uint16_t* __restrict__ c, int64_t row_halves) {
-  __shared__ int64_t covered;
-  if (threadIdx.x < 64) {  // one wave: inclusive sums of 64 sizes at a time; every block finds the covered rows itself
-    const int lane = (int)threadIdx.x;
+  constexpr int kPer = MANY ? 8 : 1, kWaves = MANY ? 4 : 1;
+  __shared__ int64_t wave_sum[kWaves], wave_most[kWaves];
+  const int lane = (int)threadIdx.x & 63, wave = (int)threadIdx.x >> 6;
+  if (MANY || wave == 0) {
     int64_t before = 0, most = 0;
-    if (blockIdx.x == 0 && lane == 0) offsets[0] = 0;
-    for (int64_t g0 = 0; g0 < groups; g0 += 64) {
-      int64_t s = g0 + lane < groups ? (int64_t)sizes[g0 + lane] : 0;
+    if (blockIdx.x == 0 && threadIdx.x == 0) offsets[0] = 0;
+    for (int64_t g0 = 0; g0 < groups; g0 += 64 * kWaves * kPer) {
+      const int64_t mine = g0 + (int64_t)threadIdx.x * kPer;
+      int32_t size[kPer];
+      int64_t sum = 0;
+#pragma unroll
+      for (int u = 0; u < kPer; ++u) size[u] = mine + u < groups ? sizes[mine + u] : 0;
+#pragma unroll
+      for (int u = 0; u < kPer; ++u) sum += size[u];
+      const int64_t own = sum;
 #pragma unroll
       for (int off = 1; off < 64; off <<= 1) {
-        const int64_t up = __shfl_up(s, off, 64);
-        if (lane >= off) s += up;
+        const int64_t up = __shfl_up(sum, off, 64);
+        if (lane >= off) sum += up;
       }
-      int64_t end = (int64_t)(int32_t)(before + s);
-      if (end > m) end = m;
-      if (blockIdx.x == 0 && g0 + lane < groups) offsets[g0 + lane + 1] = (int32_t)end;
-      if (end > most) most = end;
-      before += __shfl(s, 63, 64);
+      int64_t at = before + sum - own;
+      if constexpr (MANY) {
+        if (lane == 63) wave_sum[wave] = sum;
+        __syncthreads();
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) {
+          if (w < wave) at += wave_sum[w];
+          before += wave_sum[w];
+        }
+      } else {
+        before += __shfl(sum, 63, 64);
+      }
+#pragma unroll
+      for (int u = 0; u < kPer; ++u) {
+        at += size[u];
+        int64_t end = (int64_t)(int32_t)at;
+        if (end > m) end = m;
+        if (mine + u < groups) {
+          if (blockIdx.x == 0) offsets[mine + u + 1] = (int32_t)end;
+          if (end > most) most = end;
+        }
+      }
+      if constexpr (MANY) __syncthreads();  // the sums have been read
     }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) {
       const int64_t other = __shfl_xor(most, off, 64);
       most = other > most ? other : most;
     }
-    if (lane == 0) covered = most;
+    if (lane == 0) wave_most[wave] = most;
   }
   __syncthreads();
+  int64_t covered = 0;
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) covered = wave_most[w] > covered ? wave_most[w] : covered;
   const int64_t first = covered * row_halves, total = m * row_halves, stride = (int64_t)gridDim.x * 256;
   for (int64_t i = first + (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += stride) c[i] = 0;
 }
@@ -56,8 +88,9 @@ extern "C" int aqtx_ragged_prepare(const int32_t* sizes, int64_t groups, int64_t
                "aqtx_ragged_prepare: buffers are not element aligned");
   int64_t blocks = (m * (row_bytes / 2) + 256 * 64 - 1) / (256 * 64);
   blocks = blocks < 1 ? 1 : blocks > 1024 ? 1024 : blocks;
-  ragged_prepare_kernel<<<dim3((unsigned)blocks), 256, 0, reinterpret_cast<hipStream_t>(stream)>>>(
-      sizes, groups, m, offsets, reinterpret_cast<uint16_t*>(c), row_bytes / 2);
+  const auto kernel = groups <= 128 ? ragged_prepare_kernel<false> : ragged_prepare_kernel<true>;
+  kernel<<<dim3((unsigned)blocks), 256, 0, reinterpret_cast<hipStream_t>(stream)>>>(sizes, groups, m, offsets,
+                                                                                    reinterpret_cast<uint16_t*>(c), row_bytes / 2);
   AQTX_HIP_CHECK_LAUNCH("ragged_prepare_kernel");
   return 0;
 }

@@ -136,14 +136,14 @@ def test_ragged_gemm_prepares_offsets_and_zeros_from_the_sizes(gpu, groups, left
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize('groups', [63, 64, 65, 130, 200])
+@pytest.mark.parametrize('groups', [63, 64, 65, 128, 129, 200, 513, 1500, 2049])
 def test_ragged_gemm_of_many_groups_against_integer_reference(gpu, groups):
-  """Groups on both sides of the 64 a wave looks up at a time, some of several 256-row tiles, some empty, n of two tiles:
-  every group meets its own B.  Sizes and offsets made on the host, on the device and by the contraction itself."""
+  """Groups on both sides of the 64, 512 and 2048 looked up or summed at a time, some of several 256-row tiles, some empty, n
+  of two tiles: every group meets its own B.  Sizes and offsets made on the host, on the device and by the contraction itself."""
   from aqt_amd import ops
   rng = np.random.default_rng(groups)
-  sizes = rng.integers(0, 30, groups) * rng.integers(0, 2, groups)
-  for g, rows in ((2, 600), (61, 257), (62, 512), (64, 300), (65, 1), (groups - 1, 513)):
+  sizes = rng.integers(0, max(2, 3000 // groups), groups) * rng.integers(0, 2, groups)
+  for g, rows in ((2, 600), (61, 257), (62, 512), (64, 300), (65, 1), (511, 257), (512, 300), (groups - 1, 513)):
     if g < groups:
       sizes[g] = rows
   m, k, n = int(sizes.sum()) + 7, 32, 300
@@ -159,3 +159,21 @@ def test_ragged_gemm_of_many_groups_against_integer_reference(gpu, groups):
              dict(group_offsets=ops.ragged_offsets(on_device, m, gpu))):
     out = ops.gemm(ta, tb, row_scale=None, col_scale=None, out_dtype=torch.int32, **kw)[0]
     np.testing.assert_array_equal(out.cpu().numpy(), want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('m,groups', [(5, 2100), (1, 129), (300, 1000)])
+def test_ragged_gemm_of_more_groups_than_rows(gpu, m, groups):
+  from aqt_amd import ops
+  rng = np.random.default_rng(m)
+  sizes = np.zeros(groups, np.int64)
+  np.add.at(sizes, rng.integers(0, groups, m), 1)
+  a = rng.integers(-127, 128, (m, 16)).astype(np.int8)
+  b = rng.integers(-127, 128, (groups, 24, 16)).astype(np.int8)
+  owner = np.repeat(np.arange(groups), sizes)
+  want = np.einsum('mk,mnk->mn', a.astype(np.int64), b[owner].astype(np.int64))
+  ta, tb = torch.from_numpy(a).to(gpu)[None], torch.from_numpy(b).to(gpu)
+  out = ops.gemm(ta, tb, row_scale=None, col_scale=None, out_dtype=torch.int32, group_sizes=ops.ragged_sizes(sizes.tolist(), gpu))[0]
+  np.testing.assert_array_equal(out.cpu().numpy(), want)
+  empty = ops.gemm(ta, tb, row_scale=None, col_scale=None, out_dtype=torch.int32, group_sizes=ops.ragged_sizes([0] * groups, gpu))[0]
+  assert not bool(empty.any())
