@@ -667,6 +667,14 @@ __device__ __forceinline__ void finalize_merged(const QArgs& a, int64_t i) {
   a.ws_inv[i] = inv;
 }
 
+// Scale (output) and reciprocal scale (workspace) of index i from a maximum that nothing is merged with.
+__device__ __forceinline__ void finalize_alone(const QArgs& a, int64_t i, float m) {
+  float scale, inv;
+  scale_from_absmax(m, a, scale, inv);
+  store_scale(a, i, scale);
+  a.ws_inv[i] = inv;
+}
+
 // Column abs-max: block = WAVES waves x (64 lanes x VEC cols); the waves interleave
 // over the rows of one chunk, partial maxima meet in LDS and leave through one
 // atomic max per column (|x| >= 0, so the float bit pattern orders like a uint).
@@ -676,7 +684,7 @@ __device__ __forceinline__ void finalize_merged(const QArgs& a, int64_t i) {
 // which spares finalize_scales_kernel, 4 to 5 us mostly of gap: 512 to 2048 columns take 6-12 us instead of 9-14 and that
 // launch.  On a chip full of blocks both cost more than they give, as blocks wait at barriers and for the atomics' returns:
 // 8192 x 14336 with a prescale 61-88 us against 57 and the launch.  Chunks of 16 rows, for more blocks, take four times the
-// atomics (4096 x 2048 float32: 22 us against 12).
+// atomics (4096 x 2048 float32: 22 us against 12).  A group of one chunk has its scales from its block, with no atomics.
 template <typename TIn, int VEC, bool FOLD>
 __global__ __launch_bounds__(FOLD ? 1024 : 256) void absmax_cols_kernel(const QArgs a) {
   constexpr int WAVES = FOLD ? 16 : 4;
@@ -763,12 +771,14 @@ __global__ __launch_bounds__(FOLD ? 1024 : 256) void absmax_cols_kernel(const QA
       float mm = smem[0][i];
 #pragma unroll
       for (int w = 1; w < WAVES; ++w) mm = nanmax(mm, smem[w][i]);
-      uint32_t* word = a.ws_absmax + b * a.ssb + g * a.ssg + c * a.ssc;
-      if constexpr (FOLD) merge_absmax(word, mm);
-      else atomicMax(word, __float_as_uint(mm));
+      const int64_t index = b * a.ssb + g * a.ssg + c * a.ssc;
+      if (chunks_per_group == 1) finalize_alone(a, index, mm);
+      else if constexpr (FOLD) merge_absmax(a.ws_absmax + index, mm);
+      else atomicMax(a.ws_absmax + index, __float_as_uint(mm));
     }
   }
   if constexpr (FOLD) {
+    if (chunks_per_group == 1) return;
     if (!last_arrival(a.ws_arrived + (b * a.ngroups + g) * gridDim.x + blockIdx.x, (uint32_t)chunks_per_group, &last)) return;
     const int64_t end = (int64_t)(blockIdx.x + 1) * WIDTH;
     for (int64_t c = (int64_t)blockIdx.x * WIDTH + threadIdx.x; c < end && c < a.cols; c += 64 * WAVES)
@@ -776,11 +786,11 @@ __global__ __launch_bounds__(FOLD ? 1024 : 256) void absmax_cols_kernel(const QA
   }
 }
 
-// Whole-tensor abs-max per batch entry (one entry for the whole batch where the batch shares its scale).
-constexpr int kAbsThreads = 1024;
-template <typename TIn>
-__global__ __launch_bounds__(kAbsThreads) void absmax_all_kernel(const QArgs a) {
-  __shared__ float smem[kAbsThreads / 64];
+// Whole-tensor abs-max per batch entry (one entry for the whole batch where the batch shares its scale).  An entry of one
+// block has its scale from it, with no atomics.
+template <typename TIn, int THREADS>
+__global__ __launch_bounds__(THREADS) void absmax_all_kernel(const QArgs a) {
+  __shared__ float smem[THREADS / 64];
   __shared__ int last;
   const int64_t b = blockIdx.y;
   const int64_t n = a.rows * a.cols;
@@ -789,8 +799,8 @@ __global__ __launch_bounds__(kAbsThreads) void absmax_all_kernel(const QArgs a) 
   if (n >= 8 && (a.ps_mode == AQTX_PRESCALE_NONE || a.cols % 8 == 0)) {
     // 8 elements per lane and load (with a prescale: of one row); the last eight of the entry are met twice where their
     // number is no multiple of 8
-    const int64_t stride = (int64_t)gridDim.x * kAbsThreads * 8;
-    const int64_t j0 = ((int64_t)blockIdx.x * kAbsThreads + threadIdx.x) * 8;
+    const int64_t stride = (int64_t)gridDim.x * THREADS * 8;
+    const int64_t j0 = ((int64_t)blockIdx.x * THREADS + threadIdx.x) * 8;
     bool done = false;
     if constexpr (sizeof(TIn) == 2) {
       if (a.ps_mode == AQTX_PRESCALE_NONE) {
@@ -828,7 +838,7 @@ __global__ __launch_bounds__(kAbsThreads) void absmax_all_kernel(const QArgs a) 
       }
     }
   } else {
-    for (int64_t i = (int64_t)blockIdx.x * kAbsThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kAbsThreads) {
+    for (int64_t i = (int64_t)blockIdx.x * THREADS + threadIdx.x; i < n; i += (int64_t)gridDim.x * THREADS) {
       float v = Loader<TIn>::load1(xb + i);
       if (a.ps_mode == AQTX_PRESCALE_PER_ROW) v = apply_prescale(v, a.prescale[b * a.psb + i / a.cols], a);
       else if (a.ps_mode == AQTX_PRESCALE_PER_COL) v = apply_prescale(v, a.prescale[b * a.psb + i % a.cols], a);
@@ -841,11 +851,15 @@ __global__ __launch_bounds__(kAbsThreads) void absmax_all_kernel(const QArgs a) 
   __syncthreads();
   if (threadIdx.x == 0) {
 #pragma unroll
-    for (int w = 1; w < kAbsThreads / 64; ++w) m = nanmax(m, smem[w]);
-    merge_absmax(a.ws_absmax + b * a.ssb, m);
+    for (int w = 1; w < THREADS / 64; ++w) m = nanmax(m, smem[w]);
   }
-  if (a.ws_arrived == nullptr) return;
   const uint32_t blocks = a.ssb != 0 ? gridDim.x : gridDim.x * gridDim.y;
+  if (blocks == 1) {
+    if (threadIdx.x == 0) finalize_alone(a, b * a.ssb, m);
+    return;
+  }
+  if (threadIdx.x == 0) merge_absmax(a.ws_absmax + b * a.ssb, m);
+  if (a.ws_arrived == nullptr) return;
   if (last_arrival(a.ws_arrived + b * a.ssb, blocks, &last) && threadIdx.x == 0) finalize_merged(a, b * a.ssb);
 }
 
@@ -1275,15 +1289,24 @@ int launch_tiles(const QArgs& a, int reduce, int partitionable, int64_t nscales,
       // and at most 512, two of 16 waves on each CU; a batch of more entries has one block for each.  (Calibrated and
       // quantized, against blocks of 4 waves for 48 KiB each, 256 to 2048 of them, and a launch for the scales: bf16 64 x
       // 64 9.6 and 10.3 us, 2048 x 2048 10.6 and 13.4, 8192 x 4096 33.7 and 45.4, 256 entries of 64 x 64 10.9 and 11.0.)
-      int64_t nblk = (a.rows * a.cols + kAbsThreads * 8 - 1) / (kAbsThreads * 8);
-      const int64_t total_bytes = a.batch * a.rows * a.cols * (int64_t)sizeof(TIn);
+      QArgs whole = a;
+      if (reduce == AQTX_REDUCE_ALL_BATCH && a.ps_mode == AQTX_PRESCALE_NONE) {  // the entries follow one another
+        whole.rows = a.batch * a.rows;
+        whole.batch = 1;
+      }
+      const int64_t values = whole.rows * whole.cols;
+      int64_t nblk = (values + 1024 * 8 - 1) / (1024 * 8);
+      const int64_t total_bytes = whole.batch * values * (int64_t)sizeof(TIn);
       int64_t cap_total = total_bytes / (96 << 10);
       cap_total = cap_total < 64 ? 64 : cap_total > 512 ? 512 : cap_total;
-      const int64_t cap = a.batch >= cap_total ? 1 : cap_total / a.batch;
+      const int64_t cap = whole.batch >= cap_total ? 1 : cap_total / whole.batch;
       if (nblk > cap) nblk = cap;
       if (nblk < 1) nblk = 1;
-      folded = a.ws_arrived != nullptr;
-      absmax_all_kernel<TIn><<<dim3((unsigned)nblk, (unsigned)a.batch), kAbsThreads, 0, st>>>(a);
+      folded = a.ws_arrived != nullptr || (nblk == 1 && (whole.batch == 1 || a.ssb != 0));
+      const dim3 grid((unsigned)nblk, (unsigned)whole.batch);
+      // many small entries: blocks of 4 waves, more of which a CU holds at a time
+      if (whole.batch >= 512 && values <= 16384) absmax_all_kernel<TIn, 256><<<grid, 256, 0, st>>>(whole);
+      else absmax_all_kernel<TIn, 1024><<<grid, 1024, 0, st>>>(whole);
       AQTX_HIP_CHECK_LAUNCH("absmax_all_kernel");
     } else {
       const dim3 grid((unsigned)absmax_col_groups(a.cols), (unsigned)(a.ngroups * ((a.G + kAbsRowChunk - 1) / kAbsRowChunk)), (unsigned)a.batch);
@@ -1298,10 +1321,13 @@ int launch_tiles(const QArgs& a, int reduce, int partitionable, int64_t nscales,
       //   int8           2048 x 4096 16.3 / 17.4, 4096 x 4096 24.1 / 24.1, 4096 x 5120 28.6 / 25.9; 50000 x 64 24.7 / 27.0
       const int64_t blocks = (int64_t)grid.x * grid.y * grid.z, values = a.batch * a.rows * a.cols;
       const bool bytes_bound = sizeof(TIn) != 1 && a.ps_mode == AQTX_PRESCALE_NONE && values >= (8 << 20) && a.G > 16 * kAbsRowChunk;
-      folded = a.ws_arrived != nullptr && a.cols >= 8 && !bytes_bound && blocks <= (values < (4 << 20) ? 1023 : 512);
+      const bool alone = a.G <= kAbsRowChunk;  // (a block has all rows of its columns)
+      folded = a.cols >= 8 && (alone ? blocks <= 512
+                                     : a.ws_arrived != nullptr && !bytes_bound && blocks <= (values < (4 << 20) ? 1023 : 512));
       if (a.cols < 8) absmax_cols_kernel<TIn, 1, false><<<grid, 256, 0, st>>>(a);
       else if (folded) absmax_cols_kernel<TIn, 8, true><<<grid, 1024, 0, st>>>(a);
       else absmax_cols_kernel<TIn, 8, false><<<grid, 256, 0, st>>>(a);
+      folded |= alone;
       AQTX_HIP_CHECK_LAUNCH("absmax_cols_kernel");
     }
   }

@@ -476,6 +476,33 @@ def test_a_workspace_of_twice_the_bytes_holds_the_counts(gpu, reduce, shape, sca
       assert not bool(ws[:8 * scales].any()) and bool((buf[16 * scales:] == 0x5A).all())
 
 
+@pytest.mark.parametrize('reduce', [L.REDUCE_ROWS, L.REDUCE_ALL, L.REDUCE_ALL_BATCH])
+@pytest.mark.parametrize('shape', [(511, 7, 24), (512, 7, 24), (513, 64, 9), (600, 65, 16), (520, 130, 127), (3, 64, 1000), (1, 9, 5),
+                                   (2, 40, 3000)])
+@pytest.mark.parametrize('dt', ['bf16', 'f32'])
+def test_scales_of_many_small_entries(gpu, dt, shape, reduce):
+  """Entries and groups whose maximum one block finds, in blocks of 4 and of 16 waves, next to ones of several blocks; an
+  entry of zeros, one of the largest finite values, a NaN in another."""
+  x = torch.randn(shape, generator=torch.Generator().manual_seed(sum(shape)))
+  x[0] = 0.0
+  x[-1, -1, -1] = torch.finfo(torch.bfloat16).max
+  dtype = torch.bfloat16 if dt == 'bf16' else torch.float32
+  x = x.to(dtype).to(gpu)
+  axes = {L.REDUCE_ROWS: (1,), L.REDUCE_ALL: (1, 2), L.REDUCE_ALL_BATCH: (0, 1, 2)}[reduce]
+  for nan in (False, True):
+    if nan:
+      x[shape[0] // 2, 0, 1] = float('nan')
+    want = x.float().abs().amax(axes)
+    want = torch.where(want == 0, torch.ones_like(want), want) / 128.0
+    kw = dict(reduce=reduce, out_dtype=L.I8, quant_bound=128.0, clip_bound=127.0)
+    for _ in range(2):  # (the second call finds the workspace as the first has left it)
+      q, s = ops.quantize(x, **kw)
+      assert torch.equal(s.reshape(-1).nan_to_num(-1.0), want.to(dtype).float().reshape(-1).nan_to_num(-1.0))
+    if not nan:
+      given, _ = ops.quantize(x, scale=s, **kw)
+      assert torch.equal(q, given)
+
+
 @pytest.mark.parametrize('rows,cols', [(8128, 512), (8192, 512), (8193, 1024), (16384, 1024), (16385, 1024)])
 @pytest.mark.parametrize('dt,prescaled', [('bf16', False), ('bf16', True), ('f32', False), ('i8', False)])
 def test_column_scales_on_both_sides_of_the_fold(gpu, dt, prescaled, rows, cols):
