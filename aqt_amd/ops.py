@@ -291,14 +291,22 @@ def _pads_rows(a: torch.Tensor, b: torch.Tensor, fp8: bool) -> bool:
     return False
   if m > 65535:  # more rows than the kernel with one thread per element takes
     return True
-  # The two launches take 7 us (8 in fp8) where nothing else does.  One thread an element takes 3 us and 0.06 a k (0.22 in
-  # fp8) on one block a CU, and more the more waves there are.  Copied / one thread an element, us:
-  #   int8  64 x 64 x 65 7.0 / 7.2, 500 x 64 x 63 8.0 / 7.1, 300 x 1 x 64 x 65 10.4 / 7.2, 300 x 4 x 4 x 70 9.8 / 7.3, 32 x 33 x 33 x 33 7.7 / 5.1
-  #         64 x 1000 x 63 8.1 / 7.2; 129 x 257 x 33 7.4 / 6.5, x 63 8.0 / 10.2; 129 x 1000 x 23 7.5 / 5.5, x 33 7.5 / 8.7
-  #         500 x 257 x 20 7.5 / 6.3, x 33 7.5 / 10.9; 500 x 1000 x 12 7.8 / 6.5, x 17 7.5 / 8.4; 35000 x 8 x 9 10.1 / 18.7
+  # The two launches take 7 us (8 in fp8) where nothing else does, and 0.0065 a batch entry.  One thread an element takes 3 us
+  # and 0.06 a k (0.2 in fp8) on one block a CU, and more the more waves there are.  Copied / one thread an element, us:
+  #   int8  64 x 64 x 65 7.0 / 7.2, 500 x 64 x 63 8.0 / 7.1; 64 x 1000 x 63 8.1 / 7.2; 129 x 257 x 33 7.4 / 6.5, x 63 8.0 / 10.2
+  #         129 x 1000 x 23 7.5 / 5.5, x 33 7.5 / 8.7; 500 x 257 x 20 7.5 / 6.3, x 33 7.5 / 10.9; 500 x 1000 x 12 7.8 / 6.5, x 17
+  #         7.5 / 8.4; 35000 x 8 x 9 10.1 / 18.7
   #   fp8   16 x 16 x 20 7.6 / 7.3, x 33 7.5 / 10.2; 500 x 257 x 17 8.4 / 8.3, x 20 8.4 / 9.2; 500 x 1000 x 7 8.7 / 6.9,
-  #         x 17 8.6 / 11.4; 300 x 16 x 16 x 17 9.5 / 13.0
+  #         x 17 8.6 / 11.4
   blocks, waves = batch * m * -(-n // 256), batch * m * -(-n // 64)
+  if batch > 1:
+    # Entries: by what a block of that kernel costs, its dispatch or its share of the eight blocks a CU holds (fitted).  int8
+    # 300 x 1 x 64 x 65 10.4 / 7.2, 300 x 4 x 4 x 70 9.8 / 7.3, 32 x 33 x 33 x 33 7.7 / 5.1, 300 x 33 x 33 x 33 10.2 / 16.3, 5000 x 8
+    # x 8 x 20 39 / 27, 20000 x 4 x 4 x 100 137 / 243, 60000 x 1 x 1 x 33 394 / 49; fp8 300 x 16 x 16 x 17 9.5 / 13.0, 5000 x 3 x 3
+    # x 9 39 / 17, 5000 x 2 x 100 x 40 59 / 75, 20000 x 1 x 1 x 33 135 / 55.
+    columns = min(n, 256) / 64
+    a_block = max(5e-4, k * (1e-4 * max(1, columns) if fp8 else 2.7e-5 * max(1, 1.5 * columns)))
+    return 3 + (0.2 if fp8 else 0.055) * k + blocks * a_block > (8.4 if fp8 else 7.9) + 0.0065 * batch
   if fp8:
     most = 20 if waves <= 1000 else 17 if waves <= 3000 else 8 if waves <= 8000 else 0
   elif n <= 64 and blocks <= 1200:

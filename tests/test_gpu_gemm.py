@@ -625,7 +625,7 @@ def test_unaligned_operands_dequantized_in_another_dtype_than_written(gpu, m, n,
     # either side of the lines between one thread an element and the copy to padded rows, by k and by outputs
     (1, 40, 64, 76), (1, 40, 64, 77), (1, 40, 65, 63), (1, 40, 65, 65), (1, 601, 10, 41), (1, 257, 130, 40), (1, 257, 130, 41),
     (1, 1000, 300, 20), (1, 1001, 300, 20), (1, 1001, 300, 12), (3, 30, 70, 20), (3, 30, 70, 21), (1, 700, 257, 8), (1, 700, 257, 17),
-    (1, 8001, 3, 7), (1, 66000, 3, 5),
+    (1, 8001, 3, 7), (1, 66000, 3, 5), (300, 4, 4, 70), (300, 4, 4, 90), (2000, 8, 8, 20), (2000, 20, 20, 33),
 ])
 def test_unaligned_contractions_on_both_sides_of_the_padding_line(gpu, batch, m, n, k, kind):
   a, b = (np.random.default_rng(s).integers(-2, 3, size=(batch, r, k)) for s, r in ((1, m), (2, n)))
