@@ -7,12 +7,12 @@
 // own and the tiles are summed afterwards.  Here the per-group results never leave registers.
 //
 // The per-group rescale is 7 vector instructions per element and group (int->float, three
-// roundings to bf16, two multiplications, one addition) against one MFMA per 1024 elements and
-// 32 k: with groups of 128 the kernel is bound by the vector ALU, not by the matrix cores.  On
-// this device a wave issues one vector instruction every ~12 cycles however independent its
-// instructions are (measured: 2 waves per SIMD reach 2.7 ns per instruction and SIMD, 4 waves
-// 1.5 ns for add/mul/and and 2.3 ns for the conversions and shifts), so a kernel of this kind
-// wants 4 waves per SIMD, i.e. at most 128 registers per lane, more than it wants large tiles.
+// roundings to bf16, two multiplications, one addition), 4 with bf16 scales on both sides (Quad), against
+// one MFMA per 1024 elements and 32 k: with groups of 128 the kernel is bound by the vector ALU, not by
+// the matrix cores.  Measured, independent instructions: conversions, shifts, v_perm_b32 and everything with three
+// operands 1.75-1.8 ns per instruction and SIMD (one every 4 cycles) from two waves on, 2.1 with one; add, mul, and, xor
+// 1.05-1.1 among themselves, 1.6 mixed with the others.  An MFMA of 32 cycles takes 4 ns of the
+// vector ALU's time when it runs next to it, a v_mfma_f32_4x4x4_16b_bf16 2.3 (4 ns alone).
 //
 // Two tile kernels, both with 128-byte K stages double-buffered in LDS, the group scales of a stage
 // next to it in LDS (and gemm_grouped_rows_kernel, further down, for at most 64 rows of A):
@@ -101,6 +101,43 @@ struct Rescale {
   }
 };
 
+typedef short v4s __attribute__((ext_vector_type(4)));
+typedef float v4f __attribute__((ext_vector_type(4)));
+
+// EPI 0 with both products on the matrix cores: v_mfma_f32_4x4x4_16b_bf16 against a diagonal 4 x 4 matrix of scales
+// multiplies the four values a lane holds by four scales, each product alone in its sum, so exact (8 x 8 significant
+// bits) like the product the vector ALU would form, and it takes its operand packed, so that one conversion rounds
+// two values.  Left: 4 vector instructions per element and group instead of 7.  With the values as first operand the
+// result comes out transposed within every 4 lanes x 4 registers: the accumulators hold 4 rows of one column per lane,
+// the first product (row scales) turns that into 4 columns of one row, as the second (column scales) needs it.
+// Measured: 2048 x 8192 x 28672, packed b: 886 -> 833 us; 65 x 4096 x 4096 42.2 -> 38.5; 500 x 8192 x 2048 83.6 -> 76.
+// The running sum stays on the vector ALU: 1.5-10 % of the sums this instruction forms differ from float32 addition in
+// the last bit.  Tried and left out: the MFMAs of one half of the wave tile between the quarters of the other (903), and
+// waves of 64 x 64 with two of them per SIMD and the short MFMAs ahead of the long one (820, but 30-40 % behind where
+// the grid gives a CU one workgroup).
+struct Quad {
+  // Scales the products are exact for, no value becoming subnormal, infinite or NaN on the way (a sum with a
+  // neighbour's 0 * infinity would): bf16 values of 2^-60 .. 2^41.
+  static __device__ __forceinline__ bool scale_fits(float v) {
+    const uint32_t b = __builtin_bit_cast(uint32_t, v);
+    return ((b >> 23) & 255u) - 67u <= 100u && (b & 0xFFFFu) == 0;
+  }
+  static __device__ __forceinline__ v4s pack(const v4f& x) {
+    const bf16x2 lo = __builtin_convertvector(f32x2{x[0], x[1]}, bf16x2), hi = __builtin_convertvector(f32x2{x[2], x[3]}, bf16x2);
+    return __builtin_bit_cast(v4s, make_uint2(__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, hi)));
+  }
+  // acc: 4 rows (registers 4q ..) of column lane % 4; sum: 4 columns of row lane % 4
+  static __device__ __forceinline__ void add(const v16i& acc, v16f& sum, const int q, const v4s rs, const v4s cs) {
+    v4f f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) f[e] = (float)acc[4 * q + e];
+    f = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(pack(f), rs, v4f{0, 0, 0, 0}, 0, 0, 0);
+    f = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(cs, pack(f), v4f{0, 0, 0, 0}, 0, 0, 0);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) sum[4 * q + e] += round_wide<true>(f[e]);
+  }
+};
+
 // Writes registers 4q..4q+3 of a running-sum tile: four consecutive n of row mm.
 template <bool kOutBf16>
 __device__ __forceinline__ void store_out4(const GroupedArgs& g, const v16f& sum, int q, int64_t mm, int64_t nn, bool vec) {
@@ -169,22 +206,34 @@ struct ScaleFetch {
 // few loop-invariant registers plus an immediate, which this kernel needs more than it needs
 // the 12 % of LDS: it has 128 registers per lane.
 //
+// The padding holds the row's scale as the diagonal entry of its quad's matrix (kQuad): bf16 at place row % 4 of four,
+// the other three zero.
+//
 // A stage: eight MFMAs (four 32-byte k steps x two column tiles); the staging registers (stage
 // s + 1, requested during stage s - 1) go to LDS, into the buffer stage s - 1 left; the rescale of
 // the group just accumulated, with the global loads of stage s + 2 issued one per quarter of it
 // (issued in one burst, the loads of all waves queue up in the CU's address unit and the waves
 // stand still behind them); the next group's scales go to LDS; barrier.  The other three waves of
 // the SIMD fill the gaps each of these leaves.
-template <int EPI, bool PACKED>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4)))
-void gemm_grouped128_kernel(const GroupedArgs g) {
+struct Grouped128Lds {
+  static constexpr int kRow = BK + 16, kATile = GM * kRow, kBTile = grouped_cols(true) * kRow, kStage = kATile + kBTile;  // 36 KiB
+  // the small arrays first: every offset of the loop then fits the 16-bit immediate of an LDS instruction
+  __attribute__((aligned(16))) float srow[2][GM];
+  __attribute__((aligned(16))) float scol[2][grouped_cols(true)];
+  __attribute__((aligned(16))) uint8_t stage_mem[2 * kStage];
+  int odd_group[2];  // kQuad: the group of this buffer if one of its scales does not fit
+};
+
+// One tile.  kQuad: with the products of Quad; false, and nothing written, where a scale does not fit them.
+template <int EPI, bool PACKED, bool kQuad>
+__device__ __forceinline__ bool grouped128_tile(const GroupedArgs g, Grouped128Lds& lds) {
   using R = Rescale<EPI>;
   constexpr int GN = grouped_cols(true);
-  constexpr int kRow = BK + 16;
-  constexpr int kATile = GM * kRow, kBTile = GN * kRow, kStage = kATile + kBTile;  // 36 KiB
-  __shared__ __attribute__((aligned(1024))) uint8_t stage_mem[2 * kStage];
-  __shared__ __attribute__((aligned(16))) float srow[2][GM];
-  __shared__ __attribute__((aligned(16))) float scol[2][GN];
+  constexpr int kRow = Grouped128Lds::kRow, kATile = Grouped128Lds::kATile, kStage = Grouped128Lds::kStage;
+  uint8_t* const stage_mem = lds.stage_mem;
+  auto& srow = lds.srow;
+  auto& scol = lds.scol;
+  auto& odd_group = lds.odd_group;
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -229,11 +278,21 @@ void gemm_grouped128_kernel(const GroupedArgs g) {
     const int grp_c = grp < g.groups ? grp : g.groups - 1;
     if (sc_active) sc_reg = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc_s, sc_voff, grp_c * sc_step, 0));
   };
-  auto store_scales = [&](int grp, int buf) {
+  // kQuad: where this thread's scale goes in the padding of its operand row
+  const int sc_pad = (sc_row ? 0 : kATile) + sc_idx * kRow + BK + 2 * (sc_idx & 3);
+  auto store_scales = [&](int grp, auto buf_c) {
+    constexpr int BUF = decltype(buf_c)::value;
     asm volatile("" : "+v"(sc_reg));  // keeps the arithmetic on the loaded value down here
     const float v = (sc_inside && grp < g.groups) ? sc_reg * ((PACKED && !sc_row) ? 0.0625f : 1.0f) : 1.0f;
-    if (sc_row) srow[buf][sc_idx] = v;
-    else if (sc_active) scol[buf][sc_idx] = v;
+    if constexpr (kQuad) {
+      if (sc_active) {
+        *reinterpret_cast<uint16_t*>(stage_mem + BUF * kStage + sc_pad) = (uint16_t)(__builtin_bit_cast(uint32_t, v) >> 16);
+        if (!Quad::scale_fits(v)) odd_group[BUF] = grp;
+      }
+    } else {
+      if (sc_row) srow[BUF][sc_idx] = v;
+      else if (sc_active) scol[BUF][sc_idx] = v;
+    }
   };
 
   // ---- global -> registers -> LDS (rows past the operand read as zero) ----------------------
@@ -272,6 +331,8 @@ void gemm_grouped128_kernel(const GroupedArgs g) {
   const int a_off = (wm * 32 + lr) * kRow + lh * 16;
   const int b_off = kATile + (wn * 64 + lr) * kRow + lh * 16;
   const int rs_off = wm * 32 + lr, cs_off = wn * 64 + 4 * lh;
+  const int rs_pad = (wm * 32 + 4 * lh + (lane & 3)) * kRow + BK;  // kQuad: row scale of quad column lane % 4, quarter 0
+  const int cs_pad = kATile + (wn * 64 + lr) * kRow + BK;          // kQuad: column scale of quad row lane % 4
 
   v16i acc[2];
   v16f sum[2];
@@ -282,8 +343,15 @@ void gemm_grouped128_kernel(const GroupedArgs g) {
   const int nstages = g.groups;
   for (int j = 0; j < NL; ++j) load_one(j, 0);
   load_scales(0);
+  if constexpr (kQuad) {
+    // the padding of the 2 x 256 operand rows: zero but for the one half word that store_scales writes
+    static_assert(GM + GN == 256, "one row of each buffer per pair of threads");
+    *reinterpret_cast<uint2*>(stage_mem + (tid >> 8) * kStage + (tid & 255) * kRow + BK) = make_uint2(0, 0);
+    if (tid < 2) odd_group[tid] = -1;
+    __syncthreads();
+  }
   store_stage(0);
-  store_scales(0, 0);
+  store_scales(0, std::integral_constant<int, 0>{});
   for (int j = 0; j < NL; ++j) load_one(j, nstages > 1 ? BK : 0);
   __syncthreads();
 
@@ -298,41 +366,83 @@ void gemm_grouped128_kernel(const GroupedArgs g) {
       const v4i fb0 = *reinterpret_cast<const v4i*>(st + b_off + ks * 32);
       const v4i fb1 = *reinterpret_cast<const v4i*>(st + b_off + 32 * kRow + ks * 32);
       // the first MFMA of a group starts from a zero accumulator operand instead of zeroed registers
-      acc[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fb0, fa, ks == 0 ? kZero : acc[0], 0, 0, 0);
-      acc[1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fb1, fa, ks == 0 ? kZero : acc[1], 0, 0, 0);
+      if constexpr (kQuad) {
+        acc[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa, fb0, ks == 0 ? kZero : acc[0], 0, 0, 0);
+        acc[1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa, fb1, ks == 0 ? kZero : acc[1], 0, 0, 0);
+      } else {
+        acc[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fb0, fa, ks == 0 ? kZero : acc[0], 0, 0, 0);
+        acc[1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fb1, fa, ks == 0 ? kZero : acc[1], 0, 0, 0);
+      }
     }
     // Past the last stage the store and the loads are repeated harmlessly (a buffer nobody reads,
     // k offset 0) rather than branched around.
     store_stage((1 - BUF) * kStage);
     const int k_next = s + 2 < nstages ? (s + 2) * BK : 0;
-    // lane holds C[m = wm*32 + lr][n = wn*64 + ni*32 + 8q + 4lh + e], register 4q + e of tile ni
-    const float rs[1] = {srow[BUF][rs_off]};
+    if constexpr (kQuad) {
+      // accumulators: lane holds C[m = wm*32 + 8q + 4lh + e][n = wn*64 + ni*32 + lr], register 4q + e of tile ni;
+      // sums: C[m = wm*32 + 8q + 4lh + lane % 4][n = wn*64 + ni*32 + 4 (lr / 4) + e]
+      v4s rs[4];
 #pragma unroll
-    for (int ni = 0; ni < 2; ++ni)
+      for (int q = 0; q < 4; ++q) rs[q] = *reinterpret_cast<const v4s*>(st + rs_pad + 8 * q * kRow);
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        if (ni * 4 + q < NL) load_one(ni * 4 + q, k_next);
-        const v16i* const a1[1] = {&acc[ni]};
-        v16f* const s1[1] = {&sum[ni]};
-        R::template quarter<1>(a1, s1, q, rs, *reinterpret_cast<const float4*>(&scol[BUF][cs_off + ni * 32 + 8 * q]));
+      for (int ni = 0; ni < 2; ++ni) {
+        const v4s cs = *reinterpret_cast<const v4s*>(st + cs_pad + 32 * ni * kRow);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          if (ni * 4 + q < NL) load_one(ni * 4 + q, k_next);
+          Quad::add(acc[ni], sum[ni], q, rs[q], cs);
+        }
       }
-    store_scales(s + 1, 1 - BUF);
+    } else {
+      // lane holds C[m = wm*32 + lr][n = wn*64 + ni*32 + 8q + 4lh + e], register 4q + e of tile ni
+      const float rs[1] = {srow[BUF][rs_off]};
+#pragma unroll
+      for (int ni = 0; ni < 2; ++ni)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          if (ni * 4 + q < NL) load_one(ni * 4 + q, k_next);
+          const v16i* const a1[1] = {&acc[ni]};
+          v16f* const s1[1] = {&sum[ni]};
+          R::template quarter<1>(a1, s1, q, rs, *reinterpret_cast<const float4*>(&scol[BUF][cs_off + ni * 32 + 8 * q]));
+        }
+    }
+    store_scales(s + 1, std::integral_constant<int, 1 - BUF>{});
     // a bare s_barrier: a __syncthreads() would also wait for the global loads just issued
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
   };
   for (int s = 0; s < nstages; s += 2) {
+    if constexpr (kQuad) if (__builtin_amdgcn_readfirstlane(odd_group[0]) == s) return false;
     stage(s, std::integral_constant<int, 0>{});
-    if (s + 1 < nstages) stage(s + 1, std::integral_constant<int, 1>{});
+    if (s + 1 < nstages) {
+      if constexpr (kQuad) if (__builtin_amdgcn_readfirstlane(odd_group[1]) == s + 1) return false;
+      stage(s + 1, std::integral_constant<int, 1>{});
+    }
   }
 
   const bool vec = (g.ldc % 4) == 0 && ((uintptr_t)g.c % 16) == 0;
 #pragma unroll
   for (int ni = 0; ni < 2; ++ni)
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
-      store_out4<R::kOutBf16>(g, sum[ni], q, m0 + wm * 32 + lr, n0 + wn * 64 + ni * 32 + 8 * q + 4 * lh, vec);
+    for (int q = 0; q < 4; ++q) {
+      if constexpr (kQuad)
+        store_out4<R::kOutBf16>(g, sum[ni], q, m0 + wm * 32 + 8 * q + 4 * lh + (lane & 3), n0 + wn * 64 + ni * 32 + (lr & ~3), vec);
+      else
+        store_out4<R::kOutBf16>(g, sum[ni], q, m0 + wm * 32 + lr, n0 + wn * 64 + ni * 32 + 8 * q + 4 * lh, vec);
+    }
+  return true;
+}
+
+template <int EPI, bool PACKED>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4)))
+void gemm_grouped128_kernel(const GroupedArgs g) {
+  __shared__ Grouped128Lds lds;
+  if constexpr (EPI == 0) {
+    if (grouped128_tile<EPI, PACKED, true>(g, lds)) return;
+    __syncthreads();  // also waits for the loads the abandoned pass has in flight
+  }
+  grouped128_tile<EPI, PACKED, false>(g, lds);
 }
 
 // ---- groups of 256 and more ------------------------------------------------------------------------

@@ -121,6 +121,37 @@ def test_grouped_gemm_kernel(gpu, m, n, k, group, out, rdt, cdt, packed):
       assert torch.equal(eo, got)
 
 
+@pytest.mark.parametrize('where', ['none', 'first group', 'last group', 'one column', 'subnormal products'])
+@pytest.mark.parametrize('m,n,k', [(65, 8, 128), (130, 257, 384), (40, 70, 512), (16, 130, 8192 + 128)])
+def test_grouped_gemm_scales_beyond_the_matrix_products(gpu, m, n, k, where):
+  """bf16 scales of 2^-60 .. 2^41 are multiplied on the matrix cores, a tile with any other on the vector ALU: the same
+  numbers, infinite and NaN where the oracle's are."""
+  from aqt_amd import _lib as L
+  rng = np.random.default_rng(19)
+  a, b = rng.integers(-128, 128, (m, k)).astype(np.int8), rng.integers(-7, 8, (n, k)).astype(np.int8)
+  a[0], b[0] = -128, -7  # the largest sums a group can have
+  groups = k // 128
+  exps = lambda *shape: np.exp2(rng.integers(-60, 40, shape)).astype(np.float32) * (1 + rng.random(shape, np.float32) * 0.9)
+  rs, cs = nm.to_bf16(exps(groups, m)), nm.to_bf16(np.minimum(exps(groups, n), 1e3))
+  if where == 'first group':
+    rs[0, m // 2], cs[0, 1] = np.inf, 2.0 ** 100
+  elif where == 'last group':
+    rs[-1, 0], cs[-1, n - 1] = 2.0 ** 90, np.nan
+  elif where == 'one column':
+    cs[:, 3] = 0.0
+  elif where == 'subnormal products':
+    rs[:], cs[:] = nm.to_bf16(rs * 0 + np.float32(2.0 ** -80)), nm.to_bf16(cs * 0 + np.float32(2.0 ** -61))
+  with np.errstate(all='ignore'):
+    want = _grouped_ref(a, b, rs, cs, 128, 'bf16', 'bf16', 'bf16')
+  for packed in (False, True):
+    bt = torch.from_numpy(b).to(gpu)
+    for tuning in (0, 128):
+      got = ops.gemm_grouped(torch.from_numpy(a).to(gpu), ops.pack_i4(bt) if packed else bt, row_scale=torch.from_numpy(rs).to(gpu),
+                             col_scale=torch.from_numpy(cs).to(gpu), group=128, out_dtype=torch.bfloat16, tuning=tuning,
+                             row_scale_dtype=torch.bfloat16, col_scale_dtype=torch.bfloat16, b_dtype=L.I4P if packed else L.I4)
+      np.testing.assert_array_equal(got.float().cpu().numpy(), want)
+
+
 def _even_odd8(a):
   """Every aligned group of 8 along the last axis as elements 0,2,4,6,1,3,5,7."""
   g = a.reshape(a.shape[:-1] + (a.shape[-1] // 8, 8))
