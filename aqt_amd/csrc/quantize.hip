@@ -114,6 +114,16 @@ bool tiles_rowmax_ok(const aqtx_quant_plan* p) {
          p->rows % kTileR == 0 && p->cols % kTileC == 0;
 }
 
+// Threads a row (as a shift) with which the columns of this plan are calibrated and quantized in one pass, or -1: new scales
+// of whole columns, transposed output, the compile-time integer pipelines without noise or prescale, and a size that cols_once_shift takes.
+int once_shift_of(const aqtx_quant_plan* p, bool row_maxima) {
+  if (p->reduce != AQTX_REDUCE_ROWS || !p->transpose_out || (p->group != 0 && p->group != p->rows) || p->scale_given || p->noise != AQTX_NOISE_NONE ||
+      p->prescale != AQTX_PRESCALE_NONE || p->compute_dtype != p->in_dtype || p->scale_dtype != p->in_dtype)
+    return -1;
+  if ((p->in_dtype != AQTX_BF16 && p->in_dtype != AQTX_F32) || (p->out_dtype != AQTX_I8 && p->out_dtype != AQTX_I4)) return -1;
+  return cols_once_shift(p->in_dtype == AQTX_BF16 ? 2 : 4, p->batch, p->rows, p->cols, row_maxima);
+}
+
 }  // namespace
 }  // namespace aqtx
 
@@ -205,6 +215,7 @@ static int quantize_impl(const aqtx_quant_plan* p, const void* x, const float* p
   a.cbf = p->compute_dtype == AQTX_BF16; a.sbf = p->scale_dtype == AQTX_BF16;
   a.scale_given = p->scale_given;
   a.ws_zeroed = p->workspace_zeroed;
+  a.once_shift = scale_only ? -1 : once_shift_of(p, p->other_axis_absmax != nullptr);
   if (p->other_axis_absmax != nullptr) {
     AQTX_REQUIRE(aqtx_quantize_other_axis_parts(p) > 0,
                  "aqtx_quantize: this plan cannot write other_axis_absmax (aqtx_quantize_other_axis_parts is 0)");

@@ -57,6 +57,7 @@ struct QArgs {
   const uint16_t* given_bf16;  // given scales as bf16 elements, read where they lie (NULL: in `scale`)
   int ws_zeroed;  // the abs-max words of the workspace are zero on entry
   int scale_only; // the scales are all that is asked for (a calibration on its own): nothing reads or writes q
+  int once_shift; // columns: calibrated and quantized in one pass, with so many threads a row (as a shift); -1: not
   int even_odd8;  // rows kernel: bytes of each group of 8 outputs stored as elements 0,2,4,6,1,3,5,7
   // Partial maxima of |q| along the axis that carries the scales, one byte per position of the reduced axis and
   // part (aqtx_quant_plan::other_axis_absmax): written by a launch (oa_out), or read in place of an abs-max pass
@@ -78,6 +79,28 @@ constexpr int kAbsRowChunk = 64, kAbsColLanes = 64;
 inline int64_t absmax_col_groups(int64_t cols) {
   const int64_t width = kAbsColLanes * (cols >= 8 ? 8 : 1);
   return (cols + width - 1) / width;
+}
+
+// Columns in one pass (quant_cols_once_kernel): rows a thread, by the bytes of a value (64 registers of values), and threads
+// a row (as a shift), 2 to 16.
+template <int ESZ> constexpr int kOnceRows = ESZ == 2 ? 16 : 8;
+constexpr int kOnceMaxShift = 4;
+// The shift, or -1 where calibration and quantization stay launches of their own: columns beyond a block's registers, and
+// row maxima, whose parts are 64 columns, beyond those of 8 threads a row.  Few threads a row while that gives the chip two
+// blocks a CU, but a wave a block: 4096 x 4096 bf16 14.5 us with 2 and 17.6 with 4, 8 entries of 4096 x 14336 444 and 421,
+// 128 x 16384 with 2 8, with 4 5.3.  Calibration and quantization in launches of their own / in one, us:
+//   bf16     16 x 2048 9.8 / 5.6, 512 x 512 8.2 / 5.1, 1030 x 3001 11.2 / 7.0, 2048 x 64 8.6 / 6.1, 2048 x 16384 36.1 / 23.2,
+//            4096 x 1024 10.7 / 9.3, 4096 x 4096 21.8 / 14.5, 4096 x 14336 52 / 41, 8 entries of it 477 / 421
+//   float32  128 x 512 8.5 / 3.9, 512 x 2048 9.0 / 4.4, 1024 x 8192 19.0 / 9.4, 2048 x 2048 11.7 / 7.0, 2048 x 8192 28.1 / 19.5
+inline int cols_once_shift(int esz, int64_t batch, int64_t rows, int64_t cols, bool row_maxima) {
+  const int R = esz == 2 ? 16 : 8;
+  const int64_t groups = (rows + R - 1) / R;
+  if (rows < R || cols < 8 || groups > 256) return -1;
+  if (row_maxima) return groups <= 128 ? 3 : -1;
+  int shift = 1;
+  while (shift < kOnceMaxShift && (groups << shift) < 64) ++shift;
+  while (shift < kOnceMaxShift && (groups << (shift + 1)) <= 1024 && batch * (cols >> (shift + 4)) >= 512) ++shift;
+  return shift;
 }
 
 // Launches the passes of one plan for one input type.
@@ -406,6 +429,29 @@ __device__ __forceinline__ uint2 pack8(const uint32_t (&q)[8], int even_odd8) {
   if (even_odd8)
     return make_uint2(q[0] | (q[2] << 8) | (q[4] << 16) | (q[6] << 24), q[1] | (q[3] << 8) | (q[5] << 16) | (q[7] << 24));
   return make_uint2(q[0] | (q[1] << 8) | (q[2] << 16) | (q[3] << 24), q[4] | (q[5] << 8) | (q[6] << 16) | (q[7] << 24));
+}
+
+// quant_cols_once_kernel: maxima of magnitudes (bf16: two to a word) and the eight values of a row's registers.
+template <typename TIn> __device__ __forceinline__ uint32_t once_max(uint32_t x, uint32_t y) {
+  if constexpr (sizeof(TIn) == 2)
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2_t, x), __builtin_bit_cast(u16x2_t, y)));
+  return x > y ? x : y;
+}
+template <typename TIn, int W> __device__ __forceinline__ void once_unpack(const uint4 (&w)[W], float (&v)[8]) {
+  if constexpr (sizeof(TIn) == 2) {
+    const uint32_t x[4] = {w[0].x, w[0].y, w[0].z, w[0].w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      v[2 * i] = __uint_as_float(x[i] << 16);
+      v[2 * i + 1] = __uint_as_float(x[i] & 0xFFFF0000u);
+    }
+  } else {
+#pragma unroll
+    for (int h = 0; h < W; ++h) {
+      v[4 * h] = __uint_as_float(w[h].x); v[4 * h + 1] = __uint_as_float(w[h].y);
+      v[4 * h + 2] = __uint_as_float(w[h].z); v[4 * h + 3] = __uint_as_float(w[h].w);
+    }
+  }
 }
 
 // ---- rows kernel: reduced axis contiguous -------------------------------------
@@ -929,6 +975,120 @@ __global__ __launch_bounds__(256) void finalize_partials_kernel(const QArgs a, i
 }
 
 
+// Columns in one pass: a block owns 8 << tshift whole columns, reads them once into registers, finds their scales and
+// writes the quantized values; no abs-max launch, no workspace, no second read.  A thread holds kOnceRows consecutive rows of
+// 8 columns, so the bytes of a column (transposed output) leave as one 16-byte (float32: 8-byte) store a thread, 64 lanes together
+// covering whole lines.  Bound by HBM bytes: one read and one write.
+// ROWMAX (8 threads a row): see quant_tile_kernel.
+template <typename TIn, int SPEC, bool ROWMAX>
+__global__ __launch_bounds__(1024) void quant_cols_once_kernel(const QArgs a, const int tshift) {
+  constexpr int R = kOnceRows<sizeof(TIn)>, W = 8 * sizeof(TIn) / 16;
+  __shared__ __attribute__((aligned(16))) uint32_t smax[16][8 << kOnceMaxShift];
+  __shared__ __attribute__((aligned(16))) float sinv[8 << kOnceMaxShift];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int T = 1 << tshift, width = 8 << tshift, slot = tid & (T - 1);
+  // Blocks of part of a line (2 or 4 threads a row): those of one line go to blocks i, i + 8, ..., which share an XCD.
+  int cb = blockIdx.x;
+  const int sib = 3 - tshift > 0 ? 3 - tshift : 0;
+  if (cb < ((int)gridDim.x & -(8 << sib))) cb = (cb & -(8 << sib)) | ((cb & 7) << sib) | ((cb >> 3) & ((1 << sib) - 1));
+  // a thread's columns and rows; where they would hang over the end, the last ones (met twice: the same bytes twice)
+  auto columns_at = [&](int t) -> int64_t {
+    const int64_t c = (int64_t)cb * width + t * 8;
+    return c >= a.cols ? a.cols : c + 8 <= a.cols ? c : a.cols - 8;
+  };
+  const int64_t c0 = columns_at(slot);
+  int64_t r0 = (int64_t)(tid >> tshift) * R;
+  const bool active = c0 < a.cols && r0 < a.rows;
+  if (r0 + R > a.rows) r0 = a.rows - R;
+  const int64_t b = blockIdx.y;
+  uint4 w[R][W];
+  if (active) {
+    const TIn* p = reinterpret_cast<const TIn*>(a.x) + (b * a.rows + r0) * a.cols + c0;
+#pragma unroll
+    for (int j = 0; j < R; ++j)
+#pragma unroll
+      for (int h = 0; h < W; ++h) w[j][h] = load_unaligned<uint4>(p + j * a.cols + h * (8 / W));
+  } else {
+#pragma unroll
+    for (int j = 0; j < R; ++j)
+#pragma unroll
+      for (int h = 0; h < W; ++h) w[j][h] = make_uint4(0, 0, 0, 0);
+  }
+  // magnitudes order like unsigned integers, NaN above infinity
+  uint32_t m[4 * W];
+#pragma unroll
+  for (int i = 0; i < 4 * W; ++i) m[i] = 0u;
+#pragma unroll
+  for (int j = 0; j < R; ++j)
+#pragma unroll
+    for (int h = 0; h < W; ++h) {
+      const uint32_t x[4] = {w[j][h].x, w[j][h].y, w[j][h].z, w[j][h].w};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) m[4 * h + i] = once_max<TIn>(m[4 * h + i], sizeof(TIn) == 2 ? x[i] & 0x7FFF7FFFu : x[i] & 0x7FFFFFFFu);
+    }
+  for (int off = T; off < 64; off <<= 1)
+#pragma unroll
+    for (int i = 0; i < 4 * W; ++i) m[i] = once_max<TIn>(m[i], (uint32_t)__shfl_xor((int)m[i], off, 64));
+  if (lane < T) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      smax[wave][lane * 8 + e] = sizeof(TIn) == 2 ? ((e & 1) ? m[e >> 1] & 0xFFFF0000u : m[e >> 1] << 16) : m[e];
+  }
+  __syncthreads();
+  for (int i = tid; i < width; i += blockDim.x) {
+    const int64_t first = columns_at(i >> 3), c = first + (i & 7);
+    if (first < a.cols) {
+      uint32_t mm = smax[0][i];
+      for (int v = 1; v < ((int)blockDim.x >> 6); ++v) mm = mm > smax[v][i] ? mm : smax[v][i];
+      float scale, inv;
+      spec_scale_from_absmax<SPEC>(__uint_as_float(mm), a, scale, inv);
+      store_scale(a, b * a.ssb + c * a.ssc, scale);
+      sinv[i] = inv;
+    }
+  }
+  __syncthreads();
+  if (!active) return;  // (ROWMAX: whole rows of the block's threads at a time)
+  float inv[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) inv[e] = sinv[slot * 8 + e];
+  uint8_t* q = reinterpret_cast<uint8_t*>(a.q) + b * a.rows * a.cols;
+  uint32_t out[8][R / 4], rmax[R / 4];
+#pragma unroll
+  for (int i = 0; i < R / 4; ++i) {
+    rmax[i] = 0u;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) out[e][i] = 0u;
+  }
+#pragma unroll
+  for (int j = 0; j < R; ++j) {
+    float v[8], rm = 0.0f;
+    once_unpack<TIn>(w[j], v);
+    uint32_t qv[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      if constexpr (ROWMAX) {
+        float tc;
+        qv[e] = spec_quant_mag<SPEC>(v[e], inv[e], 0, a, tc);
+        rm = fmaxf(rm, fabsf(tc));
+      } else {
+        qv[e] = spec_quant<SPEC>(v[e], inv[e], 0, a);
+      }
+      out[e][j >> 2] |= qv[e] << (8 * (j & 3));
+    }
+    if constexpr (ROWMAX) {
+#pragma unroll
+      for (int off = 1; off < 8; off <<= 1) rm = fmaxf(rm, __shfl_xor(rm, off, 64));
+      rmax[j >> 2] |= (uint32_t)(int)rintf(rm) << (8 * (j & 3));
+    }
+    __builtin_amdgcn_sched_barrier(0);  // row after row, so that their bytes take the registers of the values
+  }
+#pragma unroll
+  for (int e = 0; e < 8; ++e) __builtin_memcpy(q + (c0 + e) * a.rows + r0, out[e], R);
+  if constexpr (ROWMAX) {
+    if (slot == 0) __builtin_memcpy(a.oa_out + (int64_t)cb * a.rows + r0, rmax, R);
+  }
+}
+
 // 128x64 tile: thread (rg = tid/8, cc = tid%8) owns rows 4*rg..+3, cols 8*cc..+7.
 // PAIR (SPEC 2 and 7, and SPEC 5 with value 1): 1 = the block also owns the tile `rows/2` further down (natural noise
 // layout), 2 = the tile `cols/2` further right (noise counters of the transposed tensor); the
@@ -1271,6 +1431,18 @@ int launch_rows(const QArgs& a, int partitionable, hipStream_t st) {
 
 template <typename TIn>
 int launch_tiles(const QArgs& a, int reduce, int partitionable, int64_t nscales, hipStream_t st) {
+  if constexpr (sizeof(TIn) != 1) {
+    if (a.once_shift >= 0) {
+      const int R = kOnceRows<sizeof(TIn)>, shift = a.once_shift;
+      const int threads = (int)((((a.rows + R - 1) / R << shift) + 63) / 64 * 64);
+      const dim3 grid((unsigned)((a.cols + (8 << shift) - 1) / (8 << shift)), (unsigned)a.batch);
+      constexpr int kInt = sizeof(TIn) == 2 ? 1 : 6;
+      if (a.oa_out != nullptr) quant_cols_once_kernel<TIn, kInt, true><<<grid, threads, 0, st>>>(a, shift);
+      else quant_cols_once_kernel<TIn, kInt, false><<<grid, threads, 0, st>>>(a, shift);
+      AQTX_HIP_CHECK_LAUNCH("quant_cols_once_kernel");
+      return 0;
+    }
+  }
   if (a.oa_in != nullptr) {
     finalize_partials_kernel<<<dim3((unsigned)(nscales / 16)), 256, 0, st>>>(a, nscales);
     AQTX_HIP_CHECK_LAUNCH("finalize_partials_kernel");

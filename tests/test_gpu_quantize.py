@@ -520,6 +520,34 @@ def test_column_scales_on_both_sides_of_the_fold(gpu, dt, prescaled, rows, cols)
                                   scale=s, **kw)[0], q)
 
 
+@pytest.mark.parametrize('batch,rows,cols', [(1, 8, 8), (1, 15, 40), (2, 16, 9), (3, 17, 130), (1, 129, 1024), (1, 2048, 200),
+                                             (2, 2049, 72), (1, 4096, 24), (1, 4097, 24), (17, 100, 8200), (1, 128, 64)])
+@pytest.mark.parametrize('dt,bits', [('bf16', 8), ('bf16', 4), ('f32', 8)])
+def test_columns_in_one_pass(gpu, dt, bits, batch, rows, cols):
+  """Fewest and most rows of the kernel that reads a column once, edges of its blocks, special values; the scales alone
+  and the quantization with given scales come from other kernels."""
+  x = U.rand((batch, rows, cols), dt, seed=rows + cols, outliers=True)
+  x[:, :, 1] = 0.0
+  x[:, rows - 1, 2], x[:, 0, cols - 1] = np.inf, -np.inf
+  q = R.QuantizerCfg(bits=bits)
+  qb, cb = U.bounds(q)
+  kw = dict(reduce=L.REDUCE_ROWS, out_dtype=U.OUT_DT[bits], quant_bound=qb, clip_bound=cb, transpose_out=True)
+  finite = np.isfinite(x).all((0, 1))
+  with np.errstate(all='ignore'):
+    qt = R.quantize(x, dt, q, [1])
+  xt = U.to_dev(x, dt, gpu)
+  qg, sg = ops.quantize(xt, **kw)
+  np.testing.assert_array_equal(sg.cpu().numpy().reshape(-1), qt.scale[0].reshape(-1))
+  np.testing.assert_array_equal(np.swapaxes(qg.cpu().numpy(), -1, -2)[..., finite], qt.qvalue.astype(np.int8)[..., finite])
+  assert torch.equal(ops.quantize(xt, scale_only=True, **kw)[1], sg)
+  assert torch.equal(ops.quantize(xt, scale=sg, **kw)[0], qg)  # infinite columns too
+  if rows % 128 == 0 and cols % 64 == 0 and batch == 1:
+    with_maxima, _ = ops.quantize(xt, want_other_axis_absmax=True, **kw)
+    assert torch.equal(with_maxima, qg)
+  x[0, rows // 2, 0] = np.nan
+  assert torch.isnan(ops.quantize(U.to_dev(x, dt, gpu), **kw)[1].reshape(batch, cols)[0, 0])
+
+
 @pytest.mark.parametrize('reduce,shape', [(L.REDUCE_COLS, (1, 5, 3000)), (L.REDUCE_COLS, (1, 3, 5)), (L.REDUCE_COLS, (2, 2, 20000)),
                                           (L.REDUCE_ROWS, (1, 300, 72)), (L.REDUCE_ALL, (2, 100, 64))])
 def test_calibration_alone_gives_the_scales_of_the_quantization(gpu, reduce, shape):
