@@ -636,6 +636,10 @@ def _canonical_pairs(lhs, rhs, dimension_numbers):
 
 _NotFused = lowering.NotFused
 
+# The named scope a profiler sees around a contraction.  torch's own light-weight form of record_function, for scopes entered
+# from Python in hot code (0.3 against 12 us with no profiler running), where this torch has it.
+_profiler_scope = getattr(torch._C._profiler, '_RecordFunctionFast', torch.profiler.record_function)
+
 # (lhs, rhs): whether the forward quantizers of this call should leave, next to the values they write, the partial
 # maxima with which the backward pass calibrates those values over the other axis (DotGeneralRaw._quant_side); set
 # by the differentiable entry point for the operands whose residual a backward contraction re-quantizes.
@@ -684,7 +688,7 @@ class DotGeneralRaw:
     transposed (and contiguous).  `_bwd_memo` (this build): a dict owned by one backward pass, in
     which its two contractions share per-tensor scales of the gradient.
     """
-    with torch.profiler.record_function(self.jax_scope_name):
+    with _profiler_scope(self.jax_scope_name):
       if isinstance(rhs, MultiTensor):
         lhs, rhs = _maybe_use_fwd_quant(lhs, rhs, dimension_numbers, self.rhs.use_fwd_quant)
       if self.local_aqt is None:
@@ -1200,11 +1204,11 @@ class DotGeneralRaw:
     # first serving call
     w_fragments = _kernel_layout_of(rhs_qt.qvalue, rv, pack_int4=packed, fragments=True)
     w_scale = rhs_qt.scale[0]
-    sv = lowering.view_operand(w_scale, [], rra, rca)
-    if sv.mem.numel() != N:
+    w_scale_vector = _scale_vector_f32(w_scale, [], rra, rca)
+    if w_scale_vector.numel() != N:
       return None
     sdt = dq.lhs._calibrator.dtype if dq.lhs._calibrator.dtype is not None else lhs_dtype
-    out, xs, xq = ops.decode(lv.mem[0], w_fragments, _scale_vector_f32(w_scale, [], rra, rca),
+    out, xs, xq = ops.decode(lv.mem[0], w_fragments, w_scale_vector,
                              quant_bound=spec['quant_bound'], clip_bound=spec['clip_bound'],
                              x_scale_dtype=sdt, w_scale_dtype=w_scale.dtype, want_xq=True,
                              w_dtype=L.I4P if packed else L.I4 if rhs_qt.container_dtype is utils.int4 else L.I8,
@@ -1479,7 +1483,7 @@ class DotGeneral:
     if self.apply_custom_vjp_on_jax and (lhs.requires_grad or rhs.requires_grad):
       out, lq, rq = _DgCoreFn.apply(lhs, rhs, lhs_qt, rhs_qt, dimension_numbers, self)
       return out, (lq, rq)
-    (out, qret), _ = dg_core_vjp_fwd(lhs, rhs, lhs_qt, rhs_qt, dimension_numbers, self)
+    (out, qret), _ = dg_core_vjp_fwd(lhs, rhs, lhs_qt, rhs_qt, dimension_numbers, self, fwd_only=True)
     return out, qret
 
   def fused_tile_sum(self, lhs, rhs, dimension_numbers, n_sum_axes: int, lhs_qt=None, rhs_qt=None,
@@ -1501,7 +1505,7 @@ class DotGeneral:
       return None
     (lca, rca), (lba, rba) = dimension_numbers
     lca, rca, lba, rba = list(lca), list(rca), list(lba), list(rba)
-    cfg = _fresh_cfg(self)   # calibration objects are created per call, as in dg_core_vjp_fwd
+    cfg = _fresh_cfg(self, fwd_only=True)   # calibration objects are created per call, as in dg_core_vjp_fwd
     cfg.fwd.dg_quantizer.init_calibration()
     raw, dq = cfg.fwd, cfg.fwd.dg_quantizer
     if (len(lca) != 1 or len(lba) != 1 or lhs.dtype != rhs.dtype or lhs.dtype not in (utils.bfloat16, utils.float32)
@@ -1618,12 +1622,13 @@ class DotGeneral:
                   and self.fwd.rhs.dequant_mode == dequant_mode), msg + ' for rhs.'
 
 
-def clone_down_to_quantizers(cfg: 'DotGeneral', reset_calibrators: bool = False) -> 'DotGeneral':
+def clone_down_to_quantizers(cfg: 'DotGeneral', reset_calibrators: bool = False, fwd_only: bool = False) -> 'DotGeneral':
   """New DotGeneral / DotGeneralRaw / dot-general-quantizer / Quantizer objects around the same settings
   objects (Tensor, LocalAqt, numerics, calibration factories are shared with `cfg`): everything a call
-  writes to (contexts, calibrators) is private to the copy."""
+  writes to (contexts, calibrators) is private to the copy.  fwd_only: for a call without gradients, which writes to the
+  forward contraction's objects alone; the others are shared too."""
   cfg = utils.clone_fields(cfg)
-  for name in ('fwd', 'dlhs', 'drhs'):
+  for name in ('fwd',) if fwd_only else ('fwd', 'dlhs', 'drhs'):
     raw = utils.clone_fields(getattr(cfg, name))
     dq = utils.clone_fields(raw.dg_quantizer)
     for qn in ('lhs', 'rhs', 'lhs_mid', 'rhs_mid'):
@@ -1637,23 +1642,25 @@ def clone_down_to_quantizers(cfg: 'DotGeneral', reset_calibrators: bool = False)
   return cfg
 
 
-def _fresh_cfg(cfg: 'DotGeneral') -> 'DotGeneral':
+def _fresh_cfg(cfg: 'DotGeneral', fwd_only: bool = False) -> 'DotGeneral':
   """Copy of the config tree down to the quantizers, calibrators not yet made.
 
   Under jax.custom_vjp the config reaches dg_core_vjp_fwd as a pytree argument, i.e. as a
   fresh copy on every call, which is why init_calibration() may assert that it runs once;
   this gives a reused config object the same behaviour.
   """
-  return clone_down_to_quantizers(cfg, reset_calibrators=True)
+  return clone_down_to_quantizers(cfg, reset_calibrators=True, fwd_only=fwd_only)
 
 
-def dg_core_vjp_fwd(lhs, rhs, lhs_qt, rhs_qt, dimension_numbers, cfg: DotGeneral):
-  """Forward pass (aqt_dot_general.py:1098-1124)."""
+def dg_core_vjp_fwd(lhs, rhs, lhs_qt, rhs_qt, dimension_numbers, cfg: DotGeneral, *, fwd_only: bool = False):
+  """Forward pass (aqt_dot_general.py:1098-1124).  fwd_only: for a caller that drops the residuals; the gradient
+  contractions' calibrators are not made (a layer served from Python: the copies were a quarter of a call's 124 us)."""
   assert lhs.dtype == rhs.dtype, f'Unmatched lhs and rhs dtype: {lhs.dtype} vs {rhs.dtype}'
-  cfg = _fresh_cfg(cfg)
+  cfg = _fresh_cfg(cfg, fwd_only)
   cfg.fwd.dg_quantizer.init_calibration()
-  cfg.dlhs.dg_quantizer.init_calibration()
-  cfg.drhs.dg_quantizer.init_calibration()
+  if not fwd_only:
+    cfg.dlhs.dg_quantizer.init_calibration()
+    cfg.drhs.dg_quantizer.init_calibration()
   ret, res = cfg.fwd(lhs, rhs, lhs_qt, rhs_qt, dimension_numbers)
   ret = ret.to(lhs.dtype)
   assert res is not None, 'res cannot be None in fwd pass.'

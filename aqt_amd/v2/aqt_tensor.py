@@ -60,7 +60,9 @@ class QTensor:
     return self.qvalue is not None
 
   def without_qvalue(self):
-    return self.replace(qvalue=None)
+    out = utils.clone_fields(self)
+    out.qvalue = None
+    return out
 
   def astype(self, dtype):
     return self.replace(dequant_dtype=dtype)

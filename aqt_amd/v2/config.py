@@ -42,13 +42,14 @@ def _fan_out_key(key):
 
 def set_context(cfg: DotGeneral, key, train_step: Optional[int],
                 lhs_quant_mode: utils.QuantMode = utils.QuantMode.TRAIN,
-                rhs_quant_mode: utils.QuantMode = utils.QuantMode.TRAIN, *, copy_settings: bool = True):
+                rhs_quant_mode: utils.QuantMode = utils.QuantMode.TRAIN, *, copy_settings: bool = True, fwd_only: bool = False):
   """Fans the PRNG key out to fwd/dlhs/drhs and lhs/rhs (config.py:66-90).
 
   Returns a deep copy of `cfg` with the contexts set, as the reference does.  With
   copy_settings=False the copy stops at the quantizers (the objects the contexts are written to)
   and shares the settings objects below them with `cfg`: for a caller that hands the result to
-  one dot_general call and drops it (the layer modules, on every call), at a fifth of the cost.
+  one dot_general call and drops it (the layer modules, on every call), at a fifth of the cost; with
+  fwd_only as well, the gradient contractions are left as they are, for a call without gradients.
   """
 
   def set_dg_raw_context(cfg_raw: DotGeneralRaw, keys):
@@ -64,7 +65,10 @@ def set_context(cfg: DotGeneral, key, train_step: Optional[int],
   if copy_settings or not plain:
     ret_cfg = copy.deepcopy(cfg)
   else:
-    ret_cfg = aqt_dot_general.clone_down_to_quantizers(cfg)
+    ret_cfg = aqt_dot_general.clone_down_to_quantizers(cfg, fwd_only=fwd_only)
+    if fwd_only:
+      set_dg_raw_context(ret_cfg.fwd, keys_fwd)
+      return ret_cfg
   set_dg_raw_context(ret_cfg.fwd, keys_fwd)
   set_dg_raw_context(ret_cfg.dlhs, keys_dlhs)
   set_dg_raw_context(ret_cfg.drhs, keys_drhs)

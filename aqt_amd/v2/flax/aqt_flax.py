@@ -241,8 +241,10 @@ class AqtDotGeneral(torch.nn.Module, _RngMixin):
       rhs_freezer = self._freezer(self.rhs_var_name, lambda: general_freezer.Freezer(
           name=self.rhs_var_name, collection=self.quant_collection,
           axis_metadata_wrapper=self.rhs_axis_metadata_wrapper))
-      lhs_freezer.mode = _QUANT_TO_FREEZER_MODE[self.lhs_quant_mode]
-      rhs_freezer.mode = _QUANT_TO_FREEZER_MODE[self.rhs_quant_mode]
+      for freezer, mode in ((lhs_freezer, _QUANT_TO_FREEZER_MODE[self.lhs_quant_mode]),
+                            (rhs_freezer, _QUANT_TO_FREEZER_MODE[self.rhs_quant_mode])):
+        if freezer.mode is not mode:  # (setting an attribute of a module costs a microsecond)
+          freezer.mode = mode
     pending = getattr(self, '_pending', None)
     if pending is not None:
       for name, fr in ((self.lhs_var_name, lhs_freezer), (self.rhs_var_name, rhs_freezer)):
@@ -250,8 +252,13 @@ class AqtDotGeneral(torch.nn.Module, _RngMixin):
       self._pending = None
 
     key = self.make_rng(self.prng_name) if self.prng_name is not None else None
-    cfg = config.set_context(cfg, key, train_step=None, lhs_quant_mode=self.lhs_quant_mode,
-                             rhs_quant_mode=self.rhs_quant_mode, copy_settings=False)
+    modes = dict(lhs_quant_mode=self.lhs_quant_mode, rhs_quant_mode=self.rhs_quant_mode)
+    settings, made = cfg, {}
+
+    def with_context(fwd_only):
+      if fwd_only not in made:
+        made[fwd_only] = config.set_context(settings, key, train_step=None, copy_settings=False, fwd_only=fwd_only, **modes)
+      return made[fwd_only]
 
     def ret_dg(lhs, rhs, dimension_numbers, precision=None, preferred_element_type=None):
       del preferred_element_type
@@ -260,7 +267,8 @@ class AqtDotGeneral(torch.nn.Module, _RngMixin):
       msg += f'lhs.dtype: {lhs.dtype}, rhs.dtype: {rhs.dtype}'
       assert lhs.dtype in [utils.bfloat16, utils.float32, utils.float16], msg
       assert rhs.dtype in [utils.bfloat16, utils.float32, utils.float16], msg
-      cfg.assert_config_validity()
+      settings.assert_config_validity()
+      cfg = with_context(fwd_only=not (settings.apply_custom_vjp_on_jax and (lhs.requires_grad or rhs.requires_grad)))
 
       lhs_qt = lhs_freezer.get() if self.lhs_apply_quant_mode else self.lhs_qtensor
       rhs_qt = rhs_freezer.get() if self.rhs_apply_quant_mode else self.rhs_qtensor
@@ -301,7 +309,7 @@ class AqtDotGeneral(torch.nn.Module, _RngMixin):
       # in CONVERT, and FreezerMode.CALIBRATION keeps the scales alone)
       lhs_values_kept = (self.lhs_apply_quant_mode and self.lhs_quant_mode == QuantMode.CONVERT
                          and self.lhs_freeze_mode != FreezerMode.CALIBRATION)
-      res = cfg.fused_tile_sum(tl, tr, tiled_dn, n_sum_axes, lhs_qt=lhs_qt, rhs_qt=rhs_qt, with_qt=True,
+      res = with_context(fwd_only=True).fused_tile_sum(tl, tr, tiled_dn, n_sum_axes, lhs_qt=lhs_qt, rhs_qt=rhs_qt, with_qt=True,
                                lhs_qvalue_needed=lhs_values_kept)
       if res is None:
         return None
@@ -336,7 +344,7 @@ class AqtDotGeneral(torch.nn.Module, _RngMixin):
       meta = lambda t: torch.empty(t.shape, dtype=torch.float32, device='meta')
       try:
         tiled_dot_general.tiled_dot_general_with_tiling_states(
-            meta(lhs), copy.deepcopy(xlhs), meta(rhs), copy.deepcopy(xrhs), dimension_numbers, dot_general=probe)
+            meta(lhs), xlhs, meta(rhs), xrhs, dimension_numbers, dot_general=probe)  # (reads the states only)
       except _ProbeDone:
         pass
       aqt_dg = self.make_aqt_dg(seen['l'], seen['r'], seen['dn'], lhs_tile_map=xlhs.tile_map,
