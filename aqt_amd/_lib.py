@@ -138,6 +138,7 @@ SYMBOLS = {
     'aqtx_pad_rows': (ctypes.c_int, [ctypes.c_int64, ctypes.c_int64, _vp, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, _vp,
                                      _vp, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, _vp, _vp]),
     'aqtx_gemm_i8_k_slices': (ctypes.c_int, [ctypes.POINTER(GemmPlan)]),
+    'aqtx_gemm_weight_only_k_slices': (ctypes.c_int, [ctypes.POINTER(GemmPlan)]),
     'aqtx_gemm_fp8': (ctypes.c_int, [ctypes.POINTER(GemmPlan), _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
     'aqtx_gemm_weight_only': (ctypes.c_int, [ctypes.POINTER(GemmPlan), _vp, _vp, _vp, _vp, _vp]),
     'aqtx_decode_i8': (ctypes.c_int, [ctypes.POINTER(DecodePlan), _vp, _vp, _vp, _vp, _vp, _vp,

@@ -1035,6 +1035,10 @@ int launch_gemm_i8_frag(const aqtx_gemm_plan* p, const void* a, const void* b, c
                         const float* col_scale, void* c, int32_t* acc_out, hipStream_t st);
 int launch_gemm_weight_only_mid(const aqtx_gemm_plan* p, const void* a, const void* b, const float* col_scale, void* c,
                                 hipStream_t st);
+// gemm_wo_slices.hip: the same contraction with k in slices (p->k_split_workspace holds their float32 sums)
+int gemm_weight_only_k_slices(const aqtx_gemm_plan* p);
+int launch_gemm_weight_only_slices(const aqtx_gemm_plan* p, const void* a, const void* b, const float* col_scale, void* c,
+                                   int slices, hipStream_t st);
 // gemm_wo.hip: the same contraction on 256 x 256 tiles; `workgroups` > 0: that many workgroups walk the tiles
 int launch_gemm_weight_only_large(const aqtx_gemm_plan* p, const void* a, const void* b, const float* col_scale, void* c,
                                   int workgroups, hipStream_t st);

@@ -201,6 +201,11 @@ extern "C" int aqtx_conv_i8(const aqtx_im2col_plan* w, const aqtx_gemm_plan* p, 
   return launch_conv_i8_mid(w, p, x, b, row_scale, col_scale, c, reinterpret_cast<hipStream_t>(stream));
 }
 
+extern "C" int aqtx_gemm_weight_only_k_slices(const aqtx_gemm_plan* p) {
+  if (p == nullptr || p->batch <= 0 || p->m <= 0 || p->n <= 0 || p->k <= 0) return 1;
+  return gemm_weight_only_k_slices(p);
+}
+
 extern "C" int aqtx_gemm_weight_only(const aqtx_gemm_plan* p, const void* a, const void* b, const float* col_scale,
                                      void* c, void* stream) {
   clear_error();
@@ -225,6 +230,11 @@ extern "C" int aqtx_gemm_weight_only(const aqtx_gemm_plan* p, const void* a, con
   if (p->batch == 0 || p->m == 0 || p->n == 0) return 0;
   AQTX_REQUIRE(a != nullptr && b != nullptr && c != nullptr, "%s: NULL buffer", who);
   AQTX_REQUIRE(((uintptr_t)a % 16) == 0 && ((uintptr_t)b % 16) == 0 && ((uintptr_t)c % 2) == 0, "%s: a and b must be 16-byte aligned", who);
+  // few tiles and a long k: slices, where the caller lent the memory for their sums
+  if (const int slices = gemm_weight_only_k_slices(p);
+      slices > 1 && p->k_split_workspace != nullptr && ((uintptr_t)p->k_split_workspace % 16) == 0 &&
+      p->k_split_workspace_bytes >= (int64_t)slices * p->batch * p->m * p->n * 4)
+    return launch_gemm_weight_only_slices(p, a, b, col_scale, c, slices, reinterpret_cast<hipStream_t>(stream));
   // 256 x 256 tiles where they fill the chip (the rule of aqtx_gemm_i8), walked by one workgroup per CU from two
   // rounds of them on; plan->tuning: 128 = the 128 x 128 tiles, 8 = the large ones with a workgroup per tile
   const int64_t pad256 = ((p->m + BM - 1) / BM) * ((p->n + BN - 1) / BN), pad128 = ((p->m + 127) / 128) * ((p->n + 127) / 128);

@@ -469,8 +469,9 @@ def gemm_weight_only(a: torch.Tensor, b: torch.Tensor, col_scale: torch.Tensor, 
   """Weight-only contraction C[b] = bf16(bf16(A[b] @ float(B[b])^T) * col_scale[b]) for bf16 A [batch, m, k] that
   stays unquantized and int8 B [batch, n, k] (k contiguous in both), any m; `col_scale` is float32 [batch, n]
   holding values of `col_scale_dtype`.  float32 sums; the weight is never copied as bf16.  tuning (None =
-  GEMM_TUNING): 128 = 128 x 128 tiles, 8 = 256 x 256 tiles, 16 = those walked by one workgroup per CU; every
-  choice sums k in the same order, so the results do not depend on it."""
+  GEMM_TUNING): 128 = 128 x 128 tiles, 8 = 256 x 256 tiles, 16 = those walked by one workgroup per CU; every one of them
+  sums k in the same order, so the results do not depend on it.  Without one, a long k over few output tiles is summed in
+  slices."""
   _require_gpu(a, b, col_scale)
   assert a.dim() == 3 and a.dtype == torch.bfloat16 and a.stride(2) == 1
   batch, m, k = a.shape
@@ -495,6 +496,10 @@ def gemm_weight_only(a: torch.Tensor, b: torch.Tensor, col_scale: torch.Tensor, 
   plan.tuning = GEMM_TUNING if tuning is None else tuning
   if plan.tuning == 4:
     plan.tuning = 8  # the weight-only kernel has one workgroup shape on the large tiles
+  slices = L.lib().aqtx_gemm_weight_only_k_slices(ctypes.byref(plan))
+  if slices > 1:  # slices of k leave their partial sums in slabs of a scratch array
+    slabs = torch.empty((slices, batch, m, n), dtype=torch.float32, device=a.device)
+    plan.k_split_workspace, plan.k_split_workspace_bytes = slabs.data_ptr(), slabs.numel() * 4
   with _timed('gemm'):
     L.check(L.lib().aqtx_gemm_weight_only(ctypes.byref(plan), _ptr(a), _ptr(b), _ptr(col_scale), _ptr(c), _stream()))
   return c

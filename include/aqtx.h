@@ -260,13 +260,15 @@ typedef struct aqtx_gemm_plan {
                                  one barrier per two stages                                               */
   int32_t a_k_order;          /* AQTX_K_*: byte order of a along k; EVEN_ODD8 (aqtx_gemm_i8 with b_dtype
                                  AQTX_I4P only) saves the kernel the re-interleaving of the nibbles   */
-  int32_t k_split;            /* aqtx_gemm_i8 only.  Tuning only (int32 partial sums add up exactly in any
+  int32_t k_split;            /* aqtx_gemm_i8.  Tuning only (int32 partial sums add up exactly in any
                                  order): 0 = the library chooses, 1 = one workgroup per output tile walks
                                  all of k, S > 1 = k is cut into (at most) S slices contracted by
                                  workgroups of their own, for shapes with few output tiles and a long k.
-                                 Slices write partial sums to k_split_workspace                        */
+                                 Slices write partial sums to k_split_workspace.  aqtx_gemm_weight_only: 0 =
+                                 the library chooses, 1 = no slices                                    */
   void* k_split_workspace;    /* DEVICE scratch for the slices, 16-byte aligned, at least
-                                 aqtx_gemm_i8_k_slices(plan) * batch * m * n * 4 bytes; NULL: no slices
+                                 aqtx_gemm_i8_k_slices(plan) * batch * m * n * 4 bytes (or
+                                 aqtx_gemm_weight_only_k_slices); NULL: no slices
                                  unless k_split > 1 asks for them (then an error)                      */
   int64_t k_split_workspace_bytes;
   int32_t b_layout;           /* aqtx_gemm_i8 and aqtx_gemm_weight_only.  AQTX_W_ROWS (0): b is [batch][n][k] rows.
@@ -304,6 +306,12 @@ int aqtx_gemm_i8(const aqtx_gemm_plan* plan, const void* a, const void* b,
  * contraction algorithm).
  */
 int aqtx_gemm_i8_k_slices(const aqtx_gemm_plan* plan);
+
+/*
+ * The same for aqtx_gemm_weight_only, whose slices leave float32 sums: with them the sum over k is formed slice by slice,
+ * so the last bit of a result may differ from a call without k_split_workspace (or with k_split = 1).
+ */
+int aqtx_gemm_weight_only_k_slices(const aqtx_gemm_plan* plan);
 
 /*
  * aqtx_ragged_prepare: what a ragged contraction (aqtx_gemm_plan.group_offsets) needs beside its operands:

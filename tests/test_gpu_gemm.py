@@ -1,4 +1,6 @@
 """GPU parity: aqtx_gemm_i8 against exact integer arithmetic and the oracle's dequant."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -468,6 +470,45 @@ def test_weight_only_gemm_within_float_summation_error(gpu, batch, m, n, k, w_sd
   got = got.float().cpu().numpy().astype(np.float64)
   assert ((low <= got) & (got <= high)).all(), np.argwhere((got < low) | (got > high))[:8]
   assert (got == want).mean() >= 0.99
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('layout', ['rows', 'fragments'])
+@pytest.mark.parametrize('w_sdt', ['bf16', 'f32'])
+@pytest.mark.parametrize('batch,m,n,k,slices', [(1, 1, 3, 6144, 16), (1, 65, 136, 6160, 16), (1, 129, 258, 8208, 16), (2, 200, 264, 6176, 16),
+                                                (1, 1024, 2048, 6144, 4), (1, 1025, 2048, 6144, 1), (1, 65, 136, 6128, 1)])
+def test_weight_only_gemm_in_slices_of_k(gpu, batch, m, n, k, slices, w_sdt, layout):
+  """Float32 sums of slices, added in slice order: within the bound of a float32 sum of k products in any order,
+  k * 2^-24 * sum |a b|, of the exact sum (float64), the later steps being monotone; both sides of the rule for slices, ragged
+  edges of the 128 x 256 tiles, a last slice that is shorter and no multiple of a stage of 64 k.  The call without slices
+  is held to the same interval."""
+  if layout == 'fragments' and batch > 1:
+    pytest.skip('fragment order is one weight')
+  g = torch.Generator(device=gpu).manual_seed(13)
+  a = torch.randn(batch, m, k, device=gpu, generator=g).to(torch.bfloat16)
+  b = torch.randint(-128, 128, (batch, n, k), dtype=torch.int8, device=gpu, generator=g)
+  cs = (torch.rand(batch, n, device=gpu, generator=g) * 0.01 + 1e-4).to(U.TORCH_DT[w_sdt]).float()
+  plan = L.GemmPlan()
+  plan.batch, plan.m, plan.n, plan.k = batch, m, n, k
+  assert L.lib().aqtx_gemm_weight_only_k_slices(ctypes.byref(plan)) == slices
+  kw = dict(col_scale_dtype=U.TORCH_DT[w_sdt])
+  w = b
+  if layout == 'fragments':
+    w, kw['b_layout'] = ops.tile_weight(b[0], L.I8), L.W_FRAGMENTS
+  sample = torch.randperm(m, generator=torch.Generator().manual_seed(1))[:130].sort().values.to(gpu)
+  ad = a[:, sample].double()
+  exact = torch.stack([ad[i] @ b[i].double().T for i in range(batch)])
+  slack = k * 2.0 ** -24 * torch.stack([ad[i].abs() @ b[i].double().abs().T for i in range(batch)])
+
+  def later_steps(total):
+    prod = total.float().to(torch.bfloat16).double() * cs.double()[:, None, :]
+    return prod.float().to(U.TORCH_DT[w_sdt]).to(torch.bfloat16).double()
+
+  low, high = later_steps(exact - slack), later_steps(exact + slack)
+  for tuning in (0, 128):
+    got = ops.gemm_weight_only(a, w, cs, tuning=tuning, **kw)[:, sample].double()
+    assert bool(((low <= got) & (got <= high)).all())
+    assert (got == later_steps(exact)).double().mean() >= 0.99
 
 
 @pytest.mark.gpu
