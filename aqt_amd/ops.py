@@ -114,9 +114,26 @@ def private_workspaces(store: dict):
     _QUANT_WS = prev
 
 
+def recording_workspaces(warm: dict, stream: int) -> dict:
+  """A store for a recording of calls that a first pass, on the stream with handle `stream`, made with the store `warm`: the
+  abs-max workspaces it will ask for, cleared now and not, by a launch of its own, in every replay (each call leaves them zero;
+  4 to 5 us of a replay).  The serving contraction's are left to the recording, which clears them: a call that gives up
+  waiting leaves words behind."""
+  out = {}
+  for key, ws in warm.items():
+    if key[0] != 'decode':
+      # (other streams that the recorded calls fork to are the same ones in both passes)
+      out[(key[0], 'recording') if key[1] == stream else key] = torch.zeros_like(ws)
+  return out
+
+
 def _quantize_workspace(nbytes: int, device) -> torch.Tensor:
   key = (device.index, _raw_stream(device.index))
   ws = _QUANT_WS.get(key)
+  if ws is None:
+    ws = _QUANT_WS.pop((device.index, 'recording'), None)  # the first stream a recording asks on is its own
+    if ws is not None:
+      _QUANT_WS[key] = ws
   if ws is None or ws.numel() < 2 * nbytes:
     # twice what the scales need: room for the arrival counts of the abs-max blocks (aqtx_quant_plan.workspace_zeroed)
     ws = torch.zeros(max(2 * nbytes, 1 << 20), dtype=torch.uint8, device=device)

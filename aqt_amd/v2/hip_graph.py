@@ -56,16 +56,16 @@ class GraphedCall:
         raise ValueError('GraphedCall: tensor arguments must live on the GPU')
     # A first pass on a side stream, as torch.cuda.graph requires, so that the recording finds
     # torch's allocator warm and this library's one-time work (kernel-layout copies of frozen
-    # weights) done.  The abs-max workspaces of the recorded kernels belong to this graph: they
-    # are allocated, and cleared, inside the recording.
-    side = torch.cuda.Stream()
+    # weights) done.  The workspaces of the recorded kernels belong to this graph.
+    side, warm = torch.cuda.Stream(), {}
     side.wait_stream(torch.cuda.current_stream())
-    with torch.cuda.stream(side), torch.no_grad(), ops.private_workspaces({}):
+    with torch.cuda.stream(side), torch.no_grad(), ops.private_workspaces(warm):
       for _ in range(max(1, warmup)):
         fn(*self._inputs)
     torch.cuda.current_stream().wait_stream(side)
+    self._workspaces = ops.recording_workspaces(warm, side.cuda_stream)
+    del warm
     torch.cuda.synchronize()
-    self._workspaces = {}
     self._graph = torch.cuda.CUDAGraph()
     with torch.no_grad(), ops.private_workspaces(self._workspaces), torch.cuda.graph(self._graph):
       self._outputs = fn(*self._inputs)
@@ -117,14 +117,15 @@ class GraphedStep:
   def __init__(self, fn: Callable, warmup: int = 3):
     if not torch.cuda.is_available():
       raise RuntimeError('GraphedStep needs a GPU')
-    side = torch.cuda.Stream()
+    side, warm = torch.cuda.Stream(), {}
     side.wait_stream(torch.cuda.current_stream())
-    with torch.cuda.stream(side), ops.private_workspaces({}):
+    with torch.cuda.stream(side), ops.private_workspaces(warm):
       for _ in range(max(1, warmup)):
         fn()
     torch.cuda.current_stream().wait_stream(side)
+    self._workspaces = ops.recording_workspaces(warm, side.cuda_stream)
+    del warm
     torch.cuda.synchronize()
-    self._workspaces = {}
     self._graph = torch.cuda.CUDAGraph()
     with ops.private_workspaces(self._workspaces), torch.cuda.graph(self._graph):
       self._outputs = fn()

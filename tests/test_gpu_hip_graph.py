@@ -6,6 +6,7 @@ synchronisations) between the replays, and every replay is compared with the eag
 import pytest
 import torch
 
+from aqt_amd import ops
 from aqt_amd.v2 import aqt_dot_general as aqt
 from aqt_amd.v2 import config
 from aqt_amd.v2 import hip_graph
@@ -203,3 +204,38 @@ def test_training_step_with_a_key_on_the_device_replays(gpu):
     torch.cuda.synchronize()
     for name, a, b in zip(('out', 'dlhs', 'drhs'), got, want):
       assert torch.equal(a, b), f'{name} of the replay differs from the eager step'
+
+
+@pytest.mark.parametrize('fork', [False, True])
+def test_recording_takes_workspaces_cleared_before_it(gpu, fork):
+  """Abs-max words (whole-tensor scales of many blocks) in a workspace that no launch of the recording clears: zero when
+  recorded, left zero by every replay, one a stream where the call forks; eager calls between the replays."""
+  from aqt_amd import _lib as L
+  other = torch.cuda.Stream()
+  kw = dict(reduce=L.REDUCE_ALL, out_dtype=L.I8, quant_bound=127.5, clip_bound=127.0)
+
+  def call(x):
+    if fork:
+      other.wait_stream(torch.cuda.current_stream())
+      with torch.cuda.stream(other):
+        y = ops.quantize(x * 2, **kw)
+    z = ops.quantize(x, **kw)
+    if fork:
+      torch.cuda.current_stream().wait_stream(other)
+      return z + y
+    return z
+
+  x = torch.randn(1, 1024, 512, device=gpu)
+  graphed = hip_graph.GraphedCall(call, x)
+  stores = [ws for key, ws in graphed._workspaces.items() if key[0] != 'decode']
+  assert len(stores) == (2 if fork else 1) and not any(key[1] == 'recording' for key in graphed._workspaces)
+  for seed in range(4):
+    x = torch.randn(1, 1024, 512, device=gpu, generator=torch.Generator(device=gpu).manual_seed(seed)) * (seed + 1)
+    got = graphed(x)
+    want = call(x)
+    for a, b in zip(got, want):
+      assert torch.equal(a, b)
+    torch.cuda.synchronize()
+    for ws in stores:
+      half = ws[:ws.numel() // 2]  # (the other half holds reciprocal scales)
+      assert int(half.count_nonzero()) == 0
