@@ -287,7 +287,7 @@ __global__ __launch_bounds__(256) void decode_fused_kernel(const DecodeArgs d) {
 
 // ---- a few more rows: the same, on 16 waves --------------------------------------------------------
 // Quantizing ROWS rows in every workgroup is vector work (about 8 instructions per value), and a wave
-// issues a vector instruction only every ~12 cycles: with the four waves of the kernel above it
+// alone on its SIMD issues one only every 2.1 ns or so: with the four waves of the kernel above it
 // takes longer than the weight stream it is meant to hide under.  Here a workgroup has 16 waves:
 // all of them quantize (a row is shared by 256 threads, four rows at a time), waves 0..3 alone
 // request the weights (before the quantisation) and contract.  Rows are written to LDS as in the

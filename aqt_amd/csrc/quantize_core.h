@@ -476,7 +476,7 @@ template <typename TIn, int W> __device__ __forceinline__ void once_unpack(const
 // threefry blocks; requires whole rows as segments and the natural noise layout.
 // A block is 256 threads, or 512 (LANES = 512: one long segment per block, half the row values per
 // thread, so that six waves fit a SIMD: the stochastic pipeline is bound by vector instruction
-// issue, and a wave issues one such instruction every ~12 cycles at best).
+// issue: one in 2.1 ns from a lone wave, in 1.1 to 1.8 from several).
 // The bound of four waves a SIMD goes to pipelines that fit 128 registers.  int8 values of the bf16 pipelines, held as
 // floats, do not: two paired rows of eight pieces need 182, and spill 196 bytes a lane under the bound (300 rows of 9000
 // with noise: 17.7 us, 12.8 without it; 2048 of 16384: 59 and 55).
