@@ -72,7 +72,7 @@ struct QArgs {
 // without the maxima: 62 us with 256 blocks, 40 with 512, 30 with 1024).
 constexpr int64_t kColmaxBlocks = 7 * 256;
 
-constexpr int kTileR = 128, kTileC = 64, kTilePad = 132;
+constexpr int kTileR = 128, kTileC = 64;
 
 // Column abs-max: a block takes 64 lanes x 8 columns (1 where there are fewer than 8) and 64 rows of them.
 constexpr int kAbsRowChunk = 64, kAbsColLanes = 64;
@@ -1106,25 +1106,27 @@ __global__ __launch_bounds__(1024) void quant_cols_once_kernel(const QArgs a, co
   }
 }
 
-// 128x64 tile: thread (rg = tid/8, cc = tid%8) owns rows 4*rg..+3, cols 8*cc..+7.
+// 128x64 tile: thread (rg = tid/8, cc = tid%8) owns rows 4*rg..+3, cols 8*cc..+7; with RPT = 1, a 32x64 tile and one row.
 // PAIR (SPEC 2 and 7, and SPEC 5 with value 1): 1 = the block also owns the tile `rows/2` further down (natural noise
 // layout), 2 = the tile `cols/2` further right (noise counters of the transposed tensor); the
 // two tiles' elements share threefry blocks.
 // ROWMAX (no PAIR; every tile interior): the block also finds, for each of its 128 rows, the largest |q| among its 64
 // columns, and stores them as bytes rows r0.. of row blockIdx.x of QArgs::oa_out ([column tiles][rows]).
-template <typename TIn, int SPEC, int PAIR, bool ROWMAX = false>
+template <typename TIn, int SPEC, int PAIR, bool ROWMAX = false, int RPT = 4>
 __global__ __launch_bounds__(256) void quant_tile_kernel(const QArgs a_in) {
-  static_assert(!ROWMAX || PAIR == 0, "row maxima: one tile per block");
+  static_assert(!ROWMAX || (PAIR == 0 && RPT == 4), "row maxima: one tile per block");
+  static_assert(RPT == 4 || RPT == 1, "rows a thread");
+  constexpr int TR = 32 * RPT, TPAD = TR + 4;  // rows of the tile; LDS bytes a column
   const QArgs a = with_device_key(a_in);
   constexpr int NSET = PAIR ? 2 : 1;
-  __shared__ uint32_t lds[NSET][kTileC * kTilePad / 4];
+  __shared__ uint32_t lds[NSET][kTileC * TPAD / 4];
   const int tid = threadIdx.x;
   const int cc = tid & 7, rg = tid >> 3;
   const int64_t b = blockIdx.z;
   const TIn* xb = reinterpret_cast<const TIn*>(a.x) + b * a.rows * a.cols;
   uint8_t* qb = reinterpret_cast<uint8_t*>(a.q) + b * a.rows * a.cols;
   int64_t r0[NSET], c0[NSET];
-  r0[0] = (int64_t)blockIdx.y * kTileR;
+  r0[0] = (int64_t)blockIdx.y * TR;
   c0[0] = (int64_t)blockIdx.x * kTileC;
   // the first tile of a pair stays inside the first half of the paired axis
   const int64_t row_lim = PAIR == 1 ? a.rows / 2 : a.rows;
@@ -1133,20 +1135,20 @@ __global__ __launch_bounds__(256) void quant_tile_kernel(const QArgs a_in) {
   // that every tile of a tensor of at least one tile takes the branch-free path.  SPEC 5 draws for pairs of columns
   // that start at an even one.  (1999 x 1030, 1999 x 3001 and 1030 x 3001 values with byte and element accesses on every
   // tile: 24, 36 and 18 us, the first two with noise; now 15, 26 and 7.)
-  if (r0[0] + kTileR > row_lim && row_lim >= kTileR) r0[0] = row_lim - kTileR;
+  if (r0[0] + TR > row_lim && row_lim >= TR) r0[0] = row_lim - TR;
   if (c0[0] + kTileC > col_lim && col_lim >= kTileC && (SPEC != 5 || col_lim % 2 == 0)) c0[0] = col_lim - kTileC;
   if constexpr (PAIR == 1) { r0[1] = r0[0] + a.rows / 2; c0[1] = c0[0]; }
   if constexpr (PAIR == 2) { r0[1] = r0[0]; c0[1] = c0[0] + a.cols / 2; }
 
-  uint32_t words[NSET][2][4];  // words[s][h][j] = bytes of cols c+4*h..c+4*h+3 at row 4*rg+j
+  uint32_t words[NSET][2][RPT];  // words[s][h][j] = bytes of cols c+4*h..c+4*h+3 at row RPT*rg+j
 #pragma unroll
   for (int s = 0; s < NSET; ++s)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) words[s][0][j] = words[s][1][j] = 0u;
+    for (int j = 0; j < RPT; ++j) words[s][0][j] = words[s][1][j] = 0u;
 
   // Tiles that lie wholly inside the tensor (and inside the first half of a paired axis) take a
   // branch-free path with vector loads of the reciprocal scales and the pre-scale factors.
-  const bool interior = (r0[0] + kTileR <= row_lim) && (c0[0] + kTileC <= col_lim) && a.ssc <= 1;
+  const bool interior = (r0[0] + TR <= row_lim) && (c0[0] + kTileC <= col_lim) && a.ssc <= 1;
   // Every lane of the tile that has values has eight: one decision for the tile, before each lane's own (64 x 64 values
   // with noise and one scale 15.3 us; 18.8 with the lanes' decision alone).
   const bool whole = a.cols % 8 == 0 && col_lim % 8 == 0;
@@ -1174,15 +1176,15 @@ __global__ __launch_bounds__(256) void quant_tile_kernel(const QArgs a_in) {
       }
     }
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int64_t rl = r0[0] + rg * 4 + j;  // position inside the first tile's half
+    for (int j = 0; j < RPT; ++j) {
+      const int64_t rl = r0[0] + rg * RPT + j;  // position inside the first tile's half
       const int64_t cl = c0[0] + cc * 8;
       if (FAST || (rl < row_lim && cl < col_lim)) {
         const int nvalid = FAST ? 8 : ((col_lim - cl) >= 8 ? 8 : (int)(col_lim - cl));
         float x[NSET][8], inv[NSET][8];
 #pragma unroll
         for (int s = 0; s < NSET; ++s) {
-          const int64_t r = r0[s] + rg * 4 + j, c = c0[s] + cc * 8;
+          const int64_t r = r0[s] + rg * RPT + j, c = c0[s] + cc * 8;
           if (FAST || whole) {
             Loader<TIn>::load8(xb + r * a.cols + c, x[s]);
           } else if (nvalid == 8) {
@@ -1251,7 +1253,7 @@ __global__ __launch_bounds__(256) void quant_tile_kernel(const QArgs a_in) {
                 qv[s] = spec_finish<5>(t, a);
               }
             } else if constexpr (PAIR) {
-              const uint32_t i = (uint32_t)((r0[0] + rg * 4 + j) * a.nsr + (c0[0] + cc * 8 + e) * a.nsc);
+              const uint32_t i = (uint32_t)((r0[0] + rg * RPT + j) * a.nsr + (c0[0] + cc * 8 + e) * a.nsc);
               pair_quant<SPEC>(x[0][e], inv[0][e], x[1][e], inv[1][e], i, a, qv[0], qv[1]);
             } else if constexpr (ROWMAX) {
               float tc;
@@ -1282,7 +1284,7 @@ __global__ __launch_bounds__(256) void quant_tile_kernel(const QArgs a_in) {
         if (!a.transpose_out) {
 #pragma unroll
           for (int s = 0; s < NSET; ++s) {
-            const int64_t r = r0[s] + rg * 4 + j, c = c0[s] + cc * 8;
+            const int64_t r = r0[s] + rg * RPT + j, c = c0[s] + cc * 8;
             if (FAST || whole) {
               store8(qb + r * a.cols + c, make_uint2(w[s][0], w[s][1]));
             } else if (nvalid == 8) {
@@ -1304,30 +1306,37 @@ __global__ __launch_bounds__(256) void quant_tile_kernel(const QArgs a_in) {
   }
   if (!a.transpose_out) return;  // uniform across the block
 
-  // Transposed write: LDS holds each tile as [col][row bytes], row stride 132 B.
+  // Transposed write: LDS holds each tile as [col][row bytes], row stride TPAD B.
 #pragma unroll
   for (int s = 0; s < NSET; ++s)
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      uint32_t col4[4];
-      transpose4(words[s][h], col4);
+      if constexpr (RPT == 4) {
+        uint32_t col4[4];
+        transpose4(words[s][h], col4);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) lds[s][((cc * 8 + 4 * h + e) * kTilePad + rg * 4) / 4] = col4[e];
+        for (int e = 0; e < 4; ++e) lds[s][((cc * 8 + 4 * h + e) * TPAD + rg * 4) / 4] = col4[e];
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          reinterpret_cast<uint8_t*>(lds[s])[(cc * 8 + 4 * h + e) * TPAD + rg] = (uint8_t)(words[s][h][0] >> (8 * e));
+      }
     }
   __syncthreads();
-  // thread -> (col = tid/8 + 32*h, 16-byte chunk = tid%8) of the [64][128] byte tile
+  // thread -> 16-byte chunks of the [64][TR] byte tile
+  constexpr int CH = TR / 16, ITEMS = kTileC * CH;
 #pragma unroll
   for (int s = 0; s < NSET; ++s) {
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int col = (tid >> 3) + 32 * h;
-      const int chunk = tid & 7;
+    for (int h = 0; h < (ITEMS + 255) / 256; ++h) {
+      if (ITEMS < 256 && tid >= ITEMS) break;
+      const int col = (tid + 256 * h) / CH, chunk = (tid + 256 * h) % CH;
       const int64_t gc_l = c0[0] + col, gr_l = r0[0] + chunk * 16;  // bounds in first-tile terms
       const int64_t gc = c0[s] + col, gr = r0[s] + chunk * 16;
       if (gc_l < col_lim && gr_l < row_lim) {
         uint32_t w[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) w[i] = lds[s][(col * kTilePad + chunk * 16) / 4 + i];
+        for (int i = 0; i < 4; ++i) w[i] = lds[s][(col * TPAD + chunk * 16) / 4 + i];
         uint8_t* dst = qb + gc * a.rows + gr;
         const int64_t lim = row_lim - gr_l;
         if (lim >= 16) {
@@ -1544,16 +1553,40 @@ int launch_tiles(const QArgs& a, int reduce, int partitionable, int64_t nscales,
     return dim3((unsigned)((cols + kTileC - 1) / kTileC), (unsigned)((rows + kTileR - 1) / kTileR),
                 (unsigned)a.batch);
   };
+  auto low_grid_for = [&](int pair) {
+    const int64_t rows = pair == 1 ? a.rows / 2 : a.rows;
+    dim3 g = grid_for(pair);
+    g.y = (unsigned)((rows + kTileR / 4 - 1) / (kTileR / 4));
+    return g;
+  };
+  // With noise a thread's values are a serial chain of a hundred instructions each, so few tiles are cut to 32 rows, for four
+  // times the waves.  Float32 values up to two tall tiles a CU, narrower ones up to eight; where HBM bounds the large ones the
+  // short rows of a transposed tile lose.  Calibrated and quantized, tall / low, us:
+  //   bf16     64 x 64 14.2 / 7.0, 512 x 1024 14.5 / 8.9, 1024 x 2048 15.4 / 11.0, 2048 x 2048 16.6 / 14.4,
+  //            4096 x 4096 36.9 / 35.1, 8192 x 4096 (2048 tiles) 61.0 / 59.4; to fp8 64 x 64 17.8 / 7.4,
+  //            2048 x 2048 19.8 / 14.1, 8192 x 4096 57.9 / 53.6, 8192 x 14336 168 / 198
+  //   int8     512 x 1024 15.4 / 9.9, 4096 x 4096 38.6 / 37.1, 8192 x 4096 60.9 / 58.8, two entries of it (8192 tiles) 164 / 166
+  //   float32  64 x 64 16.4 / 7.4, 1024 x 2048 15.9 / 11.5, 1999 x 3001 32.0 / 28.4, 2048 x 4096 (512 tiles) 27.8 / 27.5, 4096 x 4096 39.9 / 41.0,
+  //            8192 x 14336 249 / 296
+  auto low = [&](int pair) {
+    const dim3 g = grid_for(pair);
+    return (int64_t)g.x * g.y * g.z <= (sizeof(TIn) == 4 ? 512 : 2048);
+  };
 #define AQTX_TILE(SPEC, PAIR, ...) quant_tile_kernel<TIn, SPEC, PAIR, ##__VA_ARGS__><<<grid_for(PAIR), 256, 0, st>>>(a)
+#define AQTX_NOISE_TILE(SPEC, PAIR)                                                                        \
+  {                                                                                                      \
+    if (low(PAIR)) quant_tile_kernel<TIn, SPEC, PAIR, false, 1><<<low_grid_for(PAIR), 256, 0, st>>>(a);  \
+    else AQTX_TILE(SPEC, PAIR);                                                                          \
+  }
   // pair the two elements of each threefry block: i and i + total/2 lie rows/2 apart when the noise counters are
   // row-major over [rows, cols], cols/2 apart when over [cols, rows]
   auto uniform = [&](auto tag) {
     constexpr int S = decltype(tag)::value;
     const bool natural = a.batch == 1 && a.nsc == 1 && a.nsr == a.cols && (a.rows % 2 == 0);
     const bool transposed = a.batch == 1 && a.nsr == 1 && a.nsc == a.rows && (a.cols % 2 == 0);
-    if (natural) AQTX_TILE(S, 1);
-    else if (transposed) AQTX_TILE(S, 2);
-    else AQTX_TILE(S, 0);
+    if (natural) AQTX_NOISE_TILE(S, 1)
+    else if (transposed) AQTX_NOISE_TILE(S, 2)
+    else AQTX_NOISE_TILE(S, 0)
   };
   bool done = false;  // (oa_out: the caller has checked tiles_rowmax_ok: noise none, so spec is 1, 6 or 0)
   if constexpr (sizeof(TIn) != 4) {  // the bf16 pipelines
@@ -1570,8 +1603,8 @@ int launch_tiles(const QArgs& a, int reduce, int partitionable, int64_t nscales,
       // half of a threefry block would be thrown away unless the tile rows/2 further down, whose elements draw
       // from the other half, is quantized by the same workgroup
       const bool natural = a.batch == 1 && a.nsr == a.cols && (a.rows % 2 == 0);
-      if (natural) AQTX_TILE(5, 1);
-      else AQTX_TILE(5, 0);
+      if (natural) AQTX_NOISE_TILE(5, 1)
+      else AQTX_NOISE_TILE(5, 0)
     } else {
       done = false;
     }
@@ -1589,6 +1622,7 @@ int launch_tiles(const QArgs& a, int reduce, int partitionable, int64_t nscales,
     if (a.oa_out != nullptr) AQTX_TILE(0, 0, true);
     else AQTX_TILE(0, 0);
   }
+#undef AQTX_NOISE_TILE
 #undef AQTX_TILE
   AQTX_HIP_CHECK_LAUNCH("quant_tile_kernel");
   return 0;

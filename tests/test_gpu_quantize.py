@@ -344,6 +344,34 @@ def test_float32_pipelines_match_the_oracle(gpu, reduce, rows, cols, noise):
   _check(qt, qg.cpu().numpy(), sg.cpu().numpy(), q)
 
 
+@pytest.mark.parametrize('dt,batch,rows,cols', [
+    # around tiles of 32 x 64, halved where two tiles share the blocks of the generator; entries that do not pair
+    *[(dt, *s) for dt in ('bf16', 'f32') for s in ((1, 31, 64), (1, 32, 128), (1, 62, 70), (1, 64, 126), (1, 66, 130), (1, 254, 58),
+                                                   (2, 32, 64), (3, 33, 63), (2, 65, 57))],
+    # the last and the first sizes on either side of the line to tall tiles
+    ('f32', 1, 2 * 128 * 512, 9), ('f32', 1, 2 * 128 * 512 + 2, 9), ('bf16', 1, 2 * 128 * 2048, 9), ('bf16', 1, 2 * 128 * 2048 + 2, 9),
+])
+@pytest.mark.parametrize('bits', [8, 'e5m2'])
+def test_tiles_with_noise_low_and_tall(gpu, bits, dt, batch, rows, cols):
+  """Scales by column, with noise counters in memory order (both output orders) and, integers, in that of the transposed tensor."""
+  key = prng.prng_key(rows + cols)
+  q = R.QuantizerCfg(bits=bits, key=key, **({'noise': 'jax.uniform'} if bits == 8 else {'fp8_sr': True}))
+  qb, cb = U.bounds(q)
+  kw = dict(reduce=L.REDUCE_ROWS, out_dtype=U.OUT_DT[bits], quant_bound=qb, clip_bound=cb,
+            noise=L.NOISE_JAX_UNIFORM if bits == 8 else L.NOISE_FP8_MANTISSA, key=key)
+  x = U.rand((batch, rows, cols), dt, seed=rows + cols, outliers=True)
+  qt = R.quantize(x, dt, q, [1])
+  for transpose in (True, False):
+    qg, sg = ops.quantize(U.to_dev(x, dt, gpu), transpose_out=transpose, **kw)
+    _check(qt, qg.cpu().numpy(), sg.cpu().numpy(), q, transpose=transpose)
+  if bits == 8 and batch == 1:
+    w = np.random.default_rng(rows).integers(-127, 128, size=(cols, rows)).astype(np.int8)  # logical [cols, rows]
+    qt = R.quantize(w.astype(np.float32)[None], dt, q, [2])
+    qg, sg = ops.quantize(torch.from_numpy(np.ascontiguousarray(w.T)[None]).to(gpu), compute_dtype=U.TORCH_DT[dt],
+                          noise_strides=(rows * cols, 1, rows), noise_total=rows * cols, transpose_out=True, **kw)
+    _check(qt, qg.cpu().numpy(), sg.cpu().numpy(), q)
+
+
 @pytest.mark.parametrize('rows,cols', [
     # around the pieces of 8, the launch shapes of the rows kernel and the 128 x 64 tiles (halved where two tiles share
     # the blocks of the generator); fewer than a piece or a tile
