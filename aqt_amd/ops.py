@@ -114,7 +114,17 @@ def private_workspaces(store: dict):
     _QUANT_WS = prev
 
 
-def recording_workspaces(warm: dict, stream: int) -> dict:
+class RecordingWorkspaces(dict):
+  """A store of workspaces for a recording.  `cleared` keeps those it was made with for as long as it lives: launches recorded
+  with one hold its address, and they come from torch's general pool, not the graph's, so that one which a later call on its
+  stream outgrew, or that went with the table after a failed launch, would be somebody else's memory in the replays."""
+
+  def __init__(self, items=()):
+    super().__init__(items)
+    self.cleared = tuple(self.values())
+
+
+def recording_workspaces(warm: dict, stream: int) -> RecordingWorkspaces:
   """A store for a recording of calls that a first pass, on the stream with handle `stream`, made with the store `warm`: the
   abs-max workspaces it will ask for, cleared now and not, by a launch of its own, in every replay (each call leaves them zero;
   4 to 5 us of a replay).  The serving contraction's are left to the recording, which clears them: a call that gives up
@@ -122,16 +132,17 @@ def recording_workspaces(warm: dict, stream: int) -> dict:
   out = {}
   for key, ws in warm.items():
     if key[0] != 'decode':
-      # (other streams that the recorded calls fork to are the same ones in both passes)
+      # (a stream that the recorded calls fork to finds its workspace if it is the one of the first pass; else, or where a call
+      # asks for more, one is made in the recording, which then clears it in every replay)
       out[(key[0], 'recording') if key[1] == stream else key] = torch.zeros_like(ws)
-  return out
+  return RecordingWorkspaces(out)
 
 
 def _quantize_workspace(nbytes: int, device) -> torch.Tensor:
   key = (device.index, _raw_stream(device.index))
   ws = _QUANT_WS.get(key)
   if ws is None:
-    ws = _QUANT_WS.pop((device.index, 'recording'), None)  # the first stream a recording asks on is its own
+    ws = _QUANT_WS.pop((device.index, 'recording'), None)  # (the first stream a recording asks on)
     if ws is not None:
       _QUANT_WS[key] = ws
   if ws is None or ws.numel() < 2 * nbytes:

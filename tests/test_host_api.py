@@ -407,3 +407,35 @@ def test_copies_of_settings_ask_the_class():
   x = Slotted()
   x.more = 3
   assert utils.clone_fields(x).more == 3 and utils.clone_fields(x).n == 1
+
+
+@pytest.mark.parametrize('how', ['outgrown', 'outgrown on a stream of its own', 'table emptied'])
+def test_a_recording_keeps_the_workspaces_it_was_made_with(monkeypatch, how):
+  """Launches recorded with a workspace write to it in every replay: it stays owned where a later call asks for a larger one,
+  also on a stream that the first pass did not use, and where a failed launch empties the table."""
+  import gc
+  import weakref
+  from aqt_amd import ops
+  handle = [1]
+  monkeypatch.setattr(ops, '_raw_stream', lambda index: handle[0])
+  device, warm = torch.device('cpu'), {}
+  with ops.private_workspaces(warm):
+    ops._quantize_workspace(64, device)
+  store = ops.recording_workspaces(warm, stream=1)
+  handle[0] = 3 if how == 'outgrown on a stream of its own' else 2
+  with ops.private_workspaces(store):
+    first = ops._quantize_workspace(64, device)
+    assert int(first.count_nonzero()) == 0
+    recorded, address = weakref.ref(first), first.data_ptr()
+    del first
+    if how == 'table emptied':
+      ops._QUANT_WS.clear()
+    larger = ops._quantize_workspace(4 << 20, device)
+    handle[0] = 2
+    again = ops._quantize_workspace(64, device)
+  gc.collect()
+  assert recorded() is not None and recorded().data_ptr() == address
+  assert larger.numel() >= 8 << 20 and address not in (larger.data_ptr(), again.data_ptr())
+  del store, larger, again
+  gc.collect()
+  assert recorded() is None  # given back with the recording
