@@ -122,6 +122,14 @@ class RecordingWorkspaces(dict):
   def __init__(self, items=()):
     super().__init__(items)
     self.cleared = tuple(self.values())
+    self._made_on = tuple(_raw_stream(ws.device.index) for ws in self.cleared)
+
+  def used_on_current_stream(self):
+    """To be called for a replay: on a stream other than the one the tensors were made on, torch has to know of the use, or
+    it hands their memory on when the recording goes while the replay is under way."""
+    for ws, made_on in zip(self.cleared, self._made_on):
+      if _raw_stream(ws.device.index) != made_on:
+        ws.record_stream(torch.cuda.current_stream(ws.device))
 
 
 def recording_workspaces(warm: dict, stream: int) -> RecordingWorkspaces:

@@ -86,6 +86,7 @@ class GraphedCall:
     return self._outputs
 
   def replay(self):
+    self._workspaces.used_on_current_stream()
     self._graph.replay()
     return self._outputs
 
@@ -135,5 +136,6 @@ class GraphedStep:
     return self._outputs
 
   def replay(self):
+    self._workspaces.used_on_current_stream()
     self._graph.replay()
     return self._outputs

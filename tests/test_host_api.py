@@ -439,3 +439,35 @@ def test_a_recording_keeps_the_workspaces_it_was_made_with(monkeypatch, how):
   del store, larger, again
   gc.collect()
   assert recorded() is None  # given back with the recording
+
+
+def test_a_replay_on_another_stream_tells_the_allocator(monkeypatch):
+  """The workspaces of a recording come from torch's general pool: dropped while a replay runs on a stream other than the one
+  they were made on, their memory must wait for it."""
+  from aqt_amd import ops
+  from aqt_amd.v2 import hip_graph
+
+  class Workspace(torch.Tensor):
+    used_on = []
+
+    def record_stream(self, stream):
+      self.used_on.append(stream)
+
+  class Graph:
+    replays = 0
+
+    def replay(self):
+      self.replays += 1
+
+  handle = [5]
+  monkeypatch.setattr(ops, '_raw_stream', lambda index: handle[0])
+  monkeypatch.setattr(torch.cuda, 'current_stream', lambda device=None: f'stream {handle[0]}')
+  for cls in (hip_graph.GraphedCall, hip_graph.GraphedStep):
+    Workspace.used_on.clear()
+    handle[0] = 5
+    graphed = object.__new__(cls)
+    graphed._graph, graphed._outputs = Graph(), 'outputs'
+    graphed._workspaces = ops.RecordingWorkspaces({(0, 'recording'): torch.zeros(8).as_subclass(Workspace)})
+    assert graphed.replay() == 'outputs' and Workspace.used_on == []
+    handle[0] = 6
+    assert graphed.replay() == 'outputs' and Workspace.used_on == ['stream 6'] and graphed._graph.replays == 2
