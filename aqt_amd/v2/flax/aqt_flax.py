@@ -253,12 +253,15 @@ class AqtDotGeneral(torch.nn.Module, _RngMixin):
 
     key = self.make_rng(self.prng_name) if self.prng_name is not None else None
     modes = dict(lhs_quant_mode=self.lhs_quant_mode, rhs_quant_mode=self.rhs_quant_mode)
-    settings, made = cfg, {}
+    settings, made = cfg, []
 
-    def with_context(fwd_only):
-      if fwd_only not in made:
-        made[fwd_only] = config.set_context(settings, key, train_step=None, copy_settings=False, fwd_only=fwd_only, **modes)
-      return made[fwd_only]
+    def with_context(lhs, rhs):
+      # One context a call: the tiled shortcut and the contraction it leaves to ret_dg share it (another would be another copy
+      # and another fan-out of the key, which is a launch where the key is on the device).
+      fwd_only = not (settings.apply_custom_vjp_on_jax and (lhs.requires_grad or rhs.requires_grad))
+      if not made or made[0][0] and not fwd_only:
+        made[:] = [(fwd_only, config.set_context(settings, key, train_step=None, copy_settings=False, fwd_only=fwd_only, **modes))]
+      return made[0][1]
 
     def ret_dg(lhs, rhs, dimension_numbers, precision=None, preferred_element_type=None):
       del preferred_element_type
@@ -268,7 +271,7 @@ class AqtDotGeneral(torch.nn.Module, _RngMixin):
       assert lhs.dtype in [utils.bfloat16, utils.float32, utils.float16], msg
       assert rhs.dtype in [utils.bfloat16, utils.float32, utils.float16], msg
       settings.assert_config_validity()
-      cfg = with_context(fwd_only=not (settings.apply_custom_vjp_on_jax and (lhs.requires_grad or rhs.requires_grad)))
+      cfg = with_context(lhs, rhs)
 
       lhs_qt = lhs_freezer.get() if self.lhs_apply_quant_mode else self.lhs_qtensor
       rhs_qt = rhs_freezer.get() if self.rhs_apply_quant_mode else self.rhs_qtensor
@@ -301,16 +304,16 @@ class AqtDotGeneral(torch.nn.Module, _RngMixin):
     def fused_tile_sum(tl, tr, tiled_dn, n_sum_axes):
       """tiled_dot_general's shortcut for a tiled contraction axis (contract, dequantize and sum the
       tiles in one kernel), with the same freezer traffic as ret_dg; None if it does not apply."""
-      if self.use_legacy_freezer:
-        return None
+      if self.use_legacy_freezer or torch.is_grad_enabled() and (tl.requires_grad or tr.requires_grad):
+        return None  # (DotGeneral.fused_tile_sum would say so for gradients, after a context made for a forward pass alone)
       lhs_qt = lhs_freezer.get() if self.lhs_apply_quant_mode else self.lhs_qtensor
       rhs_qt = rhs_freezer.get() if self.rhs_apply_quant_mode else self.rhs_qtensor
       # the quantized lhs values are only looked at when this call freezes them (Freezer.set stores
       # in CONVERT, and FreezerMode.CALIBRATION keeps the scales alone)
       lhs_values_kept = (self.lhs_apply_quant_mode and self.lhs_quant_mode == QuantMode.CONVERT
                          and self.lhs_freeze_mode != FreezerMode.CALIBRATION)
-      res = with_context(fwd_only=True).fused_tile_sum(tl, tr, tiled_dn, n_sum_axes, lhs_qt=lhs_qt, rhs_qt=rhs_qt, with_qt=True,
-                               lhs_qvalue_needed=lhs_values_kept)
+      res = with_context(tl, tr).fused_tile_sum(tl, tr, tiled_dn, n_sum_axes, lhs_qt=lhs_qt, rhs_qt=rhs_qt, with_qt=True,
+                                                lhs_qvalue_needed=lhs_values_kept)
       if res is None:
         return None
       out, (out_lhs_qt, out_rhs_qt) = res

@@ -108,3 +108,35 @@ def test_unquantized_layer_is_a_float_dot_general():
   l, r = torch.randn(4, 6), torch.randn(6, 5)
   out = dg(l, r, (((1,), (0,)), ((), ())), None)
   assert torch.allclose(out, l @ r, atol=1e-5)
+
+
+@pytest.mark.parametrize('grads', [True, False])
+@pytest.mark.parametrize('tiled', [True, False])
+def test_a_layer_call_makes_one_context(monkeypatch, grads, tiled):
+  """The key of a call is fanned out once (a launch where it is on the device) and the settings are copied twice, for the
+  context and for the calibrators; a tiled call that the one-kernel shortcut declines has no more of either."""
+  from aqt_amd.v2 import aqt_dot_general, config, tiled_dot_general
+  AxisTiling, TensorTiling = tiled_dot_general.AxisTiling, tiled_dot_general.TensorTiling
+  counts = {'fan_out': 0, 'copies': 0}
+
+  def counted(name, fn):
+    def call(*args, **kw):
+      counts[name] += 1
+      return fn(*args, **kw)
+    return call
+
+  monkeypatch.setattr(config, '_fan_out_key', counted('fan_out', config._fan_out_key))
+  monkeypatch.setattr(aqt_dot_general, 'clone_down_to_quantizers', counted('copies', aqt_dot_general.clone_down_to_quantizers))
+  tiling = tiled_dot_general.Cfg(lhs=TensorTiling([AxisTiling(axis=1, tile_size=4)], []),
+                                 rhs=TensorTiling([AxisTiling(axis=0, tile_size=4)], []))
+  cfg = config.dot_general_make(None, None)  # nothing quantized: runs here
+  layer = aqt_flax.AqtDotGeneral(cfg, tiling_cfg=tiling if tiled else None, use_legacy_freezer=False,
+                                 rngs={'params': utils.prng_key(0)})
+  x, w = torch.randn(6, 8, requires_grad=grads), torch.randn(8, 5, requires_grad=grads)
+  out = layer(x, w, (((1,), (0,)), ((), ())))
+  assert torch.allclose(out, x @ w, atol=1e-5) and out.requires_grad == grads
+  shortcut = 1 if tiled and not grads else 0  # (asked with a copy of its own, and declined here)
+  assert counts == {'fan_out': 1, 'copies': 2 + shortcut}
+  if grads:
+    out.sum().backward()
+    assert torch.allclose(w.grad, x.detach().sum(0)[:, None].expand(8, 5), atol=1e-5)
