@@ -471,3 +471,38 @@ def test_a_replay_on_another_stream_tells_the_allocator(monkeypatch):
     assert graphed.replay() == 'outputs' and Workspace.used_on == []
     handle[0] = 6
     assert graphed.replay() == 'outputs' and Workspace.used_on == ['stream 6'] and graphed._graph.replays == 2
+
+
+@pytest.mark.parametrize('raises', [False, True])
+def test_contractions_are_user_annotations_of_a_profile(tmp_path, raises):
+  """Forward and gradient contractions carry their jax_scope_name, recorded as torch.profiler.record_function records a
+  scope: a user annotation in a profile, a node of an execution trace; closed also where the contraction raises."""
+  import json
+  from torch.profiler import ExecutionTraceObserver, ProfilerActivity, profile
+  cfg = config.dot_general_make(None, None)
+  for raw, name in ((cfg.fwd, 'aqt_fwd'), (cfg.dlhs, 'aqt_dlhs'), (cfg.drhs, 'aqt_drhs')):
+    assert raw.jax_scope_name == name
+  x, w = torch.randn(4, 8, requires_grad=True), torch.randn(8, 3, requires_grad=True)
+
+  def call():
+    if not raises:
+      cfg(x, w, (((1,), (0,)), ((), ()))).sum().backward()
+      return
+    cfg.fwd.dot_general = None  # (not callable)
+    with pytest.raises(TypeError):
+      cfg(x, w, (((1,), (0,)), ((), ())))
+
+  want = {'aqt_fwd'} if raises else {'aqt_fwd', 'aqt_dlhs', 'aqt_drhs'}
+  with profile(activities=[ProfilerActivity.CPU]) as prof:
+    call()
+    with torch.profiler.record_function('outside'):
+      torch.zeros(1)
+  events = {e.name: e for e in prof.events() if e.is_user_annotation}
+  assert set(events) == want | {'outside'}
+  assert all(events['outside'].time_range.start >= events[name].time_range.end for name in want)
+  observer = ExecutionTraceObserver().register_callback(str(tmp_path / 'trace.json'))
+  observer.start()
+  call()
+  observer.stop()
+  observer.unregister_callback()
+  assert want <= {n['name'] for n in json.loads((tmp_path / 'trace.json').read_text())['nodes']}
