@@ -1669,10 +1669,30 @@ def _fresh_cfg(cfg: 'DotGeneral', fwd_only: bool = False) -> 'DotGeneral':
   return clone_down_to_quantizers(cfg, reset_calibrators=True, fwd_only=fwd_only)
 
 
+def _try_calibrators(cfg: DotGeneral) -> bool:
+  """Makes and initialises the gradient contractions' calibrators without keeping them (2 us, where copies of their objects
+  take 7): settings that cannot make them are refused, and a calibration of the user's own sees every call.  False, with
+  nothing made: quantizers of the user's own, whose init_calibration() wants a copy."""
+  quantizers = []
+  for raw in (cfg.dlhs, cfg.drhs):
+    dq = raw.dg_quantizer
+    if type(dq) is not DefaultDotGeneralQuantizer:
+      return False
+    quantizers += [dq.lhs, dq.rhs]
+    quantizers += [q for q, alpha in ((dq.lhs_mid, dq.lhs_mid_alpha), (dq.rhs_mid, dq.rhs_mid_alpha)) if alpha is not None]
+  if any(type(q) is not aqt_quantizer.Quantizer for q in quantizers):
+    return False
+  for q in quantizers:
+    if q.calibration is not None:
+      q.calibration(dtype=q.scale_dtype).init_calibration()
+  return True
+
+
 def dg_core_vjp_fwd(lhs, rhs, lhs_qt, rhs_qt, dimension_numbers, cfg: DotGeneral, *, fwd_only: bool = False):
   """Forward pass (aqt_dot_general.py:1098-1124).  fwd_only: for a caller that drops the residuals; the gradient
-  contractions' calibrators are not made (a layer served from Python: the copies were a quarter of a call's 124 us)."""
+  contractions' objects are not copied (a layer served from Python: the copies were a quarter of a call's 124 us)."""
   assert lhs.dtype == rhs.dtype, f'Unmatched lhs and rhs dtype: {lhs.dtype} vs {rhs.dtype}'
+  fwd_only = fwd_only and _try_calibrators(cfg)
   cfg = _fresh_cfg(cfg, fwd_only)
   cfg.fwd.dg_quantizer.init_calibration()
   if not fwd_only:

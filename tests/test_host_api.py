@@ -506,3 +506,39 @@ def test_contractions_are_user_annotations_of_a_profile(tmp_path, raises):
   observer.stop()
   observer.unregister_callback()
   assert want <= {n['name'] for n in json.loads((tmp_path / 'trace.json').read_text())['nodes']}
+
+
+def test_a_call_without_gradients_makes_the_calibrators_of_the_gradients():
+  """Their settings are refused, and a calibration or quantizer of the user's own is initialised, whether the operands want
+  gradients or not."""
+  import functools
+  made = []
+
+  class Counted(calibration.AbsMaxCalibration):
+    def init_calibration(self):
+      made.append(self.dtype)
+
+  class OwnQuantizer(aqt_quantizer.Quantizer):
+    def init_calibration(self):
+      made.append('own')
+
+  x, w = torch.randn(4, 8), torch.randn(8, 3)
+  run = lambda cfg, **kw: cfg(x, w.requires_grad_(kw.get('grads', False)), (((1,), (0,)), ((), ())))
+  for grads in (False, True):
+    cfg = config.dot_general_make(None, None)
+    cfg.dlhs.dg_quantizer.lhs.calibration = functools.partial(calibration.AbsMaxCalibration, no_such_setting=1)
+    with pytest.raises(TypeError, match='no_such_setting'):
+      run(cfg, grads=grads)
+    cfg = config.dot_general_make(None, None)
+    cfg.dlhs.dg_quantizer.lhs.calibration = cfg.drhs.dg_quantizer.rhs.calibration = Counted
+    cfg.drhs.dg_quantizer.rhs.scale_dtype = torch.float32
+    own = cfg.drhs.dg_quantizer.lhs
+    for _ in range(2):
+      made.clear()
+      run(cfg, grads=grads)
+      assert made == [None, torch.float32]
+    cfg.drhs.dg_quantizer.lhs = OwnQuantizer(**{f.name: getattr(own, f.name) for f in dataclasses.fields(own)})
+    made.clear()
+    run(cfg, grads=grads)
+    assert made == [None, 'own', torch.float32]
+    assert cfg.dlhs.dg_quantizer.lhs._calibrator is None
