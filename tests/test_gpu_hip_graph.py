@@ -239,3 +239,37 @@ def test_recording_takes_workspaces_cleared_before_it(gpu, fork):
     for ws in stores:
       half = ws[:ws.numel() // 2]  # (the other half holds reciprocal scales)
       assert int(half.count_nonzero()) == 0
+
+
+def test_recording_that_outgrows_the_workspace_of_its_first_pass(gpu):
+  """A stream made inside the call takes the workspace meant for the recording's own and then asks for a larger one: the
+  launches recorded with the first go on using it, and nobody else gets its memory."""
+  from aqt_amd import _lib as L
+  kw = dict(out_dtype=L.I8, quant_bound=127.5, clip_bound=127.0)
+
+  def call(x, many):
+    fork = torch.cuda.Stream()
+    fork.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(fork):
+      y = ops.quantize(x * 2, reduce=L.REDUCE_ALL, **kw)
+      z = ops.quantize(many, reduce=L.REDUCE_ROWS, group=128, **kw)  # 65536 + 4096 scales
+    w = ops.quantize(x, reduce=L.REDUCE_ALL, **kw)
+    torch.cuda.current_stream().wait_stream(fork)
+    return [t.clone() for t in (*y, *z, *w)]
+
+  mk = lambda seed: (torch.randn(1, 1024, 512, device=gpu, generator=torch.Generator(device=gpu).manual_seed(seed)) * (seed + 1),
+                     torch.randn(1, 17 * 128, 4096, device=gpu, generator=torch.Generator(device=gpu).manual_seed(seed)) * (seed + 1))
+  graphed = hip_graph.GraphedCall(call, *mk(7))
+  first, = [ws for ws in graphed._workspaces.cleared if ws.numel() == 1 << 20]
+  assert all(ws is not first for ws in graphed._workspaces.values())
+  for seed in range(4):
+    for size in (1 << 20, 1 << 21):  # whoever takes memory of that size now
+      others = [torch.full((size,), 255, dtype=torch.uint8, device=gpu) for _ in range(4)]
+      assert all(t.data_ptr() != first.data_ptr() for t in others)
+      del others
+    args = mk(seed)
+    got = graphed(*args)
+    for a, b in zip(got, call(*args)):
+      assert torch.equal(a, b)
+    torch.cuda.synchronize()
+    assert int(first[:first.numel() // 2].count_nonzero()) == 0
