@@ -507,7 +507,7 @@ def gemm_weight_only(a: torch.Tensor, b: torch.Tensor, col_scale: torch.Tensor, 
   holding values of `col_scale_dtype`.  float32 sums; the weight is never copied as bf16.  tuning (None =
   GEMM_TUNING): 128 = 128 x 128 tiles, 8 = 256 x 256 tiles, 16 = those walked by one workgroup per CU; every one of them
   sums k in the same order, so the results do not depend on it.  Without one, a long k over few output tiles is summed in
-  slices."""
+  slices, as many as the tiles leave room for: the last bit of a row may then depend on how many rows the call has."""
   _require_gpu(a, b, col_scale)
   assert a.dim() == 3 and a.dtype == torch.bfloat16 and a.stride(2) == 1
   batch, m, k = a.shape

@@ -251,7 +251,8 @@ typedef struct aqtx_gemm_plan {
      outside every group are not written.  NULL: ordinary batches.                          */
   const int32_t* group_offsets;
   int32_t tuning;             /* 0 = the library chooses the launch shape.  Tuning only (results never
-                                 depend on it): 4 | 8 = waves per workgroup of the int8 kernel on
+                                 depend on it, but for the order of the sums of aqtx_gemm_weight_only, which
+                                 takes slices of k with 0 alone, see k_split): 4 | 8 = waves per workgroup of the int8 kernel on
                                  256 x 256 tiles, one workgroup per tile; 16 = 8 waves, one workgroup per CU
                                  walking the tiles; 128 = the int8 kernel on 128 x 128 tiles, two workgroups a
                                  CU; 129 | 130 | 131 | 132 = its schedule for launches of at most one
@@ -264,8 +265,9 @@ typedef struct aqtx_gemm_plan {
                                  order): 0 = the library chooses, 1 = one workgroup per output tile walks
                                  all of k, S > 1 = k is cut into (at most) S slices contracted by
                                  workgroups of their own, for shapes with few output tiles and a long k.
-                                 Slices write partial sums to k_split_workspace.  aqtx_gemm_weight_only: 0 =
-                                 the library chooses, 1 = no slices                                    */
+                                 Slices write partial sums to k_split_workspace.  aqtx_gemm_weight_only, whose
+                                 float32 sums do depend on the order: 0 = the library chooses (by batch, m, n
+                                 and k; with tuning 0 alone), 1 = no slices, more is refused            */
   void* k_split_workspace;    /* DEVICE scratch for the slices, 16-byte aligned, at least
                                  aqtx_gemm_i8_k_slices(plan) * batch * m * n * 4 bytes (or
                                  aqtx_gemm_weight_only_k_slices); NULL: no slices
@@ -309,7 +311,10 @@ int aqtx_gemm_i8_k_slices(const aqtx_gemm_plan* plan);
 
 /*
  * The same for aqtx_gemm_weight_only, whose slices leave float32 sums: with them the sum over k is formed slice by slice,
- * so the last bit of a result may differ from a call without k_split_workspace (or with k_split = 1).
+ * so the last bit of a result may differ from a call without k_split_workspace (or with k_split = 1, or a tuning).  How
+ * many there are follows from the number of output tiles, the rows among them: the same row of a may get another last bit
+ * in a call with another m.  A caller that wants the same bits for every m lends no workspace or sets k_split = 1: all
+ * tile sizes sum k in one order.
  */
 int aqtx_gemm_weight_only_k_slices(const aqtx_gemm_plan* plan);
 
@@ -341,9 +346,11 @@ int aqtx_pad_rows(int64_t batch, int64_t k, const void* a, int64_t rows_a, int64
  * (aqt_tensor.py:161-200), without the bf16 copy of the weight: the int8 bytes are widened (exactly) on their
  * way into v_mfma_f32_32x32x16_bf16.  Float32 sums: agrees with the reference's float contraction to summation
  * order, not bit for bit.  Of the plan: batch, m, n, k, lda, ldb (elements), ldc, strides, a_dtype (AQTX_BF16),
- * b_dtype (AQTX_I8 | AQTX_I4), out_dtype = dequant_dtype = AQTX_BF16, col_scale_dtype, col_scale_stride_b are
- * read.  k % 16 == 0, lda % 8 == 0, ldb % 16 == 0, a and b 16-byte aligned.  For m <= 64 aqtx_decode_weight_only
- * streams the weight faster.
+ * b_dtype (AQTX_I8 | AQTX_I4), out_dtype = dequant_dtype = AQTX_BF16, col_scale_dtype, col_scale_stride_b, tuning,
+ * b_layout, k_split (0 | 1), k_split_workspace and k_split_workspace_bytes are read; group_offsets must be NULL.
+ * k % 16 == 0, lda % 8 == 0, ldb % 16 == 0, a and b 16-byte aligned.  A long k over few output tiles is up to 2.5
+ * times as fast in slices, for which the caller lends the memory (aqtx_gemm_weight_only_k_slices).  For m <= 64
+ * aqtx_decode_weight_only streams the weight faster.
  */
 int aqtx_gemm_weight_only(const aqtx_gemm_plan* plan, const void* a, const void* b, const float* col_scale,
                           void* c, void* stream);

@@ -452,6 +452,29 @@ def test_gemm_k_slices_choice_is_a_host_decision():
   assert 'accumulate' in _err(lib.aqtx_gemm_fp8(ctypes.byref(p), FAKE, FAKE, None, None, FAKE, None, None))
 
 
+def test_weight_only_gemm_k_slices_choice_is_a_host_decision():
+  """aqtx_gemm_weight_only_k_slices: from k = 6144 on, for at most 64 tiles of 128 x 256, at most 16; none where k_split or
+  tuning says so.  A k_split beyond 1 is refused."""
+  lib = L.lib()
+
+  def slices(m, n, k, **kw):
+    p = _woplan(m=m, n=n, k=k, lda=k, ldb=k, ldc=n, **kw)
+    return lib.aqtx_gemm_weight_only_k_slices(ctypes.byref(p))
+
+  assert slices(500, 4096, 14336) == 4          # 64 tiles
+  assert slices(513, 4096, 14336) == 1          # 80 tiles
+  assert slices(128, 4096, 14336) == 16 and slices(129, 4096, 14336) == 8  # (the rows decide, and with them the order of the sum)
+  assert slices(128, 4097, 14336) == 15         # 17 tiles
+  assert slices(1, 1, 1 << 20) == 16            # never more
+  assert slices(128, 4096, 6144) == 16 and slices(128, 4096, 6128) == 1
+  assert slices(128, 4096, 14336, batch=4) == 4 and slices(128, 4096, 14336, batch=5) == 1
+  assert slices(128, 4096, 14336, b_layout=L.W_FRAGMENTS) == 16
+  for kw in (dict(k_split=1), dict(tuning=8), dict(tuning=16), dict(tuning=128)):
+    assert slices(128, 4096, 14336, **kw) == 1
+  assert slices(0, 4096, 14336) == slices(128, 0, 14336) == slices(128, 4096, 14336, batch=0) == 1
+  assert lib.aqtx_gemm_weight_only_k_slices(None) == 1
+
+
 def test_conv_validation():
   lib = L.lib()
   w = L.Im2colPlan()

@@ -513,6 +513,60 @@ def test_weight_only_gemm_in_slices_of_k(gpu, batch, m, n, k, slices, w_sdt, lay
 
 @pytest.mark.gpu
 @pytest.mark.parametrize('layout', ['rows', 'fragments'])
+@pytest.mark.parametrize('batch,m,n,k', [(1, 65, 136, 6160), (1, 129, 258, 8208), (1, 300, 1030, 6144), (2, 200, 264, 6176)])
+def test_weight_only_gemm_slices_use_the_memory_lent(gpu, batch, m, n, k, layout):
+  """The slabs of a sliced call hold the partial sums of its slices, and nothing behind them is touched; without the memory
+  (none, too little, not aligned) the call is the one without slices, bit for bit, and leaves it alone."""
+  if layout == 'fragments' and batch > 1:
+    pytest.skip('fragment order is one weight')
+  g = torch.Generator(device=gpu).manual_seed(m)
+  a = torch.randn(batch, m, k, device=gpu, generator=g).to(torch.bfloat16)
+  b = torch.randint(-128, 128, (batch, n, k), dtype=torch.int8, device=gpu, generator=g)
+  cs = torch.rand(batch, n, device=gpu, generator=g) * 0.01 + 1e-4
+  w = ops.tile_weight(b[0], L.I8) if layout == 'fragments' else b
+  plan = L.GemmPlan()
+  plan.batch, plan.m, plan.n, plan.k = batch, m, n, k
+  plan.lda, plan.ldb, plan.ldc = k, 0 if layout == 'fragments' else k, n
+  plan.stride_a, plan.stride_b, plan.stride_c = m * k, 0 if layout == 'fragments' else n * k, m * n
+  plan.b_layout = L.W_FRAGMENTS if layout == 'fragments' else L.W_ROWS
+  plan.a_dtype, plan.b_dtype = L.BF16, L.I8
+  plan.out_dtype = plan.dequant_dtype = plan.row_scale_dtype = L.BF16
+  plan.col_scale_dtype, plan.col_scale_stride_b = L.F32, n
+  slices = L.lib().aqtx_gemm_weight_only_k_slices(ctypes.byref(plan))
+  assert slices > 1
+  chunk = -(-(-(-k // slices)) // 64) * 64  # k of a slice: whole stages of 64
+  used = -(-k // chunk)
+  slab, sentinel = batch * m * n, 0x7FC0DEAD  # (a NaN)
+  lent = torch.full((slices * slab + 64,), sentinel, dtype=torch.int32, device=gpu)
+  need = slices * slab * 4
+
+  def call(pointer, nbytes, **kw):
+    lent.fill_(sentinel)
+    out = torch.empty((batch, m, n), dtype=torch.bfloat16, device=gpu)
+    plan.k_split_workspace, plan.k_split_workspace_bytes = pointer, nbytes
+    plan.k_split = kw.get('k_split', 0)
+    L.check(L.lib().aqtx_gemm_weight_only(ctypes.byref(plan), a.data_ptr(), w.data_ptr(), cs.data_ptr(), out.data_ptr(),
+                                          torch.cuda.current_stream().cuda_stream))
+    return out
+
+  whole = ops.gemm_weight_only(a, w, cs, tuning=128, b_layout=plan.b_layout)
+  at = lent.data_ptr()
+  for pointer, nbytes, kw in ((None, need, {}), (at, need - 4, {}), (at + 4, need, {}), (at, need, dict(k_split=1))):
+    assert torch.equal(call(pointer, nbytes, **kw), whole) and bool((lent == sentinel).all())
+  got = call(at, need)
+  assert torch.equal(got, ops.gemm_weight_only(a, w, cs, b_layout=plan.b_layout))
+  assert bool((lent[used * slab:] == sentinel).all())
+  sums = lent[:used * slab].view(torch.float32).reshape(used, batch, m, n).double()
+  for z in range(used):
+    part = slice(z * chunk, min((z + 1) * chunk, k))
+    ad, bd = a[:, :, part].double(), b[:, :, part].double()
+    for i in range(batch):
+      exact, size = ad[i] @ bd[i].T, ad[i].abs() @ bd[i].abs().T
+      assert bool(((sums[z, i] - exact).abs() <= chunk * 2.0 ** -24 * size).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('layout', ['rows', 'fragments'])
 @pytest.mark.parametrize('w_sdt', ['bf16', 'f32'])
 @pytest.mark.parametrize('m,n,k', [(300, 520, 144), (256, 256, 128), (1024, 768, 4096), (130, 72, 1040), (2304, 4100, 320)])
 def test_weight_only_gemm_tile_sizes_give_the_same_bits(gpu, m, n, k, w_sdt, layout):
