@@ -117,7 +117,8 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 // the grid gives a CU one workgroup).
 struct Quad {
   // Scales the products are exact for, no value becoming subnormal, infinite or NaN on the way (a sum with a
-  // neighbour's 0 * infinity would): bf16 values of 2^-60 .. 2^41.
+  // neighbour's 0 * infinity would): bf16 values from 2^-60 up to, not with, 2^41.  (A packed b carries its values times 16, so
+  // its column scales come as a sixteenth: those given may be 2^-56 to 2^45.)
   static __device__ __forceinline__ bool scale_fits(float v) {
     const uint32_t b = __builtin_bit_cast(uint32_t, v);
     return ((b >> 23) & 255u) - 67u <= 100u && (b & 0xFFFFu) == 0;

@@ -121,18 +121,32 @@ def test_grouped_gemm_kernel(gpu, m, n, k, group, out, rdt, cdt, packed):
       assert torch.equal(eo, got)
 
 
+def _matrix_product_tiles(rs, cs, packed):
+  """Which 128 x 128 tiles have all their scales in the range of the matrix products, [tiles of rows, tiles of columns]: the
+  kernel's own rule, after the sixteenth that packed column scales carry.  (Scales are bf16 values.)"""
+  def fits(v):
+    exponent = (np.asarray(v, np.float32).view(np.uint32) >> 23) & 255
+    return ((exponent >= 67) & (exponent <= 167)).all(0)
+  rows, cols = fits(rs), fits(cs * np.float32(0.0625) if packed else cs)
+  return np.array([[rows[r:r + 128].all() and cols[c:c + 128].all() for c in range(0, len(cols), 128)]
+                   for r in range(0, len(rows), 128)])
+
+
+@pytest.mark.parametrize('packed', [False, True])
 @pytest.mark.parametrize('where', ['none', 'first group', 'last group', 'one column', 'subnormal products'])
 @pytest.mark.parametrize('m,n,k', [(65, 8, 128), (130, 257, 384), (40, 70, 512), (16, 130, 8192 + 128)])
-def test_grouped_gemm_scales_beyond_the_matrix_products(gpu, m, n, k, where):
-  """bf16 scales of 2^-60 .. 2^41 are multiplied on the matrix cores, a tile with any other on the vector ALU: the same
-  numbers, infinite and NaN where the oracle's are."""
+def test_grouped_gemm_scales_beyond_the_matrix_products(gpu, m, n, k, where, packed):
+  """bf16 scales of 2^-60 up to (not with) 2^41, packed column scales sixteen times that, are multiplied on the matrix cores, a
+  tile with any other on the vector ALU: the same numbers, infinite and NaN where the oracle's are."""
   from aqt_amd import _lib as L
   rng = np.random.default_rng(19)
   a, b = rng.integers(-128, 128, (m, k)).astype(np.int8), rng.integers(-7, 8, (n, k)).astype(np.int8)
   a[0], b[0] = -128, -7  # the largest sums a group can have
-  groups = k // 128
+  groups, unit = k // 128, 16.0 if packed else 1.0
   exps = lambda *shape: np.exp2(rng.integers(-60, 40, shape)).astype(np.float32) * (1 + rng.random(shape, np.float32) * 0.9)
-  rs, cs = nm.to_bf16(exps(groups, m)), nm.to_bf16(np.minimum(exps(groups, n), 1e3))
+  rs, cs = nm.to_bf16(exps(groups, m)), nm.to_bf16(np.minimum(exps(groups, n) * np.float32(unit), 1e3))
+  top = 2.0 ** 41 * (1 - 2.0 ** -8)  # the ends of the range, in one product and alone
+  rs[0, 0], rs[0, 1], cs[0, 0], cs[0, 2] = 2.0 ** -60, top, 2.0 ** -60 * unit, top * unit
   if where == 'first group':
     rs[0, m // 2], cs[0, 1] = np.inf, 2.0 ** 100
   elif where == 'last group':
@@ -140,16 +154,28 @@ def test_grouped_gemm_scales_beyond_the_matrix_products(gpu, m, n, k, where):
   elif where == 'one column':
     cs[:, 3] = 0.0
   elif where == 'subnormal products':
-    rs[:], cs[:] = nm.to_bf16(rs * 0 + np.float32(2.0 ** -80)), nm.to_bf16(cs * 0 + np.float32(2.0 ** -61))
+    rs[:], cs[:] = 2.0 ** -80, 2.0 ** -61
+  on_matrix_cores = _matrix_product_tiles(rs, cs, packed)
+  want_tiles = np.ones_like(on_matrix_cores)
+  if where == 'first group':
+    want_tiles[m // 2 // 128], want_tiles[:, 0] = False, False
+  elif where == 'last group':
+    want_tiles[0], want_tiles[:, (n - 1) // 128] = False, False
+  elif where == 'one column':
+    want_tiles[:, 0] = False
+  elif where == 'subnormal products':
+    want_tiles[:] = False
+  np.testing.assert_array_equal(on_matrix_cores, want_tiles)
+  if where == 'last group' and groups > 1:  # found after stages that went well
+    assert _matrix_product_tiles(rs[:-1], cs[:-1], packed).all()
   with np.errstate(all='ignore'):
     want = _grouped_ref(a, b, rs, cs, 128, 'bf16', 'bf16', 'bf16')
-  for packed in (False, True):
-    bt = torch.from_numpy(b).to(gpu)
-    for tuning in (0, 128):
-      got = ops.gemm_grouped(torch.from_numpy(a).to(gpu), ops.pack_i4(bt) if packed else bt, row_scale=torch.from_numpy(rs).to(gpu),
-                             col_scale=torch.from_numpy(cs).to(gpu), group=128, out_dtype=torch.bfloat16, tuning=tuning,
-                             row_scale_dtype=torch.bfloat16, col_scale_dtype=torch.bfloat16, b_dtype=L.I4P if packed else L.I4)
-      np.testing.assert_array_equal(got.float().cpu().numpy(), want)
+  bt = torch.from_numpy(b).to(gpu)
+  for tuning in (0, 128):
+    got = ops.gemm_grouped(torch.from_numpy(a).to(gpu), ops.pack_i4(bt) if packed else bt, row_scale=torch.from_numpy(rs).to(gpu),
+                           col_scale=torch.from_numpy(cs).to(gpu), group=128, out_dtype=torch.bfloat16, tuning=tuning,
+                           row_scale_dtype=torch.bfloat16, col_scale_dtype=torch.bfloat16, b_dtype=L.I4P if packed else L.I4)
+    np.testing.assert_array_equal(got.float().cpu().numpy(), want)
 
 
 def _even_odd8(a):
