@@ -24,6 +24,7 @@ from aqt_amd import _lib as L
 from aqt_amd import ops
 from aqt_amd.v2 import aqt_quantizer
 from aqt_amd.v2 import aqt_tensor
+from aqt_amd.v2 import calibration
 from aqt_amd.v2 import lowering
 from aqt_amd.v2 import transpose
 from aqt_amd.v2 import utils
@@ -1670,9 +1671,9 @@ def _fresh_cfg(cfg: 'DotGeneral', fwd_only: bool = False) -> 'DotGeneral':
 
 
 def _try_calibrators(cfg: DotGeneral) -> bool:
-  """Makes and initialises the gradient contractions' calibrators without keeping them (2 us, where copies of their objects
-  take 7): settings that cannot make them are refused, and a calibration of the user's own sees every call.  False, with
-  nothing made: quantizers of the user's own, whose init_calibration() wants a copy."""
+  """Makes and initialises the gradient contractions' calibrators without keeping them (half a microsecond each, where
+  copies of all objects take 7): settings that cannot make them are refused, and a calibration of the user's own sees every
+  call.  False, with nothing made: quantizers of the user's own, whose init_calibration() wants a copy."""
   quantizers = []
   for raw in (cfg.dlhs, cfg.drhs):
     dq = raw.dg_quantizer
@@ -1683,7 +1684,8 @@ def _try_calibrators(cfg: DotGeneral) -> bool:
   if any(type(q) is not aqt_quantizer.Quantizer for q in quantizers):
     return False
   for q in quantizers:
-    if q.calibration is not None:
+    # (the plain abs-max calibration takes any dtype and does nothing when made)
+    if q.calibration is not None and q.calibration is not calibration.AbsMaxCalibration:
       q.calibration(dtype=q.scale_dtype).init_calibration()
   return True
 
