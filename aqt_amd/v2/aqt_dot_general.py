@@ -638,25 +638,13 @@ def _canonical_pairs(lhs, rhs, dimension_numbers):
 _NotFused = lowering.NotFused
 
 
-class _ProfilerScope:
-  """The named scope around a contraction: what torch.profiler.record_function records, for a profiler (a user annotation)
-  and for the observer of an execution trace, without its two dispatched calls (3 against 11 us, with none running)."""
-  __slots__ = ('name', 'handle')
-
-  def __init__(self, name):
-    self.name = name
-
-  def __enter__(self):
-    self.handle = torch._C._autograd._record_function_with_args_enter(self.name)
-    return self
-
-  def __exit__(self, *exc):
-    torch._C._autograd._record_function_with_args_exit(self.handle)
-    return False
-
-
-_profiler_scope = (_ProfilerScope if hasattr(torch._C._autograd, '_record_function_with_args_enter')
-                   else torch.profiler.record_function)
+# The named scope around a contraction: what torch.profiler.record_function records, for a profiler (a user annotation) and for
+# the observer of an execution trace, without its two dispatched calls and its object (2 to 3 against 11 us, with none running).
+_enter_scope = getattr(torch._C._autograd, '_record_function_with_args_enter', None)
+_leave_scope = getattr(torch._C._autograd, '_record_function_with_args_exit', None)
+if _enter_scope is None or _leave_scope is None:
+  _enter_scope = lambda name: torch.profiler.record_function(name).__enter__()
+  _leave_scope = lambda scope: scope.__exit__(None, None, None)
 
 # (lhs, rhs): whether the forward quantizers of this call should leave, next to the values they write, the partial
 # maxima with which the backward pass calibrates those values over the other axis (DotGeneralRaw._quant_side); set
@@ -706,26 +694,32 @@ class DotGeneralRaw:
     transposed (and contiguous).  `_bwd_memo` (this build): a dict owned by one backward pass, in
     which its two contractions share per-tensor scales of the gradient.
     """
-    with _profiler_scope(self.jax_scope_name):
-      if isinstance(rhs, MultiTensor):
-        lhs, rhs = _maybe_use_fwd_quant(lhs, rhs, dimension_numbers, self.rhs.use_fwd_quant)
-      if self.local_aqt is None:
-        return self._dispatch(lhs, rhs, lhs_qt, rhs_qt, dimension_numbers, _out_transpose_axes, _bwd_memo)
-      # LocalAqt (aqt_dot_general.py:773-776, 833-837): every shard of the contraction axis is
-      # calibrated and contracted on its own (the shard axis is a leading batch axis), the
-      # dequantized shard outputs are summed; no residuals come back.
-      msg = 'Custom calib_shared_axes not implemented for local AQT.'
-      if isinstance(self.dg_quantizer, DefaultDotGeneralQuantizer):
-        self.dg_quantizer.assert_calib_shared_axes_value(None, None, msg)
-      n_ca = len(dimension_numbers[0][0])
-      assert n_ca == len(dimension_numbers[0][1])
-      lhs, rhs, dn = _apply_local_aqt(self.local_aqt, lhs, rhs, dimension_numbers)
-      out, _ = self._dispatch(lhs, rhs, lhs_qt, rhs_qt, dn, None, _bwd_memo)
-      if n_ca > 0:
-        out = ops.sum_tiles(out.contiguous())
-      if _out_transpose_axes is not None:
-        out = out.permute(tuple(_out_transpose_axes))
-      return out, None
+    scope = _enter_scope(self.jax_scope_name)
+    try:
+      return self._call_in_scope(lhs, rhs, lhs_qt, rhs_qt, dimension_numbers, _out_transpose_axes, _bwd_memo)
+    finally:
+      _leave_scope(scope)
+
+  def _call_in_scope(self, lhs, rhs, lhs_qt, rhs_qt, dimension_numbers, _out_transpose_axes, _bwd_memo):
+    if isinstance(rhs, MultiTensor):
+      lhs, rhs = _maybe_use_fwd_quant(lhs, rhs, dimension_numbers, self.rhs.use_fwd_quant)
+    if self.local_aqt is None:
+      return self._dispatch(lhs, rhs, lhs_qt, rhs_qt, dimension_numbers, _out_transpose_axes, _bwd_memo)
+    # LocalAqt (aqt_dot_general.py:773-776, 833-837): every shard of the contraction axis is
+    # calibrated and contracted on its own (the shard axis is a leading batch axis), the
+    # dequantized shard outputs are summed; no residuals come back.
+    msg = 'Custom calib_shared_axes not implemented for local AQT.'
+    if isinstance(self.dg_quantizer, DefaultDotGeneralQuantizer):
+      self.dg_quantizer.assert_calib_shared_axes_value(None, None, msg)
+    n_ca = len(dimension_numbers[0][0])
+    assert n_ca == len(dimension_numbers[0][1])
+    lhs, rhs, dn = _apply_local_aqt(self.local_aqt, lhs, rhs, dimension_numbers)
+    out, _ = self._dispatch(lhs, rhs, lhs_qt, rhs_qt, dn, None, _bwd_memo)
+    if n_ca > 0:
+      out = ops.sum_tiles(out.contiguous())
+    if _out_transpose_axes is not None:
+      out = out.permute(tuple(_out_transpose_axes))
+    return out, None
 
   def _dispatch(self, lhs, rhs, lhs_qt, rhs_qt, dimension_numbers, out_transpose_axes, bwd_memo=None):
     """The lowered paths where they implement the configuration (_lowered_call: the int8 / fp8 kernels for
@@ -1674,19 +1668,21 @@ def _try_calibrators(cfg: DotGeneral) -> bool:
   """Makes and initialises the gradient contractions' calibrators without keeping them (half a microsecond each, where
   copies of all objects take 7): settings that cannot make them are refused, and a calibration of the user's own sees every
   call.  False, with nothing made: quantizers of the user's own, whose init_calibration() wants a copy."""
-  quantizers = []
+  calibrations = []
   for raw in (cfg.dlhs, cfg.drhs):
     dq = raw.dg_quantizer
     if type(dq) is not DefaultDotGeneralQuantizer:
       return False
-    quantizers += [dq.lhs, dq.rhs]
-    quantizers += [q for q, alpha in ((dq.lhs_mid, dq.lhs_mid_alpha), (dq.rhs_mid, dq.rhs_mid_alpha)) if alpha is not None]
-  if any(type(q) is not aqt_quantizer.Quantizer for q in quantizers):
-    return False
-  for q in quantizers:
-    # (the plain abs-max calibration takes any dtype and does nothing when made)
-    if q.calibration is not None and q.calibration is not calibration.AbsMaxCalibration:
-      q.calibration(dtype=q.scale_dtype).init_calibration()
+    for q, used in ((dq.lhs, True), (dq.rhs, True),
+                    (dq.lhs_mid, dq.lhs_mid_alpha is not None), (dq.rhs_mid, dq.rhs_mid_alpha is not None)):
+      if used:
+        if type(q) is not aqt_quantizer.Quantizer:
+          return False
+        # (the plain abs-max calibration takes any dtype and does nothing when made)
+        if q.calibration is not None and q.calibration is not calibration.AbsMaxCalibration:
+          calibrations.append(q)
+  for q in calibrations:
+    q.calibration(dtype=q.scale_dtype).init_calibration()
   return True
 
 
